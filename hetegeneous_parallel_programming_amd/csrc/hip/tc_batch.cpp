@@ -17,6 +17,8 @@ struct tc_batch {
   int32_t n = 0;
   int64_t* rp = nullptr;
   int32_t* ci = nullptr;
+  uint16_t* c16 = nullptr;  // 16-bit codes of ci (null when a graph has too many rows for them)
+  int32_t core_kb = 0;
   tck::GraphDesc* d_descs = nullptr;
   std::vector<tck::GraphDesc> descs;
   std::vector<int32_t> rows;
@@ -40,6 +42,7 @@ struct tc_batch {
     graph = nullptr;
     dev_free(rp);
     dev_free(ci);
+    dev_free(c16);
     dev_free(d_descs);
     partners.release();
     scratch.release();
@@ -62,6 +65,9 @@ static tc_status capture(tc_ctx* ctx, tc_batch* b) {
   b->partners.into(a);
   a.tune = to_kernel_tune(ctx->tune);
   a.bufs = b->scratch.bufs();
+  a.c16 = b->c16;
+  a.core = b->c16 ? 1 : 0;
+  a.core_kb = b->core_kb;
   for (int32_t r : b->rows) a.wide_ids |= r > tck::kNarrowIds ? 1 : 0;
   hipStream_t s = ctx->stream;
   TC_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
@@ -86,7 +92,7 @@ static tc_status capture(tc_ctx* ctx, tc_batch* b) {
   if (e == hipSuccess)
     e = hipMemcpyAsync(b->pinned, a.bufs.outs, sizeof(uint64_t) * (size_t)b->n, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess)
-    e = hipMemcpyAsync(b->pinned + b->n, a.bufs.counters, sizeof(uint32_t) * tck::kNumCounters,
+    e = hipMemcpyAsync(b->pinned + b->n, a.bufs.counters, sizeof(uint32_t) * tck::kPlanWords,
                        hipMemcpyDeviceToHost, s);
   hipGraph_t g = nullptr;
   hipError_t e2 = hipStreamEndCapture(s, &g);
@@ -135,8 +141,11 @@ tc_status tc_batch_create(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_graphs
   b->P = pro;
   b->RP = rpo;
   b->cio = cio;
+  const int32_t most_rows = b->rows.empty() ? 0 : *std::max_element(b->rows.begin(), b->rows.end());
+  const bool coded = n_graphs > 0 && most_rows <= tck::kCoreIds && cio < tck::kCorePool;
+  b->core_kb = tck::core_bits(most_rows);
   tc_status st = dev_alloc((void**)&b->rp, sizeof(int64_t) * (size_t)std::max<int64_t>(rpo, 1), "batch rowptr");
-  if (st == TC_OK) st = dev_alloc((void**)&b->ci, sizeof(int32_t) * (size_t)std::max<int64_t>(cio, 1), "batch colidx");
+  if (st == TC_OK) st = dev_alloc((void**)&b->ci, sizeof(int32_t) * (size_t)(cio + tck::kCiPad), "batch colidx");
   if (st == TC_OK)
     st = dev_alloc((void**)&b->d_descs, sizeof(tck::GraphDesc) * (size_t)std::max(n_graphs, 1), "batch descs");
   if (st == TC_OK) st = b->partners.alloc(cio, pro, n_graphs);
@@ -145,6 +154,8 @@ tc_status tc_batch_create(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_graphs
     b->release();
     return st;
   }
+  // the bitmap kernels' codes, which a count can do without
+  if (coded && dev_alloc((void**)&b->c16, tck::code_bytes(cio), "batch id codes") != TC_OK) b->c16 = nullptr;
   hipError_t e = hipHostMalloc((void**)&b->pinned, sizeof(uint64_t) * ((size_t)n_graphs + 16), hipHostMallocDefault);
   if (e != hipSuccess) {
     b->pinned = nullptr;
@@ -281,7 +292,8 @@ tc_status tc_batch_create(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_graphs
       a.vrow += f.pr_base;
       a.nv += sg.g0;
       a.gbase = sg.g0;
-      st = launch_build(a, sg.rows, sg.ids, bs, ctx->stream);
+      a.core_kb = b->core_kb;
+      st = launch_build(a, sg.rows, sg.ids, bs, ctx->stream, nullptr, nullptr, nullptr, nullptr, b->c16);
     }
     if (st == TC_OK && e == hipSuccess) e = hipEventRecord(ctx->ev[1], ctx->stream);
     std::vector<int32_t> nv((size_t)n_graphs);
@@ -303,7 +315,7 @@ tc_status tc_batch_create(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_graphs
     for (int32_t v : nv) b->nv += v;
   }
   b->bytes = sizeof(int64_t) * rpo + sizeof(int32_t) * cio + (int64_t)sizeof(tck::GraphDesc) * n_graphs +
-             b->partners.bytes + PlanScratch::bytes_for(b->P) + 8 * (int64_t)n_graphs;
+             b->partners.bytes + PlanScratch::bytes_for(b->P) + 8 * (int64_t)n_graphs + (b->c16 ? (int64_t)tck::code_bytes(cio) : 0);
   *out = b.release();
   return TC_OK;
 } catch (...) {

@@ -113,7 +113,8 @@ struct BuildScratch {
 // loc: null, or where to write each partner entry's DAG edge position and
 // partner vertex and each partner row's owner (pedge, pvid, pown).
 tc_status launch_build(const tck::LaunchArgs& a, int64_t RP, int64_t M, BuildScratch& bs, hipStream_t s,
-                       const LocalBufs* loc = nullptr, int32_t* pown = nullptr);
+                       const LocalBufs* loc = nullptr, int32_t* pown = nullptr, const uint8_t* closed = nullptr,
+                       const uint8_t* part = nullptr, uint16_t* codes = nullptr);
 
 // Makes ctx's device current for the scope of one API call.
 struct DeviceGuard {
@@ -176,6 +177,17 @@ struct tc_graph {
   int32_t row_begin = 0, row_end = 0;
   int64_t edge_begin = 0, edge_end = 0;  // DAG edge positions of rows [row_begin, row_end)
   uint8_t* own = nullptr;                 // null, or per row 1 if it is a pivot row
+  uint16_t* c16 = nullptr;  // 16-bit codes of ci for the bitmap kernels (null: none)
+  uint8_t* closed = nullptr;  // with c16, over kCoreIds rows: tck::BuildBufs::closed
+  uint8_t* part = nullptr;    // with closed: tck::BuildBufs::lpart
+  bool coded = false;         // whether enough edges can use the codes
+  void drop_codes() {
+    tcr::dev_free(c16);
+    tcr::dev_free(closed);
+    tcr::dev_free(part);
+    c16 = nullptr;
+    closed = part = nullptr;
+  }
   int32_t* pown = nullptr;  // [nv_max + 1] owner vertex of each partner row, written by every build
   int32_t max_out = 0;
   tcr::Partners partners;
@@ -186,10 +198,9 @@ struct tc_graph {
   tck::GraphDesc* d_desc = nullptr;
   int64_t bytes = 0;
   // The binned count's plan, kept across calls: valid for plan_tune; its
-  // rows per bin and tiles per bin (which size the launches) on the host.
+  // rows per bin (which size the launches) on the host.
   tcr::PlanScratch plan;
   bool plan_valid = false;
   tc_tune plan_tune{};
   int64_t plan_bins[tck::kNumBins] = {};
-  int64_t plan_tiles[tck::kNumBins] = {};
 };

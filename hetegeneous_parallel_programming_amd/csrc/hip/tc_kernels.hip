@@ -29,7 +29,9 @@
 // that bin) from a device queue, heaviest bins first.  Counts are u64 sums,
 // so the result does not depend on tile order.  Local variants of the bin
 // kernels also attribute every hit to its edge and corners.
+#include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "tc_kernels.hpp"
 
@@ -57,8 +59,8 @@ __device__ __forceinline__ int group_excl_scan(int x, int gl, int& total) {
 }
 
 // First k in [0, G) with sEnd[k] > t (sEnd non-decreasing, sEnd[G-1] > t).
-template <int G>
-__device__ __forceinline__ int find_edge(const int32_t* sEnd, int t) {
+template <int G, class T>
+__device__ __forceinline__ int find_edge(const T* sEnd, T t) {
   int k = 0;
 #pragma unroll
   for (int step = G / 2; step >= 1; step >>= 1)
@@ -85,10 +87,13 @@ __device__ __forceinline__ int tree_pos(int x, int h) {
   return (1 << (h - 1 - tz)) + (i1 >> (tz + 1));
 }
 
+// Streamed ids are taken kChunk at a time: a lane loads kChunk consecutive
+// ids of a list with one load and looks each up, so finding the lane's edge,
+// forming the address and issuing the load are paid once per kChunk ids.
 #ifndef TC_IN_FLIGHT
-#define TC_IN_FLIGHT 8
+#define TC_IN_FLIGHT 2
 #endif
-constexpr int kInFlight = TC_IN_FLIGHT;  // lookups per lane per iteration
+constexpr int kInFlight = TC_IN_FLIGHT;  // chunks per lane per iteration
 // Edge ends a lane reads together when it steps past its edge, by group
 // width, and how many such reads a wave-wide group makes before it falls
 // back to a binary search (sub-wave groups: TC_STEP_STAGES_GROUP).
@@ -111,10 +116,8 @@ constexpr int kInFlight = TC_IN_FLIGHT;  // lookups per lane per iteration
 #define TC_STEP_STAGES_GROUP 1
 #endif
 #ifndef TC_IN_FLIGHT_GROUP
-#define TC_IN_FLIGHT_GROUP 6
+#define TC_IN_FLIGHT_GROUP 1
 #endif
-// Sub-wave groups keep per-group state in vector registers; fewer lookups
-// in flight leave room for it.
 constexpr int kInFlightGroup = TC_IN_FLIGHT_GROUP;
 // Steps whose every slot holds an id skip the per-slot bounds checks: bit 0
 // for wave-wide groups, bit 1 for sub-wave groups (code size and registers
@@ -157,6 +160,10 @@ struct PivotSet {
 // values; typing them as global keeps the element loads global_load (a
 // generic pointer would make them flat loads, which also wait on LDS).
 typedef __attribute__((address_space(1))) const int32_t gint32;
+// kChunk consecutive ids anywhere in a list: only int32-aligned, which global
+// loads of any width allow.
+typedef int32_t chunk_ids __attribute__((ext_vector_type(kChunk), aligned(4)));
+typedef __attribute__((address_space(1))) const chunk_ids gchunk;
 
 constexpr int32_t kEmpty = -1;
 constexpr uint32_t kHashA0 = 0x9E3779u;  // odd 24-bit multipliers: 2^24 / phi,
@@ -311,31 +318,35 @@ __device__ __forceinline__ void count_slot_hit(uint32_t* C, int idx) {
   atomicAdd(&C[idx >> 1], 1u << ((idx & 1) << 4));
 }
 
-// Adds one lookup step's hits (f) to the counters EC of their batch edges
-// (kq).  The lanes of a wide group stream one or two edges per step, so
-// per-hit atomics would pile onto one LDS word; instead the wave adds once
-// per distinct hit counter (ballot, one lane adds the popcount; counters
-// told apart by LDS address, so the groups of a wave are kept apart).
-// Call from wave-uniform control flow.  Groups narrower than
-// TC_EDGE_HITS_MIN_G spread over as many edges as groups and add per hit,
+// Adds the hits h of one chunk per lane to the counters EC of their batch
+// edges (kq).  The lanes of a wide group stream a few edges per step, so
+// per-lane atomics would pile onto one LDS word; instead the wave adds once
+// per distinct hit counter (ballots of the bits of h, one lane adds their
+// popcounts; counters told apart by LDS address, so the groups of a wave are
+// kept apart).  Call from wave-uniform control flow.  Groups narrower than
+// TC_EDGE_HITS_MIN_G spread over as many edges as groups and add per lane,
 // and so do full local counts (their per-hit branch already bumps a slot
 // counter; a second, per-edge loop beside it costs more than it saves).
 #ifndef TC_EDGE_HITS_MIN_G
 #define TC_EDGE_HITS_MIN_G 64
 #endif
 template <int G, int kLocal>
-__device__ __forceinline__ void edge_hits(uint32_t* EC, int kq, bool f) {
+__device__ __forceinline__ void edge_hits(uint32_t* EC, int kq, uint32_t h) {
   if constexpr (kLocal == kLocalEdges && G >= TC_EDGE_HITS_MIN_G) {
+    static_assert(kChunk < 8, "hits of a chunk fit three bits");
     const uint32_t key = (uint32_t)(uintptr_t)(EC + kq);
-    uint64_t rem = __ballot(f);
+    const uint64_t h0 = __ballot((h & 1) != 0), h1 = __ballot((h & 2) != 0), h2 = __ballot((h & 4) != 0);
+    uint64_t rem = h0 | h1 | h2;
     while (rem) {
       const int lead = __builtin_ctzll(rem);
       const uint64_t same = rem & __ballot(key == (uint32_t)__builtin_amdgcn_readlane((int)key, lead));
-      if ((int)(threadIdx.x & 63) == lead) atomicAdd(&EC[kq], (uint32_t)__builtin_popcountll(same));
+      if ((int)(threadIdx.x & 63) == lead)
+        atomicAdd(&EC[kq], (uint32_t)(__builtin_popcountll(same & h0) + 2 * __builtin_popcountll(same & h1) +
+                                      4 * __builtin_popcountll(same & h2)));
       rem &= ~same;
     }
   } else {
-    if (f) atomicAdd(&EC[kq], 1u);
+    if (h) atomicAdd(&EC[kq], h);
   }
 }
 
@@ -360,32 +371,42 @@ __device__ __forceinline__ uint32_t group_sum(uint32_t x) {
   return x;
 }
 
-// NF lookups of ids w[] in a hash set: two 8-byte LDS reads (one bucket of
-// each table) and four compares per id.  kLocal: a hit also bumps the hit
-// counter of its batch edge kq[] and (kLocalFull) of its slot.
-template <int G, int NF, int kLocal, bool kWide>
-__device__ __forceinline__ void hash_probe(const PivotSet& S, const int (&w)[NF], const int (&kq)[NF],
-                                           uint32_t& hits, const LocalSink& ls) {
+// Lookups of NC chunks of ids w[] in a hash set: two 8-byte LDS reads (one
+// bucket of each table) and four compares per id.  Only the first rem[c] ids
+// of chunk c count.  kLocal: a chunk's hits also go to the hit counter of its
+// batch edge kq[] and (kLocalFull) each hit to that of its slot.
+template <int G, int NC, int kLocal, bool kWide>
+__device__ __forceinline__ void hash_probe(const PivotSet& S, const int (&w)[NC * kChunk], const int (&rem)[NC],
+                                           const int (&kq)[NC], uint32_t& hits, const LocalSink& ls) {
   const char* Tb = (const char*)S.A;
   const int lb = S.p0;
 #pragma unroll
-  for (int q = 0; q < NF; ++q) {
-    const int hk = hash_key<kWide>(w[q]);
-    const uint32_t b0 = hash_bucket(hk, kHashA0, lb), b1 = hash_bucket(hk, kHashA1, lb);
-    const int2 x = *(const int2*)(Tb + (b0 << 3));
-    const int2 y = *(const int2*)(Tb + S.p1 + (b1 << 3));
-    const bool f = (x.x == w[q]) | (x.y == w[q]) | (y.x == w[q]) | (y.y == w[q]);
-    hits += f ? 1u : 0u;
-    if constexpr (kLocal == kLocalFull) {
-      if (f) {
-        const int t1 = S.p1 >> 2;  // word offset of table 1
-        const int idx = x.x == w[q] ? 2 * (int)b0
-                      : x.y == w[q] ? 2 * (int)b0 + 1
-                      : y.x == w[q] ? t1 + 2 * (int)b1 : t1 + 2 * (int)b1 + 1;
-        count_slot_hit(ls.C, idx);
+  for (int c = 0; c < NC; ++c) {
+    uint32_t h = 0;
+#pragma unroll
+    for (int i = 0; i < kChunk; ++i) {
+      const int q = c * kChunk + i;
+      const int hk = hash_key<kWide>(w[q]);
+      const uint32_t b0 = hash_bucket(hk, kHashA0, lb), b1 = hash_bucket(hk, kHashA1, lb);
+      const int2 x = *(const int2*)(Tb + (b0 << 3));
+      const int2 y = *(const int2*)(Tb + S.p1 + (b1 << 3));
+      const bool f = ((x.x == w[q]) | (x.y == w[q]) | (y.x == w[q]) | (y.y == w[q])) & (i < rem[c]);
+      if constexpr (kLocal) h += f ? 1u : 0u;
+      else hits += f ? 1u : 0u;
+      if constexpr (kLocal == kLocalFull) {
+        if (f) {
+          const int t1 = S.p1 >> 2;  // word offset of table 1
+          const int idx = x.x == w[q] ? 2 * (int)b0
+                        : x.y == w[q] ? 2 * (int)b0 + 1
+                        : y.x == w[q] ? t1 + 2 * (int)b1 : t1 + 2 * (int)b1 + 1;
+          count_slot_hit(ls.C, idx);
+        }
       }
     }
-    if constexpr (kLocal) edge_hits<G, kLocal>(ls.EC, kq[q], f);
+    if constexpr (kLocal) {
+      hits += h;
+      edge_hits<G, kLocal>(ls.EC, kq[c], h);
+    }
   }
 }
 
@@ -394,9 +415,13 @@ __device__ __forceinline__ void hash_probe(const PivotSet& S, const int (&w)[NF]
 // sEnd/sBase are this group's G-entry LDS scratch.  kModes: the set modes
 // this instantiation handles.  Returns this lane's share of the hits.
 //
-// Flat index t of a batch maps to edge k (sEnd[k-1] <= t < sEnd[k]) and to
-// element t of the int32 array at sBase[k] (N+(v) shifted back by the edge's
-// first flat index); each lane keeps its current edge's end and base in
+// Each edge of a batch takes whole chunks of one flat index space: it starts
+// at a multiple of kChunk and ends at sEnd[k] (not rounded up), so a chunk's
+// first index t (a multiple of kChunk) lies in edge k when sEnd[k-1] <= t <
+// sEnd[k], holds ids t .. min(t + kChunk, sEnd[k]) of the int32 array at
+// sBase[k] (N+(v) shifted back by the edge's first flat index), and may read
+// up to kChunk - 1 ids past the list's end (colidx pools are padded for it),
+// which do not count.  Each lane keeps its current edge's end and base in
 // registers and searches sEnd only when it steps past that edge.
 // Where the streamed lists of a pivot's edges come from: ids of a DAG row
 // (one rowptr lookup each), or partner list references.
@@ -411,19 +436,20 @@ struct DagEdges {
 };
 struct RefEdges {
   const ListRef* refs;
+  uint32_t skip;  // edges with this mark are counted elsewhere
   __device__ __forceinline__ void operator()(int j, int64_t& b, int& c) const {
     const ListRef r = refs[j];
     b = list_start(r);
-    c = list_len(r);
+    c = ref_marks(r, skip) ? 0 : list_len(r);
   }
 };
 
 // kWide: hash sets hold keys folded for ids past 2^24 (kSetHashWide); one
 // instantiation per hash kind keeps a single lookup path in the loop.
-template <int G, int kModes, int NF = kInFlight, int kLocal = kLocalNone, bool kWide = false, class Src>
+template <int G, int kModes, int NC = kInFlight, int kLocal = kLocalNone, bool kWide = false, class Src>
 __device__ __forceinline__ uint32_t pivot_edges(const int32_t* __restrict__ ci, const Src src, int da,
                                                 const PivotSet S, int jfirst, int jstride,
-                                                int32_t* sEnd, gint32** sBase, int gl,
+                                                uint32_t* sEnd, gint32** sBase, int gl,
                                                 const LocalSink& ls = LocalSink{}) {
   uint32_t hits = 0;
   const int32_t* A = S.A;
@@ -442,31 +468,35 @@ __device__ __forceinline__ uint32_t pivot_edges(const int32_t* __restrict__ ci, 
     int64_t ej = 0;
     if constexpr (kLocal)
       if (j < da) ej = ls.pedge[j];
-    int total;
-    const int excl = group_excl_scan<G>(c, gl, total);
-    sEnd[gl] = excl + c;
+    // flat indexes are unsigned: 64 lists of almost 2^25 ids, in whole
+    // chunks, reach 2^31
+    int sum;
+    const uint32_t excl = (uint32_t)group_excl_scan<G>((c + kChunk - 1) & -kChunk, gl, sum);
+    const uint32_t total = (uint32_t)sum;
+    sEnd[gl] = excl + (uint32_t)c;
     sBase[gl] = base - excl;
     wave_sync();
     int cur_k = -1;   // the lane's current edge
-    int cur_end = 0;  // t < cur_end  <=>  t lies in the lane's current edge
+    uint32_t cur_end = 0;  // t < cur_end  <=>  t lies in the lane's current edge
     gint32* cur_base = (gint32*)ci;
-    // A lane's flat index grows by G per id, so its next edge is one of the
+    // A lane's flat index grows by G chunks a step, so its next edge is one of the
     // next few: a step reads the next kLookAhead ends together (lists of a
     // few dozen ids make a wave-wide group's lanes pass a couple of edges
     // per step, a narrow group's one), then, for lanes still past them, up
     // to kStages - 1 more such reads, and searches only past those.  Each
-    // read moves k over the run of ends at or below t.  t < total =
-    // sEnd[G - 1] keeps cur_k + 1 inside the batch and ends every run inside
+    // read moves k over the run of ends at or below t.  t < total (so t <
+    // sEnd[G - 1]) keeps cur_k + 1 inside the batch and ends every run inside
     // the group, so words read past the group's G entries (other groups'
     // ends, or the Base array after End: LDS of this block) never count.
     constexpr int kLookAhead = G >= 64 ? TC_STEP_LA64 : G >= 32 ? TC_STEP_LA32 : G >= 16 ? TC_STEP_LA16 : TC_STEP_LA8;
     constexpr int kStages = G >= 64 ? TC_STEP_STAGES : TC_STEP_STAGES_GROUP;
-    auto step_to = [&](int t) {
-      int k = cur_k, e = cur_end;  // e <= t
+    auto step_to = [&](uint32_t t) {
+      int k = cur_k;
+      uint32_t e = cur_end;  // e <= t
 #pragma unroll
       for (int st = 0; st < kStages; ++st) {
         if (st > 0 && e > t) break;
-        int ev[kLookAhead];
+        uint32_t ev[kLookAhead];
 #pragma unroll
         for (int i = 0; i < kLookAhead; ++i) ev[i] = sEnd[k + 1 + i];
         k += 1;
@@ -487,58 +517,68 @@ __device__ __forceinline__ uint32_t pivot_edges(const int32_t* __restrict__ ci, 
       cur_end = e;
       cur_base = sBase[k];
     };
-    for (int t0 = 0; t0 < total; t0 += G * NF) {
+    constexpr int NF = NC * kChunk;
+    for (uint32_t t0 = 0; t0 < total; t0 += G * NF) {
       int w[NF];
-      int kq[NF];  // kLocal: batch edge of each id
-      if ((TC_SPLIT_FULL & (G == 64 ? 1 : 2)) && t0 + G * NF <= total) {  // every slot holds an id
+      int rem[NC];  // ids of each chunk that count
+      int kq[NC];   // kLocal: batch edge of each chunk
+      auto load = [&](int c, uint32_t t) {
+        if (t >= cur_end) step_to(t);
+        const chunk_ids x = *(gchunk*)(cur_base + t);
 #pragma unroll
-        for (int q = 0; q < NF; ++q) {
-          const int t = t0 + q * G + gl;
-          if (t >= cur_end) step_to(t);
-          w[q] = cur_base[t];
-          if constexpr (kLocal) kq[q] = cur_k;
-        }
+        for (int i = 0; i < kChunk; ++i) w[c * kChunk + i] = x[i];
+        rem[c] = (int)(cur_end - t);
+        if constexpr (kLocal) kq[c] = cur_k;
+      };
+      if ((TC_SPLIT_FULL & (G == 64 ? 1 : 2)) && t0 + G * NF <= total) {  // every lane has NC chunks
+#pragma unroll
+        for (int c = 0; c < NC; ++c) load(c, t0 + (c * G + gl) * kChunk);
       } else {
 #pragma unroll
-        for (int q = 0; q < NF; ++q) {
-          const int t = t0 + q * G + gl;
-          w[q] = INT_MIN;  // ids are >= 0: never found
-          if constexpr (kLocal) kq[q] = 0;
-          if (t < total) {
-            if (t >= cur_end) step_to(t);
-            w[q] = cur_base[t];
-            if constexpr (kLocal) kq[q] = cur_k;
-          }
+        for (int c = 0; c < NC; ++c) {
+          const uint32_t t = t0 + (c * G + gl) * kChunk;
+#pragma unroll
+          for (int i = 0; i < kChunk; ++i) w[c * kChunk + i] = 0;
+          rem[c] = 0;
+          if constexpr (kLocal) kq[c] = 0;
+          if (t < total) load(c, t);
         }
       }
       if ((kModes & kModeHash) && S.mode == (kWide ? kSetHashWide : kSetHash)) {
-        hash_probe<G, NF, kLocal, kWide>(S, w, kq, hits, ls);
+        hash_probe<G, NC, kLocal, kWide>(S, w, rem, kq, hits, ls);
       } else if ((kModes & kModeTree) && ((kModes == kModeTree) || S.mode == kSetTree)) {
         // h descent steps; then the lower bound is k with its trailing one
         // bits and the following zero shifted out (0 = past the end -> -1).
         // The node index is carried as a byte offset (4k): one compare, one
         // select and one shift-add per step.  ~k is never 0 (k < 2^h).
+        // (One chunk at a time: a set is rarely a tree, and the hash lookups'
+        // loop should not pay registers for it.)
         const int h = S.p0;
         const char* Ab = (const char*)A;
-        int kb[NF];
 #pragma unroll
-        for (int q = 0; q < NF; ++q) kb[q] = 4;
-        for (int s = 0; s < h; ++s) {
-          int val[NF];
+        for (int c = 0; c < NC; ++c) {
+          int kb[kChunk];
 #pragma unroll
-          for (int q = 0; q < NF; ++q) val[q] = *(const int32_t*)(Ab + kb[q]);
+          for (int i = 0; i < kChunk; ++i) kb[i] = 4;
+          for (int s = 0; s < h; ++s) {
+            int val[kChunk];
 #pragma unroll
-          for (int q = 0; q < NF; ++q) kb[q] = 2 * kb[q] + (val[q] < w[q] ? 4 : 0);
-        }
+            for (int i = 0; i < kChunk; ++i) val[i] = *(const int32_t*)(Ab + kb[i]);
 #pragma unroll
-        for (int q = 0; q < NF; ++q) {
-          const unsigned k = (unsigned)kb[q] >> 2;
-          const unsigned lo = (k >> __builtin_ctz(~k)) >> 1;
-          const bool f = A[lo] == w[q];
-          hits += f ? 1u : 0u;
-          if constexpr (kLocal == kLocalFull)
-            if (f) count_slot_hit(ls.C, (int)lo);
-          if constexpr (kLocal) edge_hits<G, kLocal>(ls.EC, kq[q], f);
+            for (int i = 0; i < kChunk; ++i) kb[i] = 2 * kb[i] + (val[i] < w[c * kChunk + i] ? 4 : 0);
+          }
+          uint32_t hc = 0;
+#pragma unroll
+          for (int i = 0; i < kChunk; ++i) {
+            const unsigned k = (unsigned)kb[i] >> 2;
+            const unsigned lo = (k >> __builtin_ctz(~k)) >> 1;
+            const bool f = (A[lo] == w[c * kChunk + i]) & (i < rem[c]);
+            hc += f ? 1u : 0u;
+            if constexpr (kLocal == kLocalFull)
+              if (f) count_slot_hit(ls.C, (int)lo);
+          }
+          hits += hc;
+          if constexpr (kLocal) edge_hits<G, kLocal>(ls.EC, kq[c], hc);
         }
       } else if (kModes & kModeHbm) {
         int lo[NF];
@@ -551,14 +591,18 @@ __device__ __forceinline__ uint32_t pivot_edges(const int32_t* __restrict__ ci, 
           len -= half;
         }
 #pragma unroll
-        for (int q = 0; q < NF; ++q) {
-          const bool f = A[lo[q]] == w[q];
-          hits += f ? 1u : 0u;
-          if constexpr (kLocal) {
+        for (int c = 0; c < NC; ++c) {
+          uint32_t hc = 0;
+#pragma unroll
+          for (int i = 0; i < kChunk; ++i) {
+            const int q = c * kChunk + i;
+            const bool f = (A[lo[q]] == w[q]) & (i < rem[c]);
+            hc += f ? 1u : 0u;
             if constexpr (kLocal == kLocalFull)
               if (f) atomicAdd(&ls.vcount[w[q]], 1ull);
-            if constexpr (kLocal) edge_hits<G, kLocal>(ls.EC, kq[q], f);
           }
+          hits += hc;
+          if constexpr (kLocal) edge_hits<G, kLocal>(ls.EC, kq[c], hc);
         }
       }
     }
@@ -929,25 +973,36 @@ __global__ __launch_bounds__(kBlock) void partner_rows_fill_kernel(LaunchArgs a,
 
 // Pass 5: work of every partner row still at 0 (the sum of its partners'
 // list lengths), with a group of kBuildG lanes per slot.
-__global__ __launch_bounds__(kBlock) void partner_work_kernel(LaunchArgs a) {
+// flags: every row's kind of edges (kRowClosed, kRowOpen) goes to g as well.
+__global__ __launch_bounds__(kBlock) void partner_work_kernel(LaunchArgs a, bool flags) {
   const int64_t p = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kBuildG;
   const int gl = threadIdx.x % kBuildG;
   if (p >= a.P) return;  // the whole group
   VRow* vr = (VRow*)a.vrow + p;
-  if (vr->set == 0 || vr->work != 0) return;  // unused slot, or work known from the build
+  if (vr->set == 0 || (vr->work != 0 && !flags)) return;  // unused slot, or work known from the build
   const int64_t pb = a.vrp[p], pe = a.vrp[p + 1];
   int64_t w = 0;
+  int32_t kinds = 0;
   constexpr int kU = 4;  // list references in flight per lane
   for (int64_t e0 = pb + gl; e0 < pe; e0 += kU * kBuildG) {
     ListRef r[kU];
 #pragma unroll
     for (int j = 0; j < kU; ++j) r[j] = e0 + j * kBuildG < pe ? a.pci[e0 + j * kBuildG] : (ListRef)0;
 #pragma unroll
-    for (int j = 0; j < kU; ++j) w += list_len(r[j]);
+    for (int j = 0; j < kU; ++j) {
+      w += list_len(r[j]);
+      if (list_len(r[j])) kinds |= ref_marks(r[j], kMarkClosed) ? kRowClosed : kRowOpen;
+    }
   }
 #pragma unroll
-  for (int o = kBuildG / 2; o >= 1; o >>= 1) w += __shfl_xor(w, o, kBuildG);
-  if (gl == 0) vr->work = (uint32_t)min(w, (int64_t)0xFFFFFFFF);
+  for (int o = kBuildG / 2; o >= 1; o >>= 1) {
+    w += __shfl_xor(w, o, kBuildG);
+    kinds |= __shfl_xor(kinds, o, kBuildG);
+  }
+  if (gl == 0) {
+    vr->work = (uint32_t)min(w, (int64_t)0xFFFFFFFF);
+    if (flags) vr->g = kinds;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -986,7 +1041,8 @@ __global__ __launch_bounds__(kBlock) void partner_work_kernel(LaunchArgs a) {
 // row is split (batches and the server), so graph g's pairs are the ids of
 // the graphs before it.
 
-constexpr int32_t kDegSat = 65535;  // deg16 saturation
+constexpr int32_t kDegSat = 16383;      // deg16 saturation
+constexpr uint16_t kDegClosed = 0x8000, kDegOrdered = 0x4000;  // deg16: the row is closed, ordered
 
 // Exclusive scan of n (<= kBlock * per) values of s (in place); returns the
 // sum.  All threads of the block call it.
@@ -1065,8 +1121,11 @@ __global__ __launch_bounds__(kBlock) void radix_prep_kernel(LaunchArgs a, int64_
   }
   b.gid[q] = split ? lo : ~lo;
   b.erow[q] = d.eb + e0;
-  b.lref[q] = u < d.n_rows ? list_ref(d.ci_off + e0, du) : (ListRef)0;
-  b.deg16[q] = (uint16_t)min(du, (int64_t)kDegSat);
+  const uint8_t marks = b.closed && u < d.n_rows ? b.closed[u] : (uint8_t)0;
+  b.lref[q] = u >= d.n_rows ? (ListRef)0
+            : marks & kClosed ? closed_ref(d.ci_off + e0, du, kPartAll) : list_ref(d.ci_off + e0, du);
+  b.deg16[q] = (uint16_t)(min(du, (int64_t)kDegSat) | (marks & kClosed ? kDegClosed : 0) |
+                          (marks & kOrdered ? kDegOrdered : 0));
   if (q == RP - 1) b.erow[RP] = M;
 }
 
@@ -1087,10 +1146,7 @@ __global__ __launch_bounds__(kBlock) void radix_mpath_kernel(const int64_t* erow
 }
 
 // A pair's partner before placement: its list, or (kRefSlot set) the
-// partner's row slot, whose list the placement reads.  Pool offsets stay
-// below 2^38, so bit 63 of a list reference is free.
-constexpr ListRef kRefSlot = 1ull << 63;
-
+// partner's row slot, whose list the placement reads.
 // Split block blk: the ids of its merge-path range, kMPPer per thread at a
 // stride of kBlock (coalesced loads and stores); each id's row by a
 // branch-free binary search over the block's rows in LDS.  An edge its head
@@ -1152,8 +1208,14 @@ __global__ __launch_bounds__(kBlock) void radix_split_kernel(LaunchArgs a, int64
     if (R[s] < 0) continue;
     const int64_t E = j0 + (int64_t)s * kBlock + threadIdx.x;
     const int gr = s_gid[R[s]];
+    auto put_code = [&](int64_t x, int32_t v) {  // every id's code is a function of the id: written on the way
+      const int32_t at = (int32_t)(E - ebase - s_erow[R[s]]);
+      b.codes[code_start(x - at, (uint32_t)(s_erow[R[s] + 1] - s_erow[R[s]])) + at] =
+          (uint16_t)core_code((uint32_t)v, a.core_kb);
+    };
     if (gr < 0) {
       b.key[E] = -1;  // the row is not split: no pair
+      if (b.codes) put_code(E + cd0, a.ci[E + cd0]);  // (one graph)
       continue;
     }
     if (gr != gc) {
@@ -1162,7 +1224,9 @@ __global__ __launch_bounds__(kBlock) void radix_split_kernel(LaunchArgs a, int64
       cd = a.descs[g0 + gr].ci_off - a.descs[g0 + gr].eb;
     }
     cix[s] = E + cd;
-    qv[s] = (int32_t)(rb + a.ci[cix[s]]);
+    const int32_t v = a.ci[cix[s]];
+    qv[s] = (int32_t)(rb + v);
+    if (b.codes) put_code(cix[s], v);
   }
 #pragma unroll
   for (int s = 0; s < kMPPer; ++s) dv[s] = qv[s] >= 0 ? (int32_t)b.deg16[qv[s]] : 0;
@@ -1173,7 +1237,7 @@ __global__ __launch_bounds__(kBlock) void radix_split_kernel(LaunchArgs a, int64
       const int64_t E = j0 + (int64_t)s * kBlock + threadIdx.x;
       const int r = R[s];
       const int64_t du = s_erow[r + 1] - s_erow[r];
-      int64_t dvx = dv[s];
+      int64_t dvx = dv[s] & kDegSat;
       if (dvx == kDegSat && du >= kDegSat) dvx = b.erow[qv[s] + 1] - b.erow[qv[s]];  // both saturated: exact
       const int32_t q = (int32_t)(i0 + r);
       int32_t owner;
@@ -1182,7 +1246,9 @@ __global__ __launch_bounds__(kBlock) void radix_split_kernel(LaunchArgs a, int64
         b.ref[E] = kRefSlot | (ListRef)(uint32_t)qv[s];
       } else {  // the head owns it: partner = this row's list
         owner = qv[s];
-        b.ref[E] = list_ref(cix[s] - (E - ebase - s_erow[r]), du);
+        const int64_t start = cix[s] - (E - ebase - s_erow[r]);
+        b.ref[E] = dv[s] & kDegClosed ? closed_ref(start, du, dv[s] & kDegOrdered ? b.lpart[cix[s]] : kPartAll)
+                                      : list_ref(start, du);
       }
       b.key[E] = owner;
       // a local rebuild (one graph): the edge's row word, bit 31 when the head owns it
@@ -1645,7 +1711,7 @@ static hipError_t launch_partner_rows(const LaunchArgs& a, int64_t RP, const Bui
   if ((e = launch_scan(LoadI32{b.kc}, StoreI64{b.voff}, RP, b.part, s)) != hipSuccess) return e;
   partner_rows_fill_kernel<<<blocks, kBlock, 0, s>>>(a, RP, b);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if (a.P > 0) partner_work_kernel<<<(unsigned)((a.P * kBuildG + kBlock - 1) / kBlock), kBlock, 0, s>>>(a);
+  if (a.P > 0) partner_work_kernel<<<(unsigned)((a.P * kBuildG + kBlock - 1) / kBlock), kBlock, 0, s>>>(a, b.closed != nullptr);
   return hipGetLastError();
 }
 
@@ -1838,11 +1904,12 @@ __global__ __launch_bounds__(kBlock) void plan_scatter_kernel(LaunchArgs a) {
 // ---------------------------------------------------------------------------
 struct __align__(16) CountLds {
   int32_t A[kAreaBlock];         // pivot-set areas (one per group of the tile's bin)
-  int32_t End[kBlock];           // per-lane edge end in the batch's flat index
+  uint32_t End[kBlock];          // per-lane edge end in the batch's flat index
   gint32* Base[kBlock];          // per-lane N+(v) base of that edge, shifted by its first index
   uint64_t red[kWaves];
   int64_t tab_cnt[1];
-  int64_t cur_first, cur_seg;
+  int64_t cur_seg;
+  uint32_t next[2];
 };
 static_assert(kAreaWave * kWaves <= kAreaBlock, "wave areas exceed LDS region");
 static_assert(kAreaG32 * (kBlock / 32) <= kAreaBlock, "g32 areas exceed LDS region");
@@ -1909,6 +1976,13 @@ struct __align__(16) LocalLds<kLocalEdges> {
   __device__ uint32_t* ec() { return EC; }
 };
 
+// What a plain count's hash kernel leaves out of its rows: where the bitmap
+// kernels count the edges marked kRefClosed of the wave-wide bins' rows, those.
+template <int G, int kLocal>
+__device__ __forceinline__ uint32_t open_only(const LaunchArgs& a) {
+  return kLocal == kLocalNone && G >= 64 && a.core == 2 ? kMarkClosed : 0u;
+}
+
 template <int G, int AREA, int kLocal, bool kWide>
 __device__ __forceinline__ void group_tile(const LaunchArgs& a, const uint64_t* items, int64_t first,
                                            int64_t last, CountLds& L, LocalLds<kLocal>& LL, bool batch,
@@ -1918,19 +1992,21 @@ __device__ __forceinline__ void group_tile(const LaunchArgs& a, const uint64_t* 
   // is wave-uniform and lives in scalar registers.
   const int grp = G == 64 ? uniform32(threadIdx.x / 64) : threadIdx.x / G, gl = threadIdx.x % G;
   int32_t* slot = L.A + grp * AREA;
-  int32_t* sEnd = L.End + grp * G;
+  uint32_t* sEnd = L.End + grp * G;
   gint32** sBase = L.Base + grp * G;
   constexpr int kEL = edge_local(kLocal);
   uint32_t* C = kLocal == kLocalFull ? LL.c() + grp * (AREA / 2) : nullptr;
   for (int64_t i = first + grp; i < last; i += NGRP) {
     const int64_t item = (int64_t)items[i];
     const PRow pr = partner_row(a, item);
+    const uint32_t skip = open_only<G, kLocal>(a);
+    if (skip && !(pr.g & kRowOpen)) continue;
     const PivotSet S = build_pivot_set<G, kEL, kWide>(slot, AREA, a.ci + list_start(pr.set), list_len(pr.set),
                                                       gl, a.tune, a.bufs.counters + kCntFallback, C);
     const LocalSink ls{C, kEL ? LL.ec() + grp * G : nullptr, kEL ? a.local.pedge + pr.pb : nullptr,
                        kEL ? a.local.pvid + pr.pb : nullptr, a.local.ecount, a.local.vcount};
     const uint32_t h = pivot_edges<G, kModeHash | kModeTree, G == 64 ? kInFlight : kInFlightGroup, kEL, kWide>(
-        a.ci, RefEdges{a.pci + pr.pb}, (int)(pr.pe - pr.pb), S, 0, G, sEnd, sBase, gl, ls);
+        a.ci, RefEdges{a.pci + pr.pb, skip}, (int)(pr.pe - pr.pb), S, 0, G, sEnd, sBase, gl, ls);
     if constexpr (kLocal == kLocalFull) {
       group_sync<G>();
       flush_set_hits<G>(slot, C, S, gl, a.local.vcount);
@@ -1951,7 +2027,9 @@ __device__ __forceinline__ void block_pivot(const LaunchArgs& a, uint64_t item, 
   const int32_t* ci = a.ci;
   const int32_t* set = ci + list_start(pr.set);
   const int ds = list_len(pr.set);
-  const RefEdges part{a.pci + pr.pb};
+  const uint32_t skip = open_only<kBlock, kLocal>(a);
+  if (skip && !(pr.g & kRowOpen)) return;  // the whole workgroup
+  const RefEdges part{a.pci + pr.pb, skip};
   const int np = (int)(pr.pe - pr.pb);
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
   constexpr int kEL = edge_local(kLocal);
@@ -2002,14 +2080,51 @@ constexpr int waves_per_eu(int kLocal) {
        : kLocal == kLocalEdges ? TC_LOCAL_EDGES_WAVES_PER_EU : TC_COUNT_WAVES_PER_EU;  // parts: the plain count's
 }
 
+// How a persistent workgroup gets its tiles.  A queue head that every
+// workgroup adds to serves one tile per ~12 ns on MI355X, which bounds a
+// kernel of many small tiles (an R-MAT-22 graph's 66 K workgroup rows whose
+// codes leave them little to do here: 0.80 ms queued, 0.19 ms with turns); so
+// a workgroup takes its first tiles in turn (blockIdx.x + k * grid, k <
+// fixed) and only the last part, which evens out what the turns left uneven,
+// comes from the queue.  16ths of the tiles taken in turn: 15 (R-MAT-22,
+// R-MAT-18 and a partition's counts 5-8% faster than with 12); local counts,
+// whose tiles differ more, 8 (edges of R-MAT-20: 1.94 ms, 12: 2.11, 15: 2.40).
+// With fewer than kQueueFrom tiles per workgroup all are taken in turn: every
+// workgroup's last, empty answer from the queue would cost more than it evens
+// out (R-MAT n=30011: 0.15 -> 0.03 ms of the bitmap kernels).
+constexpr int kTurns = 15, kLocalTurns = 8, kQueueFrom = 4;
+struct TileTurn {
+  int64_t ntiles, fixed, grid;
+  __device__ TileTurn(int64_t n, int64_t g, int sixteenths) : ntiles(n), grid(g) {
+    fixed = sixteenths >= 16 || ntiles < kQueueFrom * g ? (ntiles + g - 1) / g : ntiles * sixteenths / 16 / g;
+  }
+  __device__ bool all() const { return fixed * grid >= ntiles; }  // no queue
+  __device__ uint32_t first() const { return (uint32_t)(fixed * grid); }  // the queue's first tile
+  // Tile k < fixed of workgroup b.  A batch's tiles are in graph order: each
+  // XCD (workgroups equal modulo 8) takes its own eighth of them, its
+  // workgroups side by side, so that the few graphs it is at stay in its L2
+  // (the batch of 512 graphs: the bitmap kernel of whole-workgroup rows 0.50
+  // -> 0.34 ms, the 16-lane bin 0.93 -> 0.83 ms).
+  __device__ int64_t tile(uint32_t b, int64_t k, bool batch) const {
+    if (batch && grid % 8 == 0) return (b & 7) * (fixed * (grid / 8)) + (b >> 3) + k * (grid / 8);
+    return b + k * grid;
+  }
+};
+
+__device__ __forceinline__ unsigned long long* out_word(const LaunchArgs& a) {
+  return (unsigned long long*)a.bufs.outs + (a.out_slots ? (blockIdx.x & (kOutSlots - 1)) * kOutStride : 0);
+}
+
 // One persistent kernel per bin, specialised so that each keeps only its own
-// working set in registers.  Blocks pull tiles from the bin's queue head.
+// working set in registers.
+// rounds: rows per group in a light bin's tile, 0: as many as still give
+// every workgroup a tile, at most the tune's.
 // kLocal: also the per-edge (and, kLocalFull, per-vertex) attribution of
 // a.local (one graph only).
 // kWide: the instantiation for graphs whose ids reach 2^24 (folded hash keys).
 template <int BIN, int kLocal, bool kWide>
 __global__ __launch_bounds__(kBlock, waves_per_eu(kLocal)) void count_kernel(
-    LaunchArgs a) {
+    LaunchArgs a, int rounds) {
   __shared__ CountLds L;
   __shared__ LocalLds<kLocal> LL;
   // batch: per-graph sums; kLocalParts: per-part sums, kept the same way
@@ -2022,17 +2137,18 @@ __global__ __launch_bounds__(kBlock, waves_per_eu(kLocal)) void count_kernel(
     L.tab_cnt[0] = a.bufs.counters[kCntBinCount + BIN];
   }
   __syncthreads();
-  const int piv = tile_pivots(BIN, a.tune.rounds > 0 ? a.tune.rounds : 1);
   const int64_t cnt = L.tab_cnt[0];
+  const int piv = tile_pivots(BIN, rounds > 0 ? rounds : tile_rounds(BIN, cnt, gridDim.x, a.tune.rounds));
   const int64_t ntiles = (cnt + piv - 1) / piv;
   const uint64_t* items = a.bufs.items + L.cur_seg;
   Acc acc;
   acc.g = 0;
-  for (;;) {
-    if (threadIdx.x == 0) L.cur_first = atomicAdd(&a.bufs.counters[kCntTileHead + BIN], 1u);
-    __syncthreads();
-    const int64_t t = uniform64(L.cur_first);
-    if (t >= ntiles) break;
+  const TileTurn turn(ntiles, gridDim.x, edge_local(kLocal) ? kLocalTurns : kTurns);
+  int64_t t = turn.tile(blockIdx.x, 0, batch);
+  for (int64_t k = 1; t < ntiles; ++k) {
+    const bool queued = k >= turn.fixed && !turn.all();
+    if (queued && threadIdx.x == 0)  // read after the barrier at the end, into the other word next time
+      L.next[k & 1] = turn.first() + atomicAdd(&a.bufs.counters[kCntHeads + kHeadStride * BIN], 1u);
     const int64_t first = t * piv;
     const int64_t last = min(first + (int64_t)piv, cnt);
     if (BIN == BIN_GLOBAL) block_pivot<false, kLocal, kWide>(a, items[first], L, LL, batch, acc);
@@ -2056,11 +2172,553 @@ __global__ __launch_bounds__(kBlock, waves_per_eu(kLocal)) void count_kernel(
       acc.sum = 0;
     }
     __syncthreads();
+    t = queued ? (int64_t)uniform32((int)L.next[k & 1]) : k < turn.fixed ? turn.tile(blockIdx.x, k, batch) : ntiles;
   }
   if (!batch) {
     const uint64_t tot = block_sum(acc.sum, L.red);
-    if (threadIdx.x == 0 && tot) atomicAdd(&a.bufs.outs[0], tot);
+    if (threadIdx.x == 0 && tot) atomicAdd(out_word(a), tot);
   }
+}
+
+// ---------------------------------------------------------------------------
+// bitmap count of heavy partner rows
+// ---------------------------------------------------------------------------
+// When every id of a graph has a 16-bit code, a row's set is a bitmap of at
+// most 8 KB in LDS and a streamed id is half as wide: a lookup is one LDS
+// byte and four VALU operations instead of two 8-byte LDS reads and eleven,
+// and a lane takes kCoreChunk ids per 16-byte load.
+typedef uint32_t code_words __attribute__((ext_vector_type(kCoreChunk / 2), aligned(2)));
+
+constexpr int kCoreInFlight = 2;  // loads in flight per lane (4: no change; 1: 12% slower on short rows)
+
+// Inclusive scan over the wave by DPP (no LDS traffic).
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1, 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2, 3
+  return x;
+}
+
+template <int NW>
+__device__ __forceinline__ void core_sync() {
+  if constexpr (NW == 1) wave_sync();
+  else __syncthreads();
+}
+
+struct CoreEdge {
+  uint32_t end;  // of the partner's list in the batch's flat index (ids)
+  uint32_t off;  // byte offset in the code pool of flat index 0 seen from this list
+};
+constexpr int kCoreSpan = 4096;  // chunks of flat index whose list starts are marked at a time
+struct CoreWave {
+  CoreEdge e[64];
+  uint64_t starts[kCoreSpan / 64];
+};
+template <int NW>
+struct __align__(16) CoreLds {
+  CoreWave w[NW];
+  uint32_t tile[2];
+};
+
+// Hits of up to 64 partners' lists in the bitmap B: one wave, lane j holding
+// partner j's list (len codes at byte offset off of the pool; len 0: none).
+// The lists take whole chunks of one flat index space; a bit per chunk marks
+// where lists start, so the list of each of 64 consecutive chunks is one
+// broadcast LDS read and two mbcnt, whatever the lists' lengths.  Codes past
+// a list's end do not count, and a load may run past the pool's end
+// (kCorePad).
+__device__ __forceinline__ uint32_t core_batch(const char* __restrict__ pool, const uint8_t* B, CoreWave& W,
+                                               uint32_t len, uint32_t off, int lane) {
+  constexpr int NC = kCoreInFlight, CH = kCoreChunk;
+  static_assert(kCoreSpan % (64 * NC) == 0 && kCoreSpan / 64 <= 64, "spans are whole iterations");
+  const uint32_t n = (len + CH - 1) / CH;
+  const uint32_t incl = wave_incl_scan(n);
+  const uint32_t s = incl - n, total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+  const uint64_t some = __ballot(len != 0);
+  if (len != 0) W.e[__popcll(some & ((1ull << lane) - 1ull))] = CoreEdge{s * CH + len, off - s * (2u * CH)};
+  uint32_t hits = 0;
+  for (uint32_t seg = 0; seg < total; seg += kCoreSpan) {
+    const uint32_t span = min(total - seg, (uint32_t)kCoreSpan);
+    if (lane < kCoreSpan / 64) W.starts[lane] = 0;
+    wave_sync();
+    if (len != 0 && s >= seg && s < seg + span)
+      atomicOr((uint32_t*)W.starts + ((s - seg) >> 5), 1u << ((s - seg) & 31u));
+    uint32_t k0 = (uint32_t)__popcll(__ballot(len != 0 && s < seg));  // lists started before the window
+    wave_sync();
+    for (uint32_t c0 = 0; c0 < span; c0 += 64 * NC) {
+      code_words d[NC];
+      int rem[NC];
+      uint64_t m[NC];
+#pragma unroll
+      for (int q = 0; q < NC; ++q) m[q] = W.starts[c0 / 64 + q];
+#pragma unroll
+      for (int q = 0; q < NC; ++q) {
+        const uint64_t mm = (uint64_t)uniform64((int64_t)m[q]);
+        const uint32_t k = __builtin_amdgcn_mbcnt_hi((uint32_t)(mm >> 33), __builtin_amdgcn_mbcnt_lo((uint32_t)(mm >> 1),
+                                                     k0 + ((uint32_t)mm & 1u) - 1u));
+        k0 += (uint32_t)__popcll(mm);
+        const CoreEdge x = W.e[k];
+        const uint32_t t = (seg + c0 + q * 64 + lane) * CH;
+        rem[q] = min(max((int)(x.end - t), 0), CH);
+        d[q] = *(const code_words*)(pool + (x.off + t * 2u));
+      }
+      // each lookup's bit enters r from the top: code i of a chunk ends up
+      // in bit 24 + i, of which the chunk's first rem count
+#pragma unroll
+      for (int q = 0; q < NC; ++q) {
+        uint32_t r = 0;
+#pragma unroll
+        for (int i = 0; i < CH / 2; ++i) {
+          const uint32_t w = d[q][i];
+          const uint32_t lo = B[w & 0x1FFFu], hi = B[(w >> 16) & 0x1FFFu];
+          r = __builtin_amdgcn_alignbit(lo >> ((w >> kCoreByteBits) & 7u), r, 1);
+          r = __builtin_amdgcn_alignbit(hi >> (w >> 29), r, 1);
+        }
+        hits += __builtin_popcount(__builtin_amdgcn_ubfe(r, 32 - CH, (uint32_t)rem[q]));
+      }
+    }
+    wave_sync();
+  }
+  return hits;
+}
+
+// Persistent kernel over the plan's rows of bins bin0..bin1, a workgroup of
+// NW waves per row: they share the bitmap and take batches of partners.
+template <int NW>
+__global__ __launch_bounds__(64 * NW, 8) void core_kernel(LaunchArgs a, int bin0, int bin1, int head) {
+  extern __shared__ uint32_t s_bits[];  // 2^core_kb bytes
+  __shared__ CoreLds<NW> L;
+  constexpr int T = 64 * NW;
+  typedef uint32_t w4 __attribute__((ext_vector_type(4)));
+  const bool batch = a.ngraphs > 1;
+  int64_t seg = 0, cnt = 0;
+  for (int b = 0; b < bin0; ++b) seg += a.bufs.counters[kCntBinCount + b];
+  for (int b = bin0; b <= bin1; ++b) cnt += a.bufs.counters[kCntBinCount + b];
+  const uint64_t* items = a.bufs.items + seg;
+  const int wid = NW == 1 ? 0 : uniform32(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const uint8_t* B = (const uint8_t*)s_bits;
+  const char* pool = (const char*)a.c16;
+  uint64_t sum = 0;
+  // (waves with a row each finish close together, and there are twice as many
+  // of them as workgroups: all in turn)
+  const TileTurn turn(cnt, gridDim.x, NW == 1 ? 16 : kTurns);
+  int64_t t = turn.tile(blockIdx.x, 0, batch);
+  PRow pr{0, 0, 0, 0, 0};
+  if (t < cnt) pr = partner_row(a, (int64_t)items[t]);
+  for (int64_t k = 1; t < cnt; ++k) {
+    // the next row's place: its turn, or the queue's answer (read after the
+    // first barrier; two words, since a late wave may still read the other)
+    const bool queued = k >= turn.fixed && !turn.all();
+    if (queued && threadIdx.x == 0)
+      L.tile[k & 1] = turn.first() + atomicAdd(&a.bufs.counters[kCntHeads + kHeadStride * head], 1u);
+    const int64_t pb = uniform64(pr.pb);
+    // core 2: a row without closed edges has nothing to do here
+    const int np = a.core == 2 && !(pr.g & kRowClosed) ? 0 : uniform32((int)(pr.pe - pr.pb));
+    const int ds = np ? uniform32(list_len(pr.set)) : 0;
+    const int g = pr.g;
+    const bool all = a.core == 1;
+    const uint16_t* src = a.c16 + code_start(uniform64(list_start(pr.set)), (uint32_t)ds);
+    const int per = NW == 1 || np >= T ? 64 : (np + NW - 1) / NW;  // partners of a wave's batch
+    int j = wid * per + lane;
+    // the first set ids and partners, in flight while the bitmap is cleared
+    const uint32_t x0 = (int)threadIdx.x < ds ? src[threadIdx.x] : (uint32_t)kNoCode;
+    ListRef r0 = lane < per && j < np ? a.pci[pb + j] : (ListRef)0;
+    for (int i = threadIdx.x; i < (1 << a.core_kb) / 16; i += T) ((w4*)s_bits)[i] = w4{0, 0, 0, 0};
+    core_sync<NW>();
+    t = queued ? (int64_t)uniform32((int)L.tile[k & 1]) : k < turn.fixed ? turn.tile(blockIdx.x, k, batch) : cnt;
+    const int64_t next_item = t < cnt ? (int64_t)items[t] : -1;
+    auto put = [&](uint32_t x) {
+      if (x != kNoCode) atomicOr(&s_bits[(x & 0x1FFFu) >> 2], 1u << (((x & 3u) << 3) | (x >> kCoreByteBits)));
+    };
+    put(x0);
+    for (int i = threadIdx.x + T; i < ds; i += T) put(src[i]);
+    core_sync<NW>();
+    if (next_item >= 0) pr = partner_row(a, next_item);
+    uint32_t hits = 0;
+    for (int j0 = wid * per; j0 < np; j0 += NW * per) {
+      const ListRef r = r0;
+      j += NW * per;
+      r0 = lane < per && j < np ? a.pci[pb + j] : (ListRef)0;  // the next batch's
+      const uint32_t full = (uint32_t)list_len(r);
+      const uint32_t len = ref_marks(r, kMarkClosed) ? closed_len(r) : all ? full : 0u;
+      hits += core_batch(pool, B, L.w[wid], len, code_start(list_start(r), full) * 2u, lane);
+    }
+    if (batch) {  // one atomic per wave and row
+      uint32_t h = hits;
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) h += __shfl_xor(h, o);
+      if (lane == 0 && h) atomicAdd(&a.bufs.outs[g], (unsigned long long)h);
+    } else {
+      sum += hits;
+    }
+    core_sync<NW>();
+  }
+  if (!batch) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) sum += shfl_down_u64(sum, d);
+    if (lane == 0 && sum) atomicAdd(out_word(a), sum);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// codes of a large graph: its kCoreIds vertices of highest degree
+// ---------------------------------------------------------------------------
+// Degrees (in + out) without per-id global atomics, whose hub counters every
+// XCD would add to: ids are counted per bucket of 2^kDegBucketBits vertices,
+// their low bits written bucket by bucket, and each bucket counted in LDS.
+constexpr int kDegTile = 16384;   // ids per block of the two bucket passes
+constexpr int kDegThreads = 512;
+constexpr int kDegPer = kDegTile / kDegThreads;
+constexpr int64_t kDegPart = (int64_t)1 << 18;  // bucketed ids per block of the count
+constexpr int kDegCap = 16384;    // degrees from here on are one class
+constexpr int kDegLeast = 16;     // lower degrees get no codes
+struct BigCodes {
+  uint32_t* cnt;    // [nb * tiles + 1]
+  int64_t* part;    // scan partials
+  uint16_t* low;    // [m]
+  uint32_t* deg;    // [n]
+  uint32_t* code;   // [n] degree class << 16 | code
+  uint32_t* hist;   // [kDegCap + 1] vertices per degree, then the threshold
+  uint8_t* cls;     // [kDegCap + 1] class of each degree
+};
+static int64_t deg_tiles(int64_t m) { return (m + kDegTile - 1) / kDegTile; }
+static int64_t deg_buckets(int64_t n) { return (n + ((int64_t)1 << kDegBucketBits) - 1) >> kDegBucketBits; }
+static BigCodes big_codes_at(char* p, int64_t n, int64_t m, int64_t* bytes) {
+  const int64_t nc = deg_buckets(n) * deg_tiles(m) + 1;
+  auto up = [](int64_t b) { return (b + 255) & ~(int64_t)255; };
+  char* q = p;
+  BigCodes x;
+  x.cnt = (uint32_t*)q;  q += up(4 * nc);
+  x.part = (int64_t*)q;  q += up(8 * scan_partials(std::max(nc, n)));
+  x.low = (uint16_t*)q;  q += up(2 * m);
+  x.deg = (uint32_t*)q;  q += up(4 * n);
+  x.code = (uint32_t*)q; q += up(4 * n);
+  x.hist = (uint32_t*)q; q += up(4 * (kDegCap + 4));
+  x.cls = (uint8_t*)q;   q += up(kDegCap + 1);
+  *bytes = q - p;
+  return x;
+}
+int64_t big_codes_bytes(int64_t n, int64_t m) {
+  int64_t b = 0;
+  big_codes_at(nullptr, n, m, &b);
+  return b;
+}
+
+// kScatter: false counts the tile's ids per bucket, true writes their low
+// bits at the scanned positions.
+template <bool kScatter>
+__global__ __launch_bounds__(kDegThreads) void deg_bucket_kernel(const int32_t* __restrict__ ci, int64_t m, int nb,
+                                                                 int64_t tiles, uint32_t* __restrict__ cnt,
+                                                                 uint16_t* __restrict__ low) {
+  __shared__ uint32_t s_n[kDegBuckets];
+  for (int i = threadIdx.x; i < nb; i += kDegThreads) s_n[i] = kScatter ? cnt[(int64_t)i * tiles + blockIdx.x] : 0u;
+  __syncthreads();
+  const int64_t e0 = (int64_t)blockIdx.x * kDegTile;
+  int32_t v[kDegPer];
+#pragma unroll
+  for (int k = 0; k < kDegPer; ++k) {
+    const int64_t e = e0 + (int64_t)k * kDegThreads + threadIdx.x;
+    v[k] = e < m ? ci[e] : -1;
+  }
+#pragma unroll
+  for (int k = 0; k < kDegPer; ++k) {
+    const uint32_t at = wave_count_add<1>(s_n, v[k] >= 0 ? v[k] >> kDegBucketBits : -1);
+    if (kScatter && v[k] >= 0) low[at] = (uint16_t)(v[k] & ((1 << kDegBucketBits) - 1));
+  }
+  if (!kScatter) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < nb; i += kDegThreads) cnt[(int64_t)i * tiles + blockIdx.x] = s_n[i];
+  }
+}
+
+// Each block counts kDegPart consecutive bucketed ids (usually of one
+// bucket) in LDS and adds the counts to deg, which holds the out-degrees.
+__global__ __launch_bounds__(1024) void deg_count_kernel(const uint16_t* __restrict__ low, int64_t m, int64_t n, int nb,
+                                                         int64_t tiles, const uint32_t* __restrict__ cnt,
+                                                         uint32_t* __restrict__ deg) {
+  __shared__ uint32_t s_n[1 << kDegBucketBits];
+  const int64_t p0 = (int64_t)blockIdx.x * kDegPart, p1 = min(p0 + kDegPart, m);
+  int b = 0;
+  for (int hi = nb - 1; b < hi;) {  // the last bucket that starts at or before p0
+    const int mid = (b + hi + 1) >> 1;
+    if ((int64_t)cnt[mid * tiles] <= p0) b = mid;
+    else hi = mid - 1;
+  }
+  for (int64_t p = p0; p < p1; ++b) {
+    const int64_t q = b + 1 < nb ? min((int64_t)cnt[(b + 1) * tiles], p1) : p1;
+    if (q <= p) continue;
+    for (int i = threadIdx.x; i < 1 << kDegBucketBits; i += 1024) s_n[i] = 0u;
+    __syncthreads();
+    for (int64_t i = p + threadIdx.x; i < q; i += 1024) atomicAdd(&s_n[low[i]], 1u);
+    __syncthreads();
+    const int64_t v0 = (int64_t)b << kDegBucketBits;
+    for (int i = threadIdx.x; i < 1 << kDegBucketBits; i += 1024)
+      if (s_n[i]) atomicAdd(&deg[v0 + i], s_n[i]);
+    __syncthreads();
+    p = q;
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void deg_out_kernel(const int64_t* __restrict__ rp, int64_t n,
+                                                         uint32_t* __restrict__ deg) {
+  const int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (v < n) deg[v] = (uint32_t)(rp[v + 1] - rp[v]);
+}
+
+__global__ __launch_bounds__(1024) void deg_hist_kernel(const uint32_t* __restrict__ deg, int64_t n,
+                                                        uint32_t* __restrict__ hist) {
+  __shared__ uint32_t s_n[kDegCap];
+  for (int i = threadIdx.x; i < kDegCap; i += 1024) s_n[i] = 0u;
+  __syncthreads();
+  for (int64_t v = (int64_t)blockIdx.x * 1024 + threadIdx.x; v < n; v += (int64_t)gridDim.x * 1024) {
+    const uint32_t d = deg[v];
+    if (d >= (uint32_t)kDegCap) atomicAdd(&hist[kDegCap], 1u);
+    else if (d >= (uint32_t)kDegLeast) atomicAdd(&s_n[d], 1u);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kDegCap; i += 1024)
+    if (s_n[i]) atomicAdd(&hist[i], s_n[i]);
+}
+
+// hist[kDegCap + 1] = the smallest degree that at most kCoreIds vertices reach.
+// Also the class of every degree: eight classes to an octave of the number of
+// vertices above it, so that a class holds a like share of any list; equal
+// degrees share one.
+constexpr uint32_t kNoClass = 255;
+constexpr int kClasses = 128;
+__device__ __forceinline__ uint32_t degree_class(uint32_t above) {
+  if (above < 8) return above;
+  const int e = 31 - __builtin_clz(above);
+  return min((uint32_t)kClasses - 1u, 8u * (uint32_t)(e - 2) + (above >> (e - 3) & 7u));
+}
+__global__ __launch_bounds__(1024) void deg_threshold_kernel(uint32_t* hist, uint8_t* cls) {
+  __shared__ int64_t s_wave[16];
+  __shared__ uint32_t s_h[kDegCap];
+  __shared__ uint32_t s_t;
+  constexpr int kPer = kDegCap / 1024;
+  for (int i = threadIdx.x; i < kDegCap; i += 1024) s_h[i] = hist[i];
+  const uint32_t over = hist[kDegCap];
+  if (threadIdx.x == 0) {
+    s_t = over <= kCoreIds ? (uint32_t)kDegCap : 0xFFFFFFFFu;
+    cls[kDegCap] = 0;
+  }
+  __syncthreads();
+  const int top = kDegCap - 1 - (int)threadIdx.x * kPer;  // this thread's classes: top, top - 1, ...
+  int64_t t = 0;
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) t += s_h[top - k];
+  int64_t total;
+  int64_t run = over + block_excl_scan(t, s_wave, &total);
+  uint32_t least = 0xFFFFFFFFu;
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    cls[top - k] = (uint8_t)degree_class((uint32_t)min(run, (int64_t)0x7FFFFFFF));
+    run += s_h[top - k];
+    if (run <= kCoreIds && top - k >= kDegLeast) least = (uint32_t)(top - k);
+  }
+  if (least != 0xFFFFFFFFu) atomicMin(&s_t, least);
+  __syncthreads();
+  if (threadIdx.x == 0) hist[kDegCap + 1] = s_t;
+}
+
+// A scan's load and store: the vertices that reach the threshold, numbered;
+// their classes and codes.
+struct LoadCoded {
+  const uint32_t* deg;
+  const uint32_t* hist;
+  __device__ int64_t operator()(int64_t v) const { return deg[v] >= hist[kDegCap + 1] ? 1 : 0; }
+};
+struct StoreCode {
+  LoadCoded in;
+  const uint8_t* cls;
+  uint32_t* code;
+  __device__ void operator()(int64_t v, int64_t i) const {
+    code[v] = in(v) ? (uint32_t)cls[min(in.deg[v], (uint32_t)kDegCap)] << 16 | core_code((uint32_t)i, kCoreByteBits)
+                    : kNoClass << 16 | kNoCode;
+  }
+};
+
+// The block of rows of workgroup b of nb: b with its low three bits, which
+// pick its XCD, shifted by a hash of the others.  An R-MAT graph's heavy rows
+// are those whose ids have few bits set, so taken in order XCD 0 would get
+// 3.5 times its share of them.
+__device__ __forceinline__ int64_t spread_block(uint32_t b, uint32_t nb) {
+  const uint32_t j = b >> 3;
+  return 8 * (j + 1) <= nb ? 8 * (int64_t)j + ((b + (j * 0x9E3779B1u >> 29)) & 7u) : b;
+}
+
+// Codes, closed and ordered rows of at most kRankLeast ids, a group of
+// kBuildG lanes per row.
+__global__ __launch_bounds__(kBlock) void code_rows_kernel(const int64_t* __restrict__ rp, const int32_t* __restrict__ ci,
+                                                           int64_t n, const uint32_t* __restrict__ code,
+                                                           uint16_t* __restrict__ c16, uint8_t* __restrict__ closed,
+                                                           uint8_t* __restrict__ part) {
+  constexpr int kU = kRankLeast / kBuildG;
+  const int gl = threadIdx.x % kBuildG, sh = (threadIdx.x & 63) & ~(kBuildG - 1);
+  const int64_t v = (spread_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x) / kBuildG;
+  if (v >= n) return;
+  const int64_t e0 = rp[v];
+  const int d = (int)min(rp[v + 1] - e0, (int64_t)kRankLeast + 1);
+  if (d > kRankLeast) return;  // the whole group: rank_rows_kernel's
+  if (d == 0) {
+    if (gl == 0) closed[v] = kClosed | kOrdered;
+    return;
+  }
+  // lanes past the row's end load its last id again: no branch between loads
+  const uint32_t own = code[v] >> 16;
+  bool open = false, below = false;
+  int32_t w[kU];
+  uint32_t x[kU];
+#pragma unroll
+  for (int j = 0; j < kU; ++j) w[j] = ci[e0 + min(gl + j * kBuildG, d - 1)];
+#pragma unroll
+  for (int j = 0; j < kU; ++j) x[j] = code[w[j]];
+#pragma unroll
+  for (int j = 0; j < kU; ++j) {
+    if (gl + j * kBuildG >= d) continue;
+    const int64_t e = e0 + gl + j * kBuildG;
+    c16[code_start(e0, (uint32_t)d) + gl + j * kBuildG] = (uint16_t)x[j];
+    part[e] = (uint8_t)kPartAll;
+    open = open || x[j] >> 16 == kNoClass;
+    below = below || x[j] >> 16 > own;
+  }
+  const uint64_t mask = (1ull << kBuildG) - 1;
+  const bool any_open = (__ballot(open) >> sh & mask) != 0, any_below = (__ballot(below) >> sh & mask) != 0;
+  if (gl == 0) closed[v] = (uint8_t)((any_open ? 0 : kClosed) | (any_below ? 0 : kOrdered));
+}
+
+// The longer rows, a wave per row: a counting sort of the row by class in
+// LDS.  A wave takes kRankRows rows together (their lengths in one load);
+// rows of at most 64 * kRankKeep ids gather each id's class and code once.
+// (Few rows: vertices of high degree have neighbouring ids in an R-MAT graph,
+// and the waves that hold them finish last.)
+constexpr int kRankRows = 8;
+constexpr int kRankKeep = 4;
+__global__ __launch_bounds__(kBlock) void rank_rows_kernel(const int64_t* __restrict__ rp, const int32_t* __restrict__ ci,
+                                                           int64_t n, const uint32_t* __restrict__ code,
+                                                           uint16_t* __restrict__ c16, uint8_t* __restrict__ closed,
+                                                           uint8_t* __restrict__ part) {
+  __shared__ uint32_t s_cur[kWaves][kClasses + 1];
+  __shared__ uint8_t s_part[kWaves][kClasses + 1];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  uint32_t* cur = s_cur[wid];
+  uint8_t* upto = s_part[wid];  // part of the row's codes in each class and above
+  const int64_t v0 = (spread_block(blockIdx.x, gridDim.x) * kWaves + wid) * kRankRows;
+  int64_t re = 0;
+  if (lane <= kRankRows) re = rp[min(v0 + lane, n)];
+  const int64_t rn = __shfl_down(re, 1);
+  uint64_t todo = __ballot(lane < kRankRows && rn - re > kRankLeast);
+  while (todo) {
+    const int r = __builtin_ctzll(todo);
+    todo &= todo - 1;
+    const int64_t v = v0 + r, e0 = __shfl(re, r), d = __shfl(rn, r) - e0;
+    for (int i = lane; i <= kClasses; i += 64) cur[i] = 0;
+    wave_sync();
+    const uint32_t own = min(code[v] >> 16, (uint32_t)kClasses);
+    auto slot = [](uint32_t x) -> uint32_t { return min(x >> 16, (uint32_t)kClasses); };  // no code: last
+    // kKeep gathers in flight; lanes past the end load the last id again
+    uint32_t keep[kRankKeep];
+    auto gather = [&]<int kKeep>(std::integral_constant<int, kKeep>, int64_t i0) {
+      int32_t w[kKeep];
+#pragma unroll
+      for (int j = 0; j < kKeep; ++j) w[j] = ci[e0 + min(i0 + lane + j * 64, d - 1)];
+#pragma unroll
+      for (int j = 0; j < kKeep; ++j) keep[j] = code[w[j]];
+    };
+    auto count = [&](int64_t i0) {
+#pragma unroll
+      for (int j = 0; j < kRankKeep; ++j)
+        if (i0 + lane + j * 64 < d) atomicAdd(&cur[slot(keep[j])], 1u);
+    };
+    constexpr std::integral_constant<int, kRankKeep> all{};
+    if (d <= 128) gather(std::integral_constant<int, 2>{}, 0);
+    else gather(all, 0);
+    count(0);
+    for (int64_t i0 = 64 * kRankKeep; i0 < d; i0 += 64 * kRankKeep) {
+      gather(all, i0);
+      count(i0);
+    }
+    wave_sync();
+    const uint32_t a = cur[2 * lane], b = cur[2 * lane + 1];
+    const uint32_t incl = wave_incl_scan(a + b), excl = incl - a - b;
+    const uint32_t none = cur[kClasses], coded = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    wave_sync();
+    cur[2 * lane] = excl;
+    cur[2 * lane + 1] = excl + a;
+    // ceil(256 end / d) - 1, rounded up with room for the float's error
+    const float scale = 256.0f / (float)d;
+    auto up_to = [&](uint32_t end) { return (uint8_t)min(kPartAll, (uint32_t)((float)end * scale * 1.000001f)); };
+    upto[2 * lane] = up_to(excl + a);
+    upto[2 * lane + 1] = up_to(incl);
+    if (lane == 0) {
+      cur[kClasses] = coded;
+      upto[kClasses] = (uint8_t)kPartAll;
+    }
+    // none of the row's ids may be in a class below its own
+    const uint32_t below = __ballot((a != 0 && 2u * lane > own) || (b != 0 && 2u * lane + 1u > own)) != 0;
+    const bool ordered = !below && (none == 0 || own == (uint32_t)kClasses);
+    wave_sync();
+    const uint32_t base = code_start(e0, (uint32_t)d);
+    auto place = [&](uint32_t x, int64_t i) {
+      const uint32_t s = slot(x);
+      c16[base + atomicAdd(&cur[s], 1u)] = (uint16_t)x;
+      part[e0 + i] = upto[s];
+    };
+    for (int64_t i0 = 0; i0 < d; i0 += 64 * kRankKeep) {
+      if (d > 64 * kRankKeep) gather(all, i0);
+#pragma unroll
+      for (int j = 0; j < kRankKeep; ++j)
+        if (i0 + lane + j * 64 < d) place(keep[j], i0 + lane + j * 64);
+    }
+    if (lane == 0) closed[v] = (uint8_t)((none || d > kCoreIds ? 0 : kClosed) | (ordered ? kOrdered : 0));
+    wave_sync();
+  }
+}
+
+// *closed_edges = ids that name closed rows.
+__global__ __launch_bounds__(kBlock) void closed_edges_kernel(const int64_t* __restrict__ rp, int64_t n,
+                                                              const uint32_t* __restrict__ deg,
+                                                              const uint8_t* __restrict__ closed,
+                                                              unsigned long long* closed_edges) {
+  uint64_t named = 0;
+  for (int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x; v < n; v += (int64_t)gridDim.x * kBlock)
+    if (closed[v] & kClosed) named += deg[v] - (uint64_t)(rp[v + 1] - rp[v]);
+  __shared__ uint64_t s_red[kWaves];
+  const uint64_t sum = block_sum(named, s_red);
+  if (threadIdx.x == 0 && sum) atomicAdd(closed_edges, (unsigned long long)sum);
+}
+
+hipError_t launch_big_codes(const int64_t* rp, const int32_t* ci, int64_t n, int64_t m, char* scratch, uint16_t* c16,
+                            uint8_t* closed, uint8_t* part, unsigned long long* closed_edges, int cus, hipStream_t s) {
+  int64_t bytes;
+  const BigCodes x = big_codes_at(scratch, n, m, &bytes);
+  const int nb = (int)deg_buckets(n);
+  const int64_t tiles = deg_tiles(m), nc = nb * tiles + 1;
+  hipError_t e = launch_zero(x.cnt + nc - 1, 1, s);
+  if (e == hipSuccess) e = launch_zero(x.hist, kDegCap + 4, s);
+  if (e == hipSuccess) e = launch_zero(closed_edges, 2, s);
+  if (e != hipSuccess) return e;
+  const unsigned vblocks = (unsigned)((n + kBlock - 1) / kBlock);
+  deg_out_kernel<<<vblocks, kBlock, 0, s>>>(rp, n, x.deg);
+  deg_bucket_kernel<false><<<(unsigned)tiles, kDegThreads, 0, s>>>(ci, m, nb, tiles, x.cnt, x.low);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if ((e = launch_scan(LoadU32{x.cnt}, StoreU32{x.cnt}, nc, x.part, s)) != hipSuccess) return e;
+  deg_bucket_kernel<true><<<(unsigned)tiles, kDegThreads, 0, s>>>(ci, m, nb, tiles, x.cnt, x.low);
+  deg_count_kernel<<<(unsigned)((m + kDegPart - 1) / kDegPart), 1024, 0, s>>>(x.low, m, n, nb, tiles, x.cnt, x.deg);
+  deg_hist_kernel<<<(unsigned)std::min<int64_t>((n + 1023) / 1024, cus), 1024, 0, s>>>(x.deg, n, x.hist);
+  deg_threshold_kernel<<<1, 1024, 0, s>>>(x.hist, x.cls);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  const LoadCoded coded{x.deg, x.hist};
+  if ((e = launch_scan(coded, StoreCode{coded, x.cls, x.code}, n, x.part, s)) != hipSuccess) return e;
+  code_rows_kernel<<<(unsigned)((n * kBuildG + kBlock - 1) / kBlock), kBlock, 0, s>>>(rp, ci, n, x.code, c16, closed, part);
+  const int64_t per = kWaves * kRankRows;
+  rank_rows_kernel<<<(unsigned)((n + per - 1) / per), kBlock, 0, s>>>(rp, ci, n, x.code, c16, closed, part);
+  closed_edges_kernel<<<(unsigned)std::min<int64_t>((n + kBlock - 1) / kBlock, 4 * cus), kBlock, 0, s>>>(rp, n, x.deg, closed,
+                                                                                                 closed_edges);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -2169,7 +2827,7 @@ __global__ __launch_bounds__(kBlock) void local_parts_kernel(const int32_t* __re
 // ---------------------------------------------------------------------------
 struct __align__(16) PlainLds {
   int32_t A[kWaves][kCapWave];
-  int32_t End[kBlock];
+  uint32_t End[kBlock];
   gint32* Base[kBlock];
   uint64_t red[kWaves];
 };
@@ -2190,7 +2848,7 @@ __global__ __launch_bounds__(kBlock, TC_COUNT_WAVES_PER_EU) void plain_kernel(co
     const int da = (int)(rp[u + 1] - rb);
     if (da < 2 || (own && !own[u])) continue;
     constexpr int kModes = kModeTree | kModeHbm;
-    constexpr int kPlainInFlight = 6;
+    constexpr int kPlainInFlight = 2;
     if (da <= kCapWave - 1) {
       stage_tree(L.A[wid], ci + rb, da, lane, 64);
       wave_sync();
@@ -2299,13 +2957,13 @@ hipError_t launch_zero(void* p, int64_t words32, hipStream_t s) {
 
 __global__ void rearm_kernel(uint32_t* counters, uint64_t* outs, int32_t nouts) {
   const int i = threadIdx.x;
-  if (i < kNumBins) counters[kCntTileHead + i] = 0u;
+  if (i < kNumHeads) counters[kCntHeads + kHeadStride * i] = 0u;
   if (i == 0) counters[kCntFallback] = 0u;
   for (int j = i; j < nouts; j += blockDim.x) outs[j] = 0ull;
 }
 
 hipError_t launch_rearm(uint32_t* counters, uint64_t* outs, int32_t nouts, hipStream_t s) {
-  rearm_kernel<<<1, 64, 0, s>>>(counters, outs, nouts);
+  rearm_kernel<<<1, kBlock, 0, s>>>(counters, outs, nouts);
   return hipGetLastError();
 }
 
@@ -2335,17 +2993,39 @@ static int bin_blocks_per_cu() {
   return n;
 }
 
-// tiles >= 0: the bin's tile count is known on the host; the grid is then
-// capped at it, and an empty bin is not launched.
+// rows >= 0: the bin's row count is known on the host; the grid is then
+// capped at its tiles, and an empty bin is not launched.
 template <int BIN, int kLocal = kLocalNone>
-static void launch_bin(const LaunchArgs& a, int cus, int grid, hipStream_t s, int64_t tiles = -1) {
-  if (tiles == 0) return;
+static void launch_bin(const LaunchArgs& a, int cus, int grid, hipStream_t s, int64_t rows = -1) {
+  if (rows == 0) return;
   const bool wide = a.wide_ids != 0;
   int64_t g = grid > 0 ? grid
                        : (int64_t)(wide ? bin_blocks_per_cu<BIN, kLocal, true>() : bin_blocks_per_cu<BIN, kLocal, false>()) * cus;
-  if (tiles > 0 && tiles < g) g = tiles;
-  if (wide) count_kernel<BIN, kLocal, true><<<(unsigned)g, kBlock, 0, s>>>(a);
-  else count_kernel<BIN, kLocal, false><<<(unsigned)g, kBlock, 0, s>>>(a);
+  int rounds = 0;
+  if (rows > 0) {
+    rounds = tile_rounds(BIN, rows, g, a.tune.rounds);
+    const int64_t piv = tile_pivots(BIN, rounds), tiles = (rows + piv - 1) / piv;
+    if (tiles < g) g = tiles;
+  }
+  if (wide) count_kernel<BIN, kLocal, true><<<(unsigned)g, kBlock, 0, s>>>(a, rounds);
+  else count_kernel<BIN, kLocal, false><<<(unsigned)g, kBlock, 0, s>>>(a, rounds);
+}
+
+// The bitmap kernel of bins bin0..bin1, which use queue head `head`; rows as
+// for launch_bin.
+template <int NW>
+static int core_blocks_per_cu(int kb) {
+  int k = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, core_kernel<NW>, 64 * NW, (size_t)1 << kb) != hipSuccess) k = 1;
+  return k > 0 ? k : 1;
+}
+template <int NW>
+static void launch_core(const LaunchArgs& a, int cus, int grid, hipStream_t s, int64_t rows, int bin0, int bin1,
+                        int head) {
+  if (rows == 0) return;
+  int64_t g = grid > 0 ? grid : (int64_t)core_blocks_per_cu<NW>(a.core_kb) * cus;
+  if (rows > 0 && rows < g) g = rows;
+  core_kernel<NW><<<(unsigned)g, 64 * NW, (size_t)1 << a.core_kb, s>>>(a, bin0, bin1, head);
 }
 
 hipError_t launch_count(const LaunchArgs& a, int cus, int grid, hipStream_t s) {
@@ -2358,38 +3038,40 @@ hipError_t launch_count(const LaunchArgs& a, int cus, int grid, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_count_bins(const LaunchArgs& a, int cus, int grid, int first, int last, hipStream_t s) {
-  if (first <= BIN_GLOBAL && BIN_GLOBAL <= last) launch_bin<BIN_GLOBAL>(a, cus, grid, s);
-  if (first <= BIN_BLOCK && BIN_BLOCK <= last) launch_bin<BIN_BLOCK>(a, cus, grid, s);
-  if (first <= BIN_WAVE && BIN_WAVE <= last) launch_bin<BIN_WAVE>(a, cus, grid, s);
-  if (first <= BIN_G32 && BIN_G32 <= last) launch_bin<BIN_G32>(a, cus, grid, s);
-  if (first <= BIN_G16 && BIN_G16 <= last) launch_bin<BIN_G16>(a, cus, grid, s);
-  if (first <= BIN_G8 && BIN_G8 <= last) launch_bin<BIN_G8>(a, cus, grid, s);
-  return hipGetLastError();
-}
-
-hipError_t launch_count_sized(const LaunchArgs& a, int cus, int grid, const int64_t* tiles, hipStream_t s) {
-  launch_bin<BIN_GLOBAL>(a, cus, grid, s, tiles[BIN_GLOBAL]);
-  launch_bin<BIN_BLOCK>(a, cus, grid, s, tiles[BIN_BLOCK]);
-  launch_bin<BIN_WAVE>(a, cus, grid, s, tiles[BIN_WAVE]);
-  launch_bin<BIN_G32>(a, cus, grid, s, tiles[BIN_G32]);
-  launch_bin<BIN_G16>(a, cus, grid, s, tiles[BIN_G16]);
-  launch_bin<BIN_G8>(a, cus, grid, s, tiles[BIN_G8]);
-  return hipGetLastError();
+int core_last_bin(const LaunchArgs& a, const int64_t* rows) {
+  if (a.core == 0) return -1;
+  if (a.core != 1 || !rows) return BIN_WAVE;
+  int64_t light = 0;
+  for (int b = BIN_G32; b <= BIN_G8; ++b) light += rows[b];
+  return light <= kCoreLightRows ? BIN_G8 : BIN_WAVE;
 }
 
 hipError_t launch_count_order(const LaunchArgs& a, int cus, int grid, const int* order, int n,
-                              const int64_t* tiles, hipStream_t s) {
+                              const int64_t* rows, hipStream_t s) {
+  const int last = core_last_bin(a, rows);
   for (int i = 0; i < n; ++i) {
     const int b = order[i];
-    const int64_t t = tiles ? tiles[b] : -1;
+    const int64_t r = rows ? rows[b] : -1;
+    if (b <= last) {
+      auto sum = [&](int b0, int b1) {
+        int64_t x = 0;
+        for (int y = b0; y <= b1; ++y) x += rows[y];
+        return x;
+      };
+      if (b == BIN_BLOCK)
+        launch_core<kWaves>(a, cus, grid, s, rows ? sum(BIN_GLOBAL, BIN_BLOCK) : -1, BIN_GLOBAL, BIN_BLOCK,
+                            kCoreHead);
+      if (b == BIN_WAVE) launch_core<1>(a, cus, grid, s, rows ? sum(BIN_WAVE, last) : -1, BIN_WAVE, last,
+                                           kCoreHead + 1);
+      if (a.core == 1) continue;
+    }
     switch (b) {
-      case BIN_GLOBAL: launch_bin<BIN_GLOBAL>(a, cus, grid, s, t); break;
-      case BIN_BLOCK: launch_bin<BIN_BLOCK>(a, cus, grid, s, t); break;
-      case BIN_WAVE: launch_bin<BIN_WAVE>(a, cus, grid, s, t); break;
-      case BIN_G32: launch_bin<BIN_G32>(a, cus, grid, s, t); break;
-      case BIN_G16: launch_bin<BIN_G16>(a, cus, grid, s, t); break;
-      default: launch_bin<BIN_G8>(a, cus, grid, s, t); break;
+      case BIN_GLOBAL: launch_bin<BIN_GLOBAL>(a, cus, grid, s, r); break;
+      case BIN_BLOCK: launch_bin<BIN_BLOCK>(a, cus, grid, s, r); break;
+      case BIN_WAVE: launch_bin<BIN_WAVE>(a, cus, grid, s, r); break;
+      case BIN_G32: launch_bin<BIN_G32>(a, cus, grid, s, r); break;
+      case BIN_G16: launch_bin<BIN_G16>(a, cus, grid, s, r); break;
+      default: launch_bin<BIN_G8>(a, cus, grid, s, r); break;
     }
   }
   return hipGetLastError();
@@ -2461,8 +3143,8 @@ hipError_t launch_read(const void* src, int64_t bytes, uint32_t* sink, int grid,
 // static scratch of the allocation-free count
 // ---------------------------------------------------------------------------
 // Pieces (256-byte aligned): bin_of [slots] u16, items [slots] u64, blk
-// [bins * plan_blocks(slots) + 1] u32, scan partials of blk, counters [64]
-// u32, outs [16] u64.
+// [bins * plan_blocks(slots) + 1] u32, scan partials of blk, counters
+// u32, outs [kOutWords] u64.
 constexpr int64_t nalloc_up(int64_t b) { return (b + 255) & ~(int64_t)255; }
 constexpr int64_t kNaBlk = kNumBins * ((kNoAllocSlots + 255) / 256) + 1;
 constexpr int64_t kNaBinOf = 0;
@@ -2470,8 +3152,8 @@ constexpr int64_t kNaItems = kNaBinOf + nalloc_up(2 * kNoAllocSlots);
 constexpr int64_t kNaBlkOff = kNaItems + nalloc_up(8 * kNoAllocSlots);
 constexpr int64_t kNaPart = kNaBlkOff + nalloc_up(4 * kNaBlk);
 constexpr int64_t kNaCounters = kNaPart + nalloc_up(8 * ((kNaBlk + kScanChunk - 1) / kScanChunk + 1));
-constexpr int64_t kNaOuts = kNaCounters + nalloc_up(4 * 64);
-constexpr int64_t kNaBytes = kNaOuts + nalloc_up(8 * 16);
+constexpr int64_t kNaOuts = kNaCounters + nalloc_up(4 * kNumCounters);
+constexpr int64_t kNaBytes = kNaOuts + nalloc_up(8 * kOutWords);
 
 // The scratch itself.  Host code never passes this name to a kernel or a
 // copy: it is a host-side stand-in there.  tc_ctx_create takes its device

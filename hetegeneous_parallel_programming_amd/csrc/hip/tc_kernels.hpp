@@ -44,12 +44,26 @@ __host__ __device__ inline int tile_pivots(int bin, int rounds) {
   }
 }
 
-// Counter words of a plan (uint32).
+// Rows per group in the tiles of a light bin of `rows` rows on a grid of
+// `grid` workgroups: `most`, or fewer where the tiles would then not reach
+// every workgroup (a mid-size graph's few thousand light rows would run on a
+// few dozen of the 256 CUs).
+__host__ __device__ inline int tile_rounds(int bin, int64_t rows, int64_t grid, int most) {
+  const int64_t r = rows / (grid * tile_pivots(bin, 1));
+  return (int)(r < 1 ? 1 : most > 0 && r > most ? most : most < 1 ? 1 : r);
+}
+
+// Counter words of a plan (uint32).  The tile queue heads are a cache line
+// apart: the bins' kernels run side by side, and heads that share a line are
+// served one after another.
 constexpr int kCntBinCount = 0;                   // [kNumBins]
-constexpr int kCntBinCursor = kNumBins;           // [kNumBins]
-constexpr int kCntTileHead = 2 * kNumBins;        // [kNumBins] tile queue heads
-constexpr int kCntFallback = 3 * kNumBins + 2;    // hash builds that fell back to the tree
-constexpr int kNumCounters = 3 * kNumBins + 3;
+constexpr int kCntFallback = kNumBins;            // hash builds that fell back to the tree
+constexpr int kPlanWords = 32;                    // words up to here are read back
+constexpr int kCntHeads = 32;                     // queue head i: word kCntHeads + kHeadStride * i
+constexpr int kHeadStride = 32;
+constexpr int kNumHeads = kNumBins + 2;           // a bin's; then the bitmap kernels' two
+constexpr int kCoreHead = kNumBins;
+constexpr int kNumCounters = kCntHeads + kHeadStride * kNumHeads;
 
 // Partner rows.  Every DAG edge (u, v) is counted from the endpoint whose
 // out-list is longer: its "owner" x keeps N+(x) as the LDS set and its
@@ -60,6 +74,55 @@ constexpr int kNumCounters = 3 * kNumBins + 3;
 // ceil(count / kPartnersPerRow) "partner rows" (vrow[k] = x, partner ids
 // pci[vrp[k] .. vrp[k+1])), the unit of work of the count.
 constexpr int kPartnersPerRow = TCH_PARTNERS_PER_ROW;
+
+// Streamed ids are loaded kChunk at a time, so a load may begin at the last id
+// of a colidx pool: pools are allocated with kCiPad ids past their end (their
+// values never count).
+constexpr int kChunk = 4;
+constexpr int64_t kCiPad = kChunk;
+
+// Rows of a graph with codes: every id of the list has one; none of them
+// ranks below the row's own vertex.
+constexpr uint8_t kClosed = 1, kOrdered = 2;
+
+// 16-bit codes of vertices for the bitmap kernels.  A code's low 13 bits are
+// a byte of the bitmap, its high 3 bits a bit of that byte; a graph of n
+// vertices (at most kCoreIds) spreads them over 2^kb bytes, the fewest that
+// hold n bits.  Vertex i's code is the bit-reversed low kb + 3 bits of
+// i * kCodeMul (a bijection): the product's top bits pick the LDS bank, so
+// ids that share low bits, as an R-MAT graph's hubs do, do not share banks.
+// kNoCode is no vertex's code.
+constexpr int kCoreByteBits = 13;
+constexpr int64_t kCoreIds = 65535;
+constexpr int kCoreChunk = 8;               // codes per load
+constexpr int64_t kCorePad = 4096;          // codes allocated past a pool's end (see kCiPad)
+constexpr int64_t kCorePool = (int64_t)1 << 30;  // ids of a pool with codes: byte offsets stay 32-bit
+// Where the codes of the list of n ids at ci position p are: twice p, rounded
+// up to a multiple of the largest power of two within n (at most a 128-byte
+// line of codes).  That leaves every list inside [2p, 2p + 2n), so lists do
+// not overlap, and long lists start on a cache line, short ones on the word
+// that holds them (RMAT-22: the lines a count reads, 19.6 -> 17 GB).
+__host__ __device__ inline uint32_t code_start(int64_t p, uint32_t n) {
+  const uint32_t a = n >= 64 ? 64u : n >= 32 ? 32u : n >= 16 ? 16u : n >= 8 ? 8u : 1u;
+  return ((uint32_t)p * 2u + a - 1u) & ~(a - 1u);
+}
+constexpr uint32_t kCodeMul = 0x9E37u;      // odd, near 2^16 / phi
+__host__ __device__ constexpr uint32_t core_code(uint32_t i, int kb) {
+  uint32_t r = i * kCodeMul;
+  r = (r & 0x5555u) << 1 | (r >> 1 & 0x5555u);
+  r = (r & 0x3333u) << 2 | (r >> 2 & 0x3333u);
+  r = (r & 0x0F0Fu) << 4 | (r >> 4 & 0x0F0Fu);
+  r = (r & 0x00FFu) << 8 | (r >> 8 & 0x00FFu);  // 16 bits reversed
+  r >>= kCoreByteBits - kb;                     // kb + 3 bits reversed
+  return (r >> kb) << kCoreByteBits | (r & ((1u << kb) - 1u));
+}
+constexpr uint16_t kNoCode = (uint16_t)core_code(65535, kCoreByteBits);
+// Smallest kb for n vertices (the bitmap is cleared 16 bytes per lane of a wave).
+inline int core_bits(int64_t n) {
+  int kb = 10;
+  while (kb < kCoreByteBits && ((int64_t)8 << kb) < n) ++kb;
+  return kb;
+}
 
 // One graph of a (possibly single-graph) count.
 //   DAG: rowptr at rp_off of the rowptr pool (values relative to ci_off of
@@ -106,8 +169,14 @@ struct PlanBufs {
   uint32_t* blk;        // [kNumBins * nblk + 1] per-(bin, planning block) counts -> offsets
   int64_t* part;        // [scan_partials(kNumBins * nblk + 1)] scan partials
   uint32_t* counters;   // [kNumCounters]
-  uint64_t* outs;       // [ngraphs] u64 counts
+  uint64_t* outs;       // [ngraphs] u64 counts, or a single graph's kOutWords words
 };
+
+// A single graph's count is summed in kOutSlots words a cache line apart:
+// every workgroup ends with an add, and adds to one word are served one per
+// ~12 ns (8192 waves: 0.1 ms).
+constexpr int kOutSlots = 32, kOutStride = 16, kOutWords = kOutSlots * kOutStride;
+
 
 // A list of the DAG as one word: offset in the colidx pool in the high 39
 // bits, length in the low 25 (out-degrees are below 2^25 by the upload
@@ -117,12 +186,40 @@ constexpr int kLenBits = 25;
 __host__ __device__ inline ListRef list_ref(int64_t start, int64_t len) {
   return ((uint64_t)start << kLenBits) | (uint64_t)len;
 }
-__host__ __device__ inline int64_t list_start(ListRef r) { return (int64_t)(r >> kLenBits); }
-__host__ __device__ inline int32_t list_len(ListRef r) { return (int32_t)(r & ((1u << kLenBits) - 1)); }
+// A partner's list reference has two more bits on top (offsets stay below
+// 2^37): kRefClosed, every id of the list N+(v) of its edge's head v has a
+// 16-bit code, so that the edge can be counted over codes; kRefSlot, during a
+// build only.
+constexpr ListRef kRefSlot = 1ull << 63, kRefClosed = 1ull << 62;
+// (Tests of the marks look at the high word alone: 64-bit mask tests with a
+// mask in registers have compiled wrongly, and cost more.)
+__host__ __device__ inline uint32_t ref_marks(ListRef r, uint32_t mask) { return (uint32_t)(r >> 32) & mask; }
+constexpr uint32_t kMarkClosed = (uint32_t)(kRefClosed >> 32);
+// A closed edge's lists have at most kCoreIds ids, so its length field holds
+// the length in 16 bits and, above them, how much of the list's codes can
+// match: the codes are ordered by degree class, highest first, and the ids
+// past the first part(r) of them rank below the edge's head, so none of them
+// is in N+(head).
+constexpr uint32_t kPartAll = 255;
+__host__ __device__ inline ListRef closed_ref(int64_t start, int64_t len, uint32_t part) {
+  return kRefClosed | ((uint64_t)start << kLenBits) | (uint64_t)(part << 16) | (uint64_t)len;
+}
+__host__ __device__ inline int32_t list_len(ListRef r) {
+  return (int32_t)((uint32_t)r & (ref_marks(r, kMarkClosed) ? 0xFFFFu : (1u << kLenBits) - 1u));
+}
+// Codes to stream of a closed edge's list (part: 1/256 of its length, less 1).
+__host__ __device__ inline uint32_t closed_len(ListRef r) {
+  const uint32_t x = (uint32_t)r;
+  return ((x & 0xFFFFu) * ((x >> 16 & 0xFFu) + 1u) + 255u) >> 8;
+}
+__host__ __device__ inline int64_t list_start(ListRef r) { return (int64_t)(r << 2 >> (kLenBits + 2)); }
 
 // A partner row: the owner's list (the set; 0 for an unused slot), the
 // total length of its partners' lists (saturated at 2^32 - 1; only compared
-// with the bin thresholds) and its graph.
+// with the bin thresholds) and its graph, or where some of a single graph's
+// ids have codes (core 2) whether the row has edges marked kRefClosed
+// (kRowClosed) and others (kRowOpen).
+constexpr int32_t kRowClosed = 1, kRowOpen = 2;
 struct VRow {
   ListRef set;
   uint32_t work;
@@ -166,7 +263,13 @@ struct LaunchArgs {
   PlanBufs bufs;
   LocalOut local;
   const uint8_t* own;   // one graph only: null, or per row 1 if it is a pivot row
+  // Bitmap counting (see core_kernel): 16-bit codes of the ids of every list
+  // (at code_start); 2^core_kb bytes hold the bitmap of any set of codes.
+  const uint16_t* c16;
+  int32_t core;         // 0: no codes; 1: every id has one; 2: edges marked kRefClosed can use them
+  int32_t core_kb;
   int32_t wide_ids;     // 1 when ids reach 2^24: hash sets fold the high id bits into the bucket
+  int32_t out_slots;    // kOutSlots where bufs.outs holds a single graph's slots, else 0
   int32_t gbase;        // partner build of a segment of graphs: index of descs[0] among all graphs
 };
 
@@ -199,6 +302,9 @@ struct BuildBufs {
   int64_t* pedge;       // null, or [partner pool]: DAG edge position of each partner entry
   int32_t* pvid;        // with pedge: [partner pool] partner vertex of each entry
   int32_t* pown;        // null, or (one graph) [P] owner vertex of each partner row
+  uint16_t* codes;          // null, or where to write the codes of all ids (core_code, a.core_kb)
+  const uint8_t* closed;    // null, or (one graph) per row kClosed | kOrdered
+  const uint8_t* lpart;     // with closed: per DAG id e = (u, v), the part of u's codes that rank with v or above
   // Radix transpose (null when the scratch has no per-id part).  Build space:
   // M ids, graph g's at eb; row slots: RP.
   int32_t* gid;         // [RP] graph of each row slot; ~graph when the row is not split
@@ -310,17 +416,38 @@ hipError_t launch_stage_copy(const StageCopy* copies, int32_t n, int64_t chunks,
 // counter to 0 (bin counts kept), outs[0..nouts) to 0.
 hipError_t launch_rearm(uint32_t* counters, uint64_t* outs, int32_t nouts, hipStream_t s);
 hipError_t launch_plan(const LaunchArgs& a, hipStream_t s);
+// Bytes of the codes of a pool of ids.
+inline size_t code_bytes(int64_t ids) { return sizeof(uint16_t) * (size_t)(2 * ids + kCorePad); }
+// Codes for a graph of more than kCoreIds rows: the at most kCoreIds vertices
+// of highest degree (in the uploaded rows) get one.  c16: the codes of each
+// row's ids, at code_start; rows of more than kRankLeast ids have
+// theirs in order of degree class, highest first, ids without a code last.
+// closed[v]: kClosed | kOrdered; part[e]: see BuildBufs::lpart; *closed_edges = ids
+// that name closed rows.  scratch: big_codes_bytes(n, m) bytes.
+constexpr int kRankLeast = 32;
+constexpr int kDegBucketBits = 14;
+constexpr int64_t kDegBuckets = 1024;
+inline bool big_codes_fit(int64_t n, int64_t m) {
+  return n > kCoreIds && (n + ((int64_t)1 << kDegBucketBits) - 1) >> kDegBucketBits <= kDegBuckets && m > 0 && m < kCorePool;
+}
+int64_t big_codes_bytes(int64_t n, int64_t m);
+hipError_t launch_big_codes(const int64_t* rp, const int32_t* ci, int64_t n, int64_t m, char* scratch, uint16_t* c16,
+                            uint8_t* closed, uint8_t* part, unsigned long long* closed_edges, int cus, hipStream_t s);
 // One full-residency persistent launch per bin (grid > 0 overrides the size).
 hipError_t launch_count(const LaunchArgs& a, int cus, int grid, hipStream_t s);
-// Bins first..last only, each at full residency.
-hipError_t launch_count_bins(const LaunchArgs& a, int cus, int grid, int first, int last, hipStream_t s);
-// Same, with each bin's tile count known on the host (tiles[kNumBins]):
-// empty bins are skipped and no grid exceeds its bin's tiles.
-hipError_t launch_count_sized(const LaunchArgs& a, int cus, int grid, const int64_t* tiles, hipStream_t s);
-// Bins order[0..n) in that order, each at full residency or, with tiles
-// (tiles[kNumBins], known on the host), sized as launch_count_sized does.
+// Bins order[0..n) in that order, each at full residency or, with rows per
+// bin known on the host (rows[kNumBins]), skipped when empty and with no more
+// workgroups than tiles.
+// Bins 0..core_last_bin are counted by the bitmap kernels (-1: none): those of
+// the rows that keep a wave busy, or all bins of a graph with few light rows
+// (rows: per bin, null if not known), where one more wide launch beats three
+// narrow ones (R-MAT n=30011 d=24: 0.17 -> 0.10 ms) -- a wave per light row
+// is slower from a few rows per resident wave on (the batch of 512 graphs,
+// 215 K rows of the 32-lane bin: 0.53 ms there, 0.64 ms here).
+constexpr int64_t kCoreLightRows = 16384;
+int core_last_bin(const LaunchArgs& a, const int64_t* rows);
 hipError_t launch_count_order(const LaunchArgs& a, int cus, int grid, const int* order, int n,
-                              const int64_t* tiles, hipStream_t s);
+                              const int64_t* rows, hipStream_t s);
 
 // Stream groups of the bins: the groups run side by side (group 0 on the
 // library stream, the others on side streams), each group's bins one after

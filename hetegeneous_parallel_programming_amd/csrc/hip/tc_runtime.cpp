@@ -16,8 +16,15 @@ namespace tcr {
 
 static thread_local std::string g_err;
 // ctx->pinned layout (uint64 words): [0] count, [8..) plan counters,
-// [kPinnedFallback] the count's hash-fallback counter.
-constexpr int kPinnedFallback = 24;
+// [kPinnedFallback] the count's hash-fallback counter, [kPinnedOuts..) a
+// count's sum words.
+constexpr int kPinnedFallback = 24, kPinnedOuts = 64;
+constexpr size_t kPinnedBytes = sizeof(uint64_t) * (kPinnedOuts + tck::kOutWords);
+static uint64_t sum_outs(const tc_ctx* ctx) {
+  uint64_t t = 0;
+  for (int i = 0; i < tck::kOutSlots; ++i) t += ctx->pinned[kPinnedOuts + i * tck::kOutStride];
+  return t;
+}
 
 tc_status fail(tc_status st, const std::string& msg) {
   g_err = msg;
@@ -61,7 +68,7 @@ void dev_free(void* p) {
 
 tc_status PlanScratch::ensure(int64_t pivots, int64_t nouts) {
   if (!counters) {
-    tc_status st = dev_alloc((void**)&counters, sizeof(uint32_t) * 64, "plan counters");
+    tc_status st = dev_alloc((void**)&counters, sizeof(uint32_t) * tck::kNumCounters, "plan counters");
     if (st != TC_OK) return st;
   }
   if (pivots > cap) {
@@ -233,7 +240,8 @@ void BuildScratch::release() {
 }
 
 tc_status launch_build(const tck::LaunchArgs& a, int64_t RP, int64_t M, BuildScratch& bs, hipStream_t s,
-                       const LocalBufs* loc, int32_t* pown) {
+                       const LocalBufs* loc, int32_t* pown, const uint8_t* closed,
+                       const uint8_t* part, uint16_t* codes) {
   // The local rebuild also writes each entry's edge position and partner
   // vertex: the radix path carries the positions along (one graph, its
   // edges' rows in loc->esrc, filled before); the per-edge atomic path
@@ -243,6 +251,9 @@ tc_status launch_build(const tck::LaunchArgs& a, int64_t RP, int64_t M, BuildScr
   if (st != TC_OK) return st;
   bs.b.pedge = loc ? loc->pedge : nullptr;
   bs.b.pvid = loc ? loc->pvid : nullptr;
+  bs.b.codes = codes;
+  bs.b.closed = closed;
+  bs.b.lpart = part;
   bs.b.pown = pown;  // one graph: each partner row's owner
   bs.b.esrc = loc ? loc->esrc : nullptr;
   TC_HIP_TRY(tck::launch_partners(a, RP, M, bs.b, s));
@@ -301,6 +312,10 @@ static tc_status check_dag(const tc_csr_view* dag, uint32_t check, int32_t* max_
   return TC_OK;
 }
 
+// Graphs past tck::kCoreIds rows get codes only when some list is this long:
+// flat ones have no set of 65535 vertices that most edges lead to.
+constexpr int32_t kCodesMinOut = 64;
+
 static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_begin, int32_t row_end,
                             const uint8_t* owned, int32_t max_out, tc_graph** out) {
   std::unique_ptr<tc_graph> g(new tc_graph);
@@ -316,6 +331,7 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
   auto cleanup = [&]() {
     dev_free(g->rp);
     dev_free(g->ci);
+    g->drop_codes();
     dev_free(g->d_desc);
     dev_free(g->own);
     dev_free(g->pown);
@@ -324,7 +340,7 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
   tc_status st = dev_alloc((void**)&g->rp, sizeof(int64_t) * ((size_t)g->n + 1), "rowptr");
   if (st == TC_OK && owned)
     st = dev_alloc((void**)&g->own, std::max<size_t>((size_t)g->n, 1), "owned-row mask");
-  if (st == TC_OK) st = dev_alloc((void**)&g->ci, sizeof(int32_t) * (size_t)std::max<int64_t>(g->nnz, 1), "colidx");
+  if (st == TC_OK) st = dev_alloc((void**)&g->ci, sizeof(int32_t) * (size_t)(g->nnz + tck::kCiPad), "colidx");
   if (st == TC_OK) st = dev_alloc((void**)&g->d_desc, sizeof(tck::GraphDesc), "graph desc");
   if (st == TC_OK) st = g->partners.alloc(g->nnz, (int64_t)g->nv_max + 1, 1);
   if (st == TC_OK)
@@ -332,6 +348,17 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
   if (st != TC_OK) {
     cleanup();
     return st;
+  }
+  // The bitmap kernels' codes, which a count can do without: none where there
+  // is no memory for them.
+  bool big = max_out >= kCodesMinOut && tck::big_codes_fit(g->n, g->nnz);
+  if (big || (g->n <= tck::kCoreIds && g->nnz < tck::kCorePool)) {
+    st = dev_alloc((void**)&g->c16, tck::code_bytes(g->nnz), "id codes");
+    if (st == TC_OK && big) st = dev_alloc((void**)&g->closed, (size_t)g->n, "closed rows");
+    if (st == TC_OK && big) st = dev_alloc((void**)&g->part, (size_t)g->nnz, "code parts");
+    if (st != TC_OK) g->drop_codes();
+    big = big && st == TC_OK;
+    st = TC_OK;
   }
   const tck::GraphDesc d{0, 0, 0, 0, 0, g->n, g->nv_max, row_begin, row_end, 0};
   hipError_t e = hipMemcpy(g->rp, dag->rowptr, sizeof(int64_t) * ((size_t)g->n + 1), hipMemcpyHostToDevice);
@@ -356,16 +383,27 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
   hipStream_t s = ctx->stream;
   // the scratch is allocated before the timed span: build_ms is the device's build
   st = bs.ensure((int64_t)g->n + 1, g->nnz);
+  if (big && tck::big_codes_bytes(g->n, g->nnz) > bs.cap) {
+    g->drop_codes();
+    big = false;
+  }
   if (st != TC_OK) {
     cleanup();
     return st;
   }
   e = hipEventRecord(ctx->ev[0], s);
   if (e == hipSuccess) {
-    st = launch_build(a, (int64_t)g->n + 1, g->nnz, bs, s, nullptr, g->pown);
-    if (st == TC_OK) e = hipEventRecord(ctx->ev[1], s);
+    a.core_kb = tck::core_bits(g->n);
+    if (big)  // (the build's scratch is free until the build)
+      e = tck::launch_big_codes(g->rp, g->ci, g->n, g->nnz, bs.mem, g->c16, g->closed, g->part,
+                                (unsigned long long*)ctx->plain_out + 4, ctx->cus, s);
+    if (e == hipSuccess) st = launch_build(a, (int64_t)g->n + 1, g->nnz, bs, s, nullptr, g->pown, g->closed, g->part,
+                                             big ? nullptr : g->c16);
+    if (st == TC_OK && e == hipSuccess) e = hipEventRecord(ctx->ev[1], s);
     if (st == TC_OK && e == hipSuccess)
       e = hipMemcpyAsync(ctx->pinned, g->partners.nv, sizeof(int32_t), hipMemcpyDeviceToHost, s);
+    if (big && st == TC_OK && e == hipSuccess)
+      e = hipMemcpyAsync(ctx->pinned + 1, ctx->plain_out + 4, sizeof(uint64_t), hipMemcpyDeviceToHost, s);
     if (st == TC_OK && e == hipSuccess) e = hipStreamSynchronize(s);
   }
   bs.release();
@@ -378,8 +416,10 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
   (void)hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]);
   g->build_ms = ms;
   g->nv = *(const int32_t*)ctx->pinned;
+  g->coded = big ? 4 * (int64_t)ctx->pinned[1] >= g->nnz : g->c16 != nullptr;
   g->bytes = sizeof(int64_t) * ((int64_t)g->n + 1) + sizeof(int32_t) * g->nnz + sizeof(tck::GraphDesc) +
-             g->partners.bytes + (owned ? (int64_t)g->n : 0) + sizeof(int32_t) * ((int64_t)g->nv_max + 1);
+             g->partners.bytes + (owned ? (int64_t)g->n : 0) + (g->c16 ? (int64_t)tck::code_bytes(g->nnz) : 0) +
+             (big ? (int64_t)g->n + g->nnz : 0) + sizeof(int32_t) * ((int64_t)g->nv_max + 1);
   *out = g.release();
   return TC_OK;
 }
@@ -437,7 +477,7 @@ tc_status tc_ctx_create(int32_t device, tc_ctx** out) try {
   }
   TC_HIP_TRY(hipEventCreateWithFlags(&c->fork, hipEventDisableTiming));
   for (auto& ev : c->ev) TC_HIP_TRY(hipEventCreate(&ev));
-  TC_HIP_TRY(hipHostMalloc((void**)&c->pinned, 4096, hipHostMallocDefault));
+  TC_HIP_TRY(hipHostMalloc((void**)&c->pinned, kPinnedBytes, hipHostMallocDefault));
   {
     tc_status st = dev_alloc((void**)&c->plain_out, 256, "plain count word");
     if (st != TC_OK) return st;
@@ -560,6 +600,7 @@ tc_status tc_graph_free(tc_ctx* ctx, tc_graph* g) try {
   (void)hipStreamSynchronize(c->stream);
   dev_free(g->rp);
   dev_free(g->ci);
+  g->drop_codes();
   dev_free(g->d_desc);
   dev_free(g->own);
   dev_free(g->pown);
@@ -599,7 +640,11 @@ static tck::LaunchArgs count_args(tc_ctx* ctx, tc_graph* g) {
   g->partners.into(a);
   a.tune = to_kernel_tune(ctx->tune);
   a.bufs = ctx->scratch.bufs();
+  a.out_slots = tck::kOutSlots;
   a.own = g->own;
+  a.c16 = g->c16;
+  a.core = !g->coded ? 0 : g->closed ? 2 : 1;
+  a.core_kb = tck::core_bits(g->n);
   a.wide_ids = g->n > tck::kNarrowIds ? 1 : 0;
   return a;
 }
@@ -616,37 +661,32 @@ static int first_group(const bool* any, int n) {
 }
 
 // The binned count over plan buffers `bufs`.  kept: the plan in bufs is
-// already built for this graph and tune (its rows per bin in bins[], tiles
-// per bin in tiles[]): re-arm the tile queues and count.  Otherwise plan
-// first (one host round trip for the rows per bin, which size the launches)
-// and fill bins[] and tiles[].
+// already built for this graph and tune (its rows per bin in bins[]): re-arm
+// the tile queues and count.  Otherwise plan first (one host round trip for
+// the rows per bin, which size the launches) and fill bins[].
 static tc_status binned_count(tc_ctx* ctx, tc_graph* g, const tck::PlanBufs& bufs, bool kept, int64_t* bins,
-                              int64_t* tiles, uint64_t* total, tc_stats* stats) {
+                              uint64_t* total, tc_stats* stats) {
   const double t0 = now_ms();
   tck::LaunchArgs a = count_args(ctx, g);
   a.bufs = bufs;
   hipStream_t s = ctx->stream;
   TC_HIP_TRY(hipEventRecord(ctx->ev[0], s));
   if (kept) {
-    TC_HIP_TRY(tck::launch_rearm(a.bufs.counters, a.bufs.outs, 2, s));
+    TC_HIP_TRY(tck::launch_rearm(a.bufs.counters, a.bufs.outs, tck::kOutWords, s));
     TC_HIP_TRY(hipEventRecord(ctx->ev[3], s));
   } else {
     TC_HIP_TRY(tck::launch_zero(a.bufs.counters, tck::kNumCounters, s));
-    TC_HIP_TRY(tck::launch_zero(a.bufs.outs, 2, s));
+    TC_HIP_TRY(tck::launch_zero(a.bufs.outs, 2 * tck::kOutWords, s));
     TC_HIP_TRY(tck::launch_plan(a, s));
     TC_HIP_TRY(hipEventRecord(ctx->ev[3], s));
     // The plan's rows per bin size each bin's launch: empty bins are skipped
     // and small ones get no more workgroups than tiles (a small graph would
     // otherwise pay for six full-residency grids).
-    TC_HIP_TRY(hipMemcpyAsync(ctx->pinned + 8, a.bufs.counters, sizeof(uint32_t) * tck::kNumCounters,
+    TC_HIP_TRY(hipMemcpyAsync(ctx->pinned + 8, a.bufs.counters, sizeof(uint32_t) * tck::kPlanWords,
                               hipMemcpyDeviceToHost, s));
     TC_HIP_TRY(hipStreamSynchronize(s));
     const uint32_t* c = (const uint32_t*)(ctx->pinned + 8);
-    for (int b = 0; b < tck::kNumBins; ++b) {
-      const int64_t piv = tck::tile_pivots(b, ctx->tune.rounds > 0 ? ctx->tune.rounds : 1);
-      bins[b] = c[tck::kCntBinCount + b];
-      tiles[b] = (bins[b] + piv - 1) / piv;
-    }
+    for (int b = 0; b < tck::kNumBins; ++b) bins[b] = c[tck::kCntBinCount + b];
   }
   TC_HIP_TRY(hipEventRecord(ctx->ev[1], s));
   // The bin groups (tck::kBinOrder) run on separate streams (default
@@ -657,8 +697,14 @@ static tc_status binned_count(tc_ctx* ctx, tc_graph* g, const tck::PlanBufs& buf
   // stream alone.
   const tck::BinGroups& G = tck::kBinOrder;
   bool any[tck::kBinGroups] = {};
+  const int last = tck::core_last_bin(a, bins);
   for (int gi = 0; gi < G.n; ++gi)
-    for (int j = 0; j < G.len[gi]; ++j) any[gi] = any[gi] || tiles[G.bin[gi][j]] > 0;
+    for (int j = 0; j < G.len[gi]; ++j) {
+      const int b = G.bin[gi][j];
+      int64_t rows = b > tck::BIN_WAVE && b <= last ? 0 : bins[b];  // counted with the wave bin's
+      for (int x = tck::BIN_WAVE + 1; b == tck::BIN_WAVE && x <= last; ++x) rows += bins[x];
+      any[gi] = any[gi] || rows > 0;
+    }
   const int g0 = first_group(any, G.n);
   int side = 0;
   for (int gi = 0; gi < G.n; ++gi) {
@@ -668,18 +714,19 @@ static tc_status binned_count(tc_ctx* ctx, tc_graph* g, const tck::PlanBufs& buf
       gs = ctx->side[side++];
       TC_HIP_TRY(hipStreamWaitEvent(gs, ctx->ev[1], 0));  // timing starts before any group
     }
-    TC_HIP_TRY(tck::launch_count_order(a, ctx->cus, ctx->tune.grid, G.bin[gi], G.len[gi], tiles, gs));
+    TC_HIP_TRY(tck::launch_count_order(a, ctx->cus, ctx->tune.grid, G.bin[gi], G.len[gi], bins, gs));
   }
   for (int i = 0; i < side; ++i) {
     TC_HIP_TRY(hipEventRecord(ctx->join[i], ctx->side[i]));
     TC_HIP_TRY(hipStreamWaitEvent(s, ctx->join[i], 0));
   }
   TC_HIP_TRY(hipEventRecord(ctx->ev[2], s));
-  TC_HIP_TRY(hipMemcpyAsync(ctx->pinned, a.bufs.outs, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+  TC_HIP_TRY(hipMemcpyAsync(ctx->pinned + kPinnedOuts, a.bufs.outs, sizeof(uint64_t) * tck::kOutWords,
+                            hipMemcpyDeviceToHost, s));
   TC_HIP_TRY(hipMemcpyAsync(ctx->pinned + kPinnedFallback, a.bufs.counters + tck::kCntFallback, sizeof(uint32_t),
                             hipMemcpyDeviceToHost, s));
   TC_HIP_TRY(hipStreamSynchronize(s));
-  *total = ctx->pinned[0];
+  *total = sum_outs(ctx);
   if (stats) {
     std::memset(stats, 0, sizeof(*stats));
     stats->total_ms = now_ms() - t0;
@@ -706,12 +753,12 @@ static tc_status count_binned(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_stat
   const bool kept = g->plan_valid && std::memcmp(&g->plan_tune, &ctx->tune, sizeof(tc_tune)) == 0;
   if (!kept) {
     const int64_t had = g->plan.cap;
-    tc_status st = g->plan.ensure(P, 1);
+    tc_status st = g->plan.ensure(P, tck::kOutWords);
     if (st != TC_OK) return st;
     if (g->plan.cap != had) g->bytes += PlanScratch::bytes_for(g->plan.cap) - (had ? PlanScratch::bytes_for(had) : 0);
     g->plan_valid = false;
   }
-  tc_status st = binned_count(ctx, g, g->plan.bufs(), kept, g->plan_bins, g->plan_tiles, total, stats);
+  tc_status st = binned_count(ctx, g, g->plan.bufs(), kept, g->plan_bins, total, stats);
   if (st == TC_OK && !kept) {
     g->plan_tune = ctx->tune;
     g->plan_valid = true;
@@ -830,7 +877,7 @@ tc_status tc_count_csr(tc_ctx* ctx, const tc_csr_view* dag, uint32_t check, uint
   if (!small && !tcr::plain_fits(dag->n_rows, dag->nnz, max_out)) return whole();
   const size_t rp_bytes = sizeof(int64_t) * ((size_t)dag->n_rows + 1);
   const size_t ci_off = (rp_bytes + 255) & ~(size_t)255;
-  const size_t bytes = ci_off + sizeof(int32_t) * (size_t)std::max<int64_t>(dag->nnz, 1);
+  const size_t bytes = ci_off + sizeof(int32_t) * (size_t)(dag->nnz + tck::kCiPad);
   if (bytes > ctx->once_cap) {
     dev_free(ctx->once_dev);
     ctx->once_dev = nullptr;
@@ -902,8 +949,8 @@ tc_status tc_count_noalloc(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_stats* 
     return fail(TC_ERANGE, "tc_count_noalloc: the graph needs " + std::to_string(P) +
                                " plan slots (rows + ids/1024 + 2); the static scratch holds " +
                                std::to_string(tck::kNoAllocSlots));
-  int64_t bins[tck::kNumBins], tiles[tck::kNumBins];
-  return binned_count(ctx, g, bufs, false, bins, tiles, total, stats);
+  int64_t bins[tck::kNumBins];
+  return binned_count(ctx, g, bufs, false, bins, total, stats);
 } catch (...) {
   return tcr::caught();
 }
@@ -941,7 +988,7 @@ static tc_status ensure_local(tc_ctx* ctx, tc_graph* g) {
     tck::LaunchArgs a = count_args(ctx, g);
     BuildScratch bs;
     hipError_t e = tck::launch_local_prep(g->rp, g->n, L.esrc, ctx->stream);  // the rebuild reads and marks esrc
-    if (e == hipSuccess) st = launch_build(a, (int64_t)g->n + 1, g->nnz, bs, ctx->stream, &L, g->pown);
+    if (e == hipSuccess) st = launch_build(a, (int64_t)g->n + 1, g->nnz, bs, ctx->stream, &L, g->pown, g->closed, g->part);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     bs.release();
     if (st == TC_OK && e != hipSuccess)
@@ -979,7 +1026,7 @@ tc_status tc_count_local(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_local* ou
   const bool vertices = out->vertex_counts != nullptr;
   const bool parts_only = k > 0 && !vertices && !out->edge_counts;
   const int mode = vertices ? tck::kLocalFull : parts_only ? tck::kLocalParts : tck::kLocalEdges;
-  tc_status st = ctx->scratch.ensure(P, 1);
+  tc_status st = ctx->scratch.ensure(P, tck::kOutWords);
   if (st == TC_OK) st = parts_only ? ensure_split(g->local) : ensure_local(ctx, g);
   if (st != TC_OK) return st;
   LocalBufs& L = g->local;
@@ -993,7 +1040,7 @@ tc_status tc_count_local(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_local* ou
     TC_HIP_TRY(hipMemcpyAsync(L.bounds, out->bounds, sizeof(int32_t) * ((size_t)k + 1), hipMemcpyHostToDevice, s));
   TC_HIP_TRY(hipEventRecord(ctx->ev[0], s));
   TC_HIP_TRY(tck::launch_zero(a.bufs.counters, tck::kNumCounters, s));
-  TC_HIP_TRY(tck::launch_zero(a.bufs.outs, 2, s));
+  TC_HIP_TRY(tck::launch_zero(a.bufs.outs, 2 * tck::kOutWords, s));
   if (!parts_only) TC_HIP_TRY(tck::launch_zero(L.ecount, std::max<int64_t>(g->nnz, 1), s));
   if (vertices) TC_HIP_TRY(tck::launch_zero(L.vcount, 2 * ((int64_t)g->n + 1), s));
   TC_HIP_TRY(tck::launch_zero(L.pe, 2 * (int64_t)tck::kMaxParts, s));
@@ -1014,11 +1061,12 @@ tc_status tc_count_local(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_local* ou
     TC_HIP_TRY(tck::launch_local_parts(g->ci, L.esrc, g->n, g->edge_begin, g->edge_end, L.ecount, L.bounds, k, L.pe,
                                        ctx->cus, s));
   TC_HIP_TRY(hipEventRecord(ctx->ev[2], s));
-  TC_HIP_TRY(hipMemcpyAsync(ctx->pinned, a.bufs.outs, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
-  TC_HIP_TRY(hipMemcpyAsync(ctx->pinned + 8, a.bufs.counters, sizeof(uint32_t) * tck::kNumCounters,
+  TC_HIP_TRY(hipMemcpyAsync(ctx->pinned + kPinnedOuts, a.bufs.outs, sizeof(uint64_t) * tck::kOutWords,
+                            hipMemcpyDeviceToHost, s));
+  TC_HIP_TRY(hipMemcpyAsync(ctx->pinned + 8, a.bufs.counters, sizeof(uint32_t) * tck::kPlanWords,
                             hipMemcpyDeviceToHost, s));
   TC_HIP_TRY(hipStreamSynchronize(s));
-  *total = ctx->pinned[0];
+  *total = sum_outs(ctx);
   const int64_t fallbacks = ((const uint32_t*)(ctx->pinned + 8))[tck::kCntFallback];
   // pageable destinations: synchronous copies after the stream is done
   if (out->edge_counts && g->edge_end > g->edge_begin)

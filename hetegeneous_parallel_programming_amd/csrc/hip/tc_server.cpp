@@ -568,7 +568,7 @@ tc_status tc_server_create(tc_ctx* ctx, const tc_server_config* cfg, tc_server**
   const int64_t nb = tck::kNumBins * tck::plan_blocks(R) + 1;
   const uint64_t o_items = 0, o_bin = o_items + align_up(8 * R), o_blk = o_bin + align_up(2 * R),
                  o_part = o_blk + align_up(4 * nb), o_cnt = o_part + align_up(8 * tck::scan_partials(nb)),
-                 o_outs = o_cnt + align_up(4 * 64), o_desc = o_outs + align_up(8 * G),
+                 o_outs = o_cnt + align_up(4 * tck::kNumCounters), o_desc = o_outs + align_up(8 * G),
                  o_nv = o_desc + align_up(sizeof(tck::GraphDesc) * G) + align_up(sizeof(tck::StageCopy) * G),
                  o_vrow = o_nv + align_up(4 * G),
                  o_vrp = o_vrow + align_up(sizeof(tck::VRow) * R), total = o_vrp + align_up(8 * (R + 1));
