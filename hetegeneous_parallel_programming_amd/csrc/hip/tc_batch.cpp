@@ -75,19 +75,19 @@ static tc_status capture(tc_ctx* ctx, tc_batch* b) {
   hipError_t e = tck::launch_zero(a.bufs.counters, tck::kNumCounters, s);
   if (e == hipSuccess) e = tck::launch_zero(a.bufs.outs, 2 * (int64_t)b->n, s);
   if (e == hipSuccess) e = tck::launch_plan(a, s);
-  // The bin groups (tck::kBinOrder): group 0 on the capture stream, the
-  // others on forked branches, whose workgroups fill the CUs the other
-  // groups' tails free.
-  static_assert(tck::kBinGroups == tc_ctx::kSides + 1, "one side stream per bin group past the first");
-  const tck::BinGroups& G = tck::kBinOrder;
+  // The first part on the capture stream, the others on forked branches.
+  static_assert(tck::kCountParts == tc_ctx::kSides + 1, "one side stream per part past the first");
   if (e == hipSuccess) e = hipEventRecord(ctx->fork, s);
-  for (int i = 1; i < G.n && e == hipSuccess; ++i) e = hipStreamWaitEvent(ctx->side[i - 1], ctx->fork, 0);
-  for (int i = 0; i < G.n && e == hipSuccess; ++i)
-    e = tck::launch_count_order(a, ctx->cus, ctx->tune.grid, G.bin[i], G.len[i], nullptr,
-                                i == 0 ? s : ctx->side[i - 1]);
-  for (int i = 1; i < G.n && e == hipSuccess; ++i) {
-    e = hipEventRecord(ctx->join[i - 1], ctx->side[i - 1]);
-    if (e == hipSuccess) e = hipStreamWaitEvent(s, ctx->join[i - 1], 0);
+  int side = -1;
+  for (int p = 0; p < tck::kCountParts && e == hipSuccess; ++p) {
+    if (tck::part_empty(a, p, nullptr)) continue;
+    if (++side > 0) e = hipStreamWaitEvent(ctx->side[side - 1], ctx->fork, 0);
+    if (e == hipSuccess)
+      e = tck::launch_count_part(a, ctx->cus, ctx->tune.grid, p, nullptr, side == 0 ? s : ctx->side[side - 1]);
+  }
+  for (int i = 0; i < side && e == hipSuccess; ++i) {
+    e = hipEventRecord(ctx->join[i], ctx->side[i]);
+    if (e == hipSuccess) e = hipStreamWaitEvent(s, ctx->join[i], 0);
   }
   if (e == hipSuccess)
     e = hipMemcpyAsync(b->pinned, a.bufs.outs, sizeof(uint64_t) * (size_t)b->n, hipMemcpyDeviceToHost, s);

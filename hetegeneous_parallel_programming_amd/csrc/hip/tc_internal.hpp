@@ -114,7 +114,7 @@ struct BuildScratch {
 // partner vertex and each partner row's owner (pedge, pvid, pown).
 tc_status launch_build(const tck::LaunchArgs& a, int64_t RP, int64_t M, BuildScratch& bs, hipStream_t s,
                        const LocalBufs* loc = nullptr, int32_t* pown = nullptr, const uint8_t* closed = nullptr,
-                       const uint8_t* part = nullptr, uint16_t* codes = nullptr);
+                       const uint8_t* part = nullptr, uint16_t* codes = nullptr, int32_t* lines = nullptr);
 
 // Makes ctx's device current for the scope of one API call.
 struct DeviceGuard {
@@ -138,10 +138,10 @@ tc_tune default_tune();
 struct tc_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
-  // Bin groups 1.. of a count run on side streams beside group 0 on
-  // `stream` (default priority); join[i]: side stream i done, fork: side
-  // streams may start (events without timing).
-  static constexpr int kSides = 3;
+  // A count's parts past the first run on side streams beside `stream`
+  // (default priority); join[i]: side stream i done, fork: side streams may
+  // start (events without timing).
+  static constexpr int kSides = 2;
   hipStream_t side[kSides] = {};
   hipEvent_t join[kSides] = {};
   hipEvent_t fork = nullptr;
@@ -177,6 +177,7 @@ struct tc_graph {
   int32_t row_begin = 0, row_end = 0;
   int64_t edge_begin = 0, edge_end = 0;  // DAG edge positions of rows [row_begin, row_end)
   uint8_t* own = nullptr;                 // null, or per row 1 if it is a pivot row
+  int32_t* lines = nullptr; // ci with its lists on cache lines (null: none)
   uint16_t* c16 = nullptr;  // 16-bit codes of ci for the bitmap kernels (null: none)
   uint8_t* closed = nullptr;  // with c16, over kCoreIds rows: tck::BuildBufs::closed
   uint8_t* part = nullptr;    // with closed: tck::BuildBufs::lpart

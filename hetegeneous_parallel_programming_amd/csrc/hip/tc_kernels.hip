@@ -436,11 +436,13 @@ struct DagEdges {
 };
 struct RefEdges {
   const ListRef* refs;
+  bool lines;     // lists are at line_start of their position
   uint32_t skip;  // edges with this mark are counted elsewhere
   __device__ __forceinline__ void operator()(int j, int64_t& b, int& c) const {
     const ListRef r = refs[j];
-    b = list_start(r);
-    c = ref_marks(r, skip) ? 0 : list_len(r);
+    c = list_len(r);
+    b = lines ? line_start(list_start(r), c) : list_start(r);
+    if (ref_marks(r, skip)) c = 0;
   }
 };
 
@@ -1208,14 +1210,14 @@ __global__ __launch_bounds__(kBlock) void radix_split_kernel(LaunchArgs a, int64
     if (R[s] < 0) continue;
     const int64_t E = j0 + (int64_t)s * kBlock + threadIdx.x;
     const int gr = s_gid[R[s]];
-    auto put_code = [&](int64_t x, int32_t v) {  // every id's code is a function of the id: written on the way
-      const int32_t at = (int32_t)(E - ebase - s_erow[R[s]]);
-      b.codes[code_start(x - at, (uint32_t)(s_erow[R[s] + 1] - s_erow[R[s]])) + at] =
-          (uint16_t)core_code((uint32_t)v, a.core_kb);
+    auto put = [&](int64_t x, int32_t v) {  // the streamed forms of every id, written on the way
+      const int32_t at = (int32_t)(E - ebase - s_erow[R[s]]), n = s_erow[R[s] + 1] - s_erow[R[s]];
+      if (b.codes) b.codes[code_start(x - at, (uint32_t)n) + at] = (uint16_t)core_code((uint32_t)v, a.core_kb);
+      if (b.lines) b.lines[line_start(x - at, n) + at] = v;
     };
     if (gr < 0) {
       b.key[E] = -1;  // the row is not split: no pair
-      if (b.codes) put_code(E + cd0, a.ci[E + cd0]);  // (one graph)
+      if (b.codes || b.lines) put(E + cd0, a.ci[E + cd0]);  // (one graph)
       continue;
     }
     if (gr != gc) {
@@ -1226,7 +1228,7 @@ __global__ __launch_bounds__(kBlock) void radix_split_kernel(LaunchArgs a, int64
     cix[s] = E + cd;
     const int32_t v = a.ci[cix[s]];
     qv[s] = (int32_t)(rb + v);
-    if (b.codes) put_code(cix[s], v);
+    if (b.codes || b.lines) put(cix[s], v);
   }
 #pragma unroll
   for (int s = 0; s < kMPPer; ++s) dv[s] = qv[s] >= 0 ? (int32_t)b.deg16[qv[s]] : 0;
@@ -1907,8 +1909,6 @@ struct __align__(16) CountLds {
   uint32_t End[kBlock];          // per-lane edge end in the batch's flat index
   gint32* Base[kBlock];          // per-lane N+(v) base of that edge, shifted by its first index
   uint64_t red[kWaves];
-  int64_t tab_cnt[1];
-  int64_t cur_seg;
   uint32_t next[2];
 };
 static_assert(kAreaWave * kWaves <= kAreaBlock, "wave areas exceed LDS region");
@@ -2006,7 +2006,7 @@ __device__ __forceinline__ void group_tile(const LaunchArgs& a, const uint64_t* 
     const LocalSink ls{C, kEL ? LL.ec() + grp * G : nullptr, kEL ? a.local.pedge + pr.pb : nullptr,
                        kEL ? a.local.pvid + pr.pb : nullptr, a.local.ecount, a.local.vcount};
     const uint32_t h = pivot_edges<G, kModeHash | kModeTree, G == 64 ? kInFlight : kInFlightGroup, kEL, kWide>(
-        a.ci, RefEdges{a.pci + pr.pb, skip}, (int)(pr.pe - pr.pb), S, 0, G, sEnd, sBase, gl, ls);
+        a.lines ? a.lines : a.ci, RefEdges{a.pci + pr.pb, a.lines != nullptr, skip}, (int)(pr.pe - pr.pb), S, 0, G, sEnd, sBase, gl, ls);
     if constexpr (kLocal == kLocalFull) {
       group_sync<G>();
       flush_set_hits<G>(slot, C, S, gl, a.local.vcount);
@@ -2024,12 +2024,12 @@ template <bool kLdsPivot, int kLocal, bool kWide>
 __device__ __forceinline__ void block_pivot(const LaunchArgs& a, uint64_t item, CountLds& L,
                                             LocalLds<kLocal>& LL, bool batch, Acc& acc) {
   const PRow pr = partner_row(a, (int64_t)item);
-  const int32_t* ci = a.ci;
-  const int32_t* set = ci + list_start(pr.set);
+  const int32_t* ci = a.lines ? a.lines : a.ci;
+  const int32_t* set = a.ci + list_start(pr.set);
   const int ds = list_len(pr.set);
   const uint32_t skip = open_only<kBlock, kLocal>(a);
   if (skip && !(pr.g & kRowOpen)) return;  // the whole workgroup
-  const RefEdges part{a.pci + pr.pb, skip};
+  const RefEdges part{a.pci + pr.pb, a.lines != nullptr, skip};
   const int np = (int)(pr.pe - pr.pb);
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
   constexpr int kEL = edge_local(kLocal);
@@ -2080,34 +2080,80 @@ constexpr int waves_per_eu(int kLocal) {
        : kLocal == kLocalEdges ? TC_LOCAL_EDGES_WAVES_PER_EU : TC_COUNT_WAVES_PER_EU;  // parts: the plain count's
 }
 
-// How a persistent workgroup gets its tiles.  A queue head that every
-// workgroup adds to serves one tile per ~12 ns on MI355X, which bounds a
+// How a persistent workgroup gets its tiles.  The tiles are cut into an eighth
+// per XCD (workgroups are placed on XCD blockIdx.x mod 8), each with a queue
+// head of its own: one head serves a tile per ~12 ns on MI355X, which bounds a
 // kernel of many small tiles (an R-MAT-22 graph's 66 K workgroup rows whose
-// codes leave them little to do here: 0.80 ms queued, 0.19 ms with turns); so
-// a workgroup takes its first tiles in turn (blockIdx.x + k * grid, k <
-// fixed) and only the last part, which evens out what the turns left uneven,
-// comes from the queue.  16ths of the tiles taken in turn: 15 (R-MAT-22,
-// R-MAT-18 and a partition's counts 5-8% faster than with 12); local counts,
-// whose tiles differ more, 8 (edges of R-MAT-20: 1.94 ms, 12: 2.11, 15: 2.40).
-// With fewer than kQueueFrom tiles per workgroup all are taken in turn: every
-// workgroup's last, empty answer from the queue would cost more than it evens
-// out (R-MAT n=30011: 0.15 -> 0.03 ms of the bitmap kernels).
-constexpr int kTurns = 15, kLocalTurns = 8, kQueueFrom = 4;
-struct TileTurn {
-  int64_t ntiles, fixed, grid;
-  __device__ TileTurn(int64_t n, int64_t g, int sixteenths) : ntiles(n), grid(g) {
-    fixed = sixteenths >= 16 || ntiles < kQueueFrom * g ? (ntiles + g - 1) / g : ntiles * sixteenths / 16 / g;
+// codes leave them little to do in the hash kernel: 0.80 ms).  A workgroup
+// starts with a tile of its own, then takes its eighth's in order and, when
+// those are gone, the other eighths'.  A fixed share each is no substitute: a
+// count's kernels share the CUs, so their workgroups start at different times
+// (15/16 of the tiles in turn: the batch of 512 graphs 3.45 ms; queues: 2.52).
+// In a batch an eighth is a run of tiles, which keeps the few graphs that an
+// XCD is at in its L2 (the bitmap kernel of workgroup rows 0.50 -> 0.33 ms);
+// in one graph it is every eighth tile, which spreads the heavy ones (part 0
+// of R-MAT-21 in four: runs 0.70 ms, so 0.52).
+// A kernel of at most this many tiles per workgroup takes them all in turn:
+// every workgroup's last, empty answers would cost more than its queue evens
+// out (the bitmap kernels of R-MAT n=30011: 0.072 -> 0.044 ms).
+constexpr uint32_t kHashTurns = 2, kBlockTurns = 4, kWaveTurns = 8;
+struct TileQueue {
+  uint32_t* heads;  // the eighths' heads, kHeadStride words apart
+  uint32_t n, grid, home, j;
+  bool runs;          // eighths are runs of tiles, not every eighth tile
+  uint32_t turns;     // tiles every workgroup takes before its XCD's head
+  uint32_t k = 0;     // of those, taken
+  uint32_t past = 0;  // eighths done with, from home on
+  uint32_t raw = 0;   // head's answer for the next tile
+
+  __device__ uint32_t lo(uint32_t e) const { return (uint32_t)((uint64_t)n * e >> 3); }
+  __device__ uint32_t size(uint32_t e) const { return runs ? lo(e + 1) - lo(e) : (n + 7 - e) >> 3; }
+  __device__ uint32_t tile(uint32_t e, uint32_t i) const { return runs ? lo(e) + i : 8 * i + e; }
+  __device__ uint32_t groups(uint32_t e) const { return (grid + 7 - e) >> 3; }  // workgroups of XCD e
+  __device__ uint32_t* head(uint32_t e) const { return heads + kHeadStride * e; }
+  // base: tiles of this XCD that the workgroup's launch had before (its first
+  // tiles go to the workgroups after those).
+  __device__ TileQueue(const LaunchArgs& a, int queue, uint32_t ntiles, uint32_t base, bool batch, uint32_t all)
+      : heads(a.bufs.counters + kCntHeads + 8 * kHeadStride * queue), n(ntiles), grid(gridDim.x),
+        home(blockIdx.x & 7), runs(batch), turns(1) {
+    const uint32_t own = groups(home);
+    j = ((blockIdx.x >> 3) + own - base % own) % own;
+    if ((n + 7) >> 3 <= all * (grid >> 3)) {  // (then no eighth has more tiles than its XCD takes in turn)
+      turns = all;
+      past = 8;
+    }
   }
-  __device__ bool all() const { return fixed * grid >= ntiles; }  // no queue
-  __device__ uint32_t first() const { return (uint32_t)(fixed * grid); }  // the queue's first tile
-  // Tile k < fixed of workgroup b.  A batch's tiles are in graph order: each
-  // XCD (workgroups equal modulo 8) takes its own eighth of them, its
-  // workgroups side by side, so that the few graphs it is at stay in its L2
-  // (the batch of 512 graphs: the bitmap kernel of whole-workgroup rows 0.50
-  // -> 0.34 ms, the 16-lane bin 0.93 -> 0.83 ms).
-  __device__ int64_t tile(uint32_t b, int64_t k, bool batch) const {
-    if (batch && grid % 8 == 0) return (b & 7) * (fixed * (grid / 8)) + (b >> 3) + k * (grid / 8);
-    return b + k * grid;
+  // The workgroup's first tile (all its threads; word: shared).
+  __device__ uint32_t first(uint32_t* word) {
+    if (threadIdx.x == 0 && past < 8) raw = atomicAdd(head(home), 1u);
+    if (j < size(home)) return tile(home, j);
+    if (past >= 8) return n;
+    if (threadIdx.x == 0) {  // (an eighth with tiles may have no workgroups)
+      k = turns;
+      *word = take();
+    }
+    __syncthreads();
+    return uniform32((int)*word);
+  }
+  // One thread: the next tile (n: none left); asks its head for the one after.
+  __device__ uint32_t take() {
+    if (++k < turns) {
+      const uint32_t i = j + k * groups(home);
+      return i < size(home) ? tile(home, i) : n;
+    }
+    while (past < 8) {
+      uint32_t e = (home + past) & 7;
+      const uint32_t i = turns * groups(e) + raw;
+      if (i < size(e)) {
+        raw = atomicAdd(head(e), 1u);
+        return tile(e, i);
+      }
+      do {
+        e = (home + ++past) & 7;
+      } while (past < 8 && turns * groups(e) + __hip_atomic_load(head(e), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= size(e));
+      if (past < 8) raw = atomicAdd(head(e), 1u);
+    }
+    return n;
   }
 };
 
@@ -2115,40 +2161,23 @@ __device__ __forceinline__ unsigned long long* out_word(const LaunchArgs& a) {
   return (unsigned long long*)a.bufs.outs + (a.out_slots ? (blockIdx.x & (kOutSlots - 1)) * kOutStride : 0);
 }
 
-// One persistent kernel per bin, specialised so that each keeps only its own
-// working set in registers.
-// rounds: rows per group in a light bin's tile, 0: as many as still give
-// every workgroup a tile, at most the tune's.
-// kLocal: also the per-edge (and, kLocalFull, per-vertex) attribution of
-// a.local (one graph only).
-// kWide: the instantiation for graphs whose ids reach 2^24 (folded hash keys).
+// The rows of one bin: this workgroup's share of its tiles.
 template <int BIN, int kLocal, bool kWide>
-__global__ __launch_bounds__(kBlock, waves_per_eu(kLocal)) void count_kernel(
-    LaunchArgs a, int rounds) {
-  __shared__ CountLds L;
-  __shared__ LocalLds<kLocal> LL;
-  // batch: per-graph sums; kLocalParts: per-part sums, kept the same way
-  const bool batch = (!kLocal && a.ngraphs > 1) || kLocal == kLocalParts;
-  if constexpr (edge_local(kLocal) != kLocalNone) LL.EC[threadIdx.x] = 0;  // ordered by the barrier below
-  if (threadIdx.x == 0) {
-    int64_t seg = 0;
-    for (int b = 0; b < BIN; ++b) seg += a.bufs.counters[kCntBinCount + b];
-    L.cur_seg = seg;
-    L.tab_cnt[0] = a.bufs.counters[kCntBinCount + BIN];
-  }
-  __syncthreads();
-  const int64_t cnt = L.tab_cnt[0];
-  const int piv = tile_pivots(BIN, rounds > 0 ? rounds : tile_rounds(BIN, cnt, gridDim.x, a.tune.rounds));
+__device__ __forceinline__ void bin_tiles(const LaunchArgs& a, CountLds& L, LocalLds<kLocal>& LL, bool batch,
+                                          uint32_t& base, Acc& acc) {
+  int64_t seg = 0;
+  for (int b = 0; b < BIN; ++b) seg += a.bufs.counters[kCntBinCount + b];
+  const int64_t cnt = uniform32((int)a.bufs.counters[kCntBinCount + BIN]);
+  if (cnt == 0) return;
+  const int piv = tile_pivots(BIN, tile_rounds(BIN, cnt, gridDim.x, a.tune.rounds));
   const int64_t ntiles = (cnt + piv - 1) / piv;
-  const uint64_t* items = a.bufs.items + L.cur_seg;
-  Acc acc;
-  acc.g = 0;
-  const TileTurn turn(ntiles, gridDim.x, edge_local(kLocal) ? kLocalTurns : kTurns);
-  int64_t t = turn.tile(blockIdx.x, 0, batch);
-  for (int64_t k = 1; t < ntiles; ++k) {
-    const bool queued = k >= turn.fixed && !turn.all();
-    if (queued && threadIdx.x == 0)  // read after the barrier at the end, into the other word next time
-      L.next[k & 1] = turn.first() + atomicAdd(&a.bufs.counters[kCntHeads + kHeadStride * BIN], 1u);
+  const uint64_t* items = a.bufs.items + uniform64(seg);
+  __syncthreads();  // a late wave may still read the last bin's L.next
+  TileQueue q(a, BIN, (uint32_t)ntiles, base, batch, kHashTurns);
+  base += q.size(q.home);
+  int64_t t = q.first(&L.next[1]);
+  for (int k = 0; t < ntiles; k ^= 1) {
+    if (threadIdx.x == 0) L.next[k] = q.take();  // read after the barrier at the end, into the other word next time
     const int64_t first = t * piv;
     const int64_t last = min(first + (int64_t)piv, cnt);
     if (BIN == BIN_GLOBAL) block_pivot<false, kLocal, kWide>(a, items[first], L, LL, batch, acc);
@@ -2172,8 +2201,40 @@ __global__ __launch_bounds__(kBlock, waves_per_eu(kLocal)) void count_kernel(
       acc.sum = 0;
     }
     __syncthreads();
-    t = queued ? (int64_t)uniform32((int)L.next[k & 1]) : k < turn.fixed ? turn.tile(blockIdx.x, k, batch) : ntiles;
+    t = (int64_t)uniform32((int)L.next[k]);
   }
+}
+
+// The persistent hash kernel: the rows of the bins in the mask `bins`, heavy
+// bins first.  One launch for all bins: with a kernel per bin, on a stream
+// per group of them, the chip was left to a few long rows at the end of each
+// (R-MAT-18: 0.32 ms, six kernels of 10-90 us; so 0.22).
+// kLight: the sub-wave bins only (fewer registers: the bitmap kernels have
+// the others).
+// kLocal: also the per-edge (and, kLocalFull, per-vertex) attribution of
+// a.local (one graph only).
+// kWide: the instantiation for graphs whose ids reach 2^24 (folded hash keys).
+template <bool kLight, int kLocal, bool kWide>
+__global__ __launch_bounds__(kBlock, waves_per_eu(kLocal)) void count_kernel(LaunchArgs a, uint32_t bins) {
+  __shared__ CountLds L;
+  __shared__ LocalLds<kLocal> LL;
+  // batch: per-graph sums; kLocalParts: per-part sums, kept the same way
+  const bool batch = (!kLocal && a.ngraphs > 1) || kLocal == kLocalParts;
+  if constexpr (edge_local(kLocal) != kLocalNone) {
+    LL.EC[threadIdx.x] = 0;
+    __syncthreads();
+  }
+  Acc acc;
+  acc.g = 0;
+  uint32_t base = 0;
+  if constexpr (!kLight) {
+    if (bins >> BIN_GLOBAL & 1) bin_tiles<BIN_GLOBAL, kLocal, kWide>(a, L, LL, batch, base, acc);
+    if (bins >> BIN_BLOCK & 1) bin_tiles<BIN_BLOCK, kLocal, kWide>(a, L, LL, batch, base, acc);
+    if (bins >> BIN_WAVE & 1) bin_tiles<BIN_WAVE, kLocal, kWide>(a, L, LL, batch, base, acc);
+  }
+  if (bins >> BIN_G32 & 1) bin_tiles<BIN_G32, kLocal, kWide>(a, L, LL, batch, base, acc);
+  if (bins >> BIN_G16 & 1) bin_tiles<BIN_G16, kLocal, kWide>(a, L, LL, batch, base, acc);
+  if (bins >> BIN_G8 & 1) bin_tiles<BIN_G8, kLocal, kWide>(a, L, LL, batch, base, acc);
   if (!batch) {
     const uint64_t tot = block_sum(acc.sum, L.red);
     if (threadIdx.x == 0 && tot) atomicAdd(out_word(a), tot);
@@ -2181,6 +2242,7 @@ __global__ __launch_bounds__(kBlock, waves_per_eu(kLocal)) void count_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// bitmap count of heavy partner rows// ---------------------------------------------------------------------------
 // bitmap count of heavy partner rows
 // ---------------------------------------------------------------------------
 // When every id of a graph has a 16-bit code, a row's set is a bitmap of at
@@ -2302,18 +2364,14 @@ __global__ __launch_bounds__(64 * NW, 8) void core_kernel(LaunchArgs a, int bin0
   const uint8_t* B = (const uint8_t*)s_bits;
   const char* pool = (const char*)a.c16;
   uint64_t sum = 0;
-  // (waves with a row each finish close together, and there are twice as many
-  // of them as workgroups: all in turn)
-  const TileTurn turn(cnt, gridDim.x, NW == 1 ? 16 : kTurns);
-  int64_t t = turn.tile(blockIdx.x, 0, batch);
+  TileQueue q(a, head, (uint32_t)cnt, 0, batch, NW == 1 ? kWaveTurns : kBlockTurns);
+  int64_t t = q.first(&L.tile[1]);
   PRow pr{0, 0, 0, 0, 0};
   if (t < cnt) pr = partner_row(a, (int64_t)items[t]);
-  for (int64_t k = 1; t < cnt; ++k) {
-    // the next row's place: its turn, or the queue's answer (read after the
-    // first barrier; two words, since a late wave may still read the other)
-    const bool queued = k >= turn.fixed && !turn.all();
-    if (queued && threadIdx.x == 0)
-      L.tile[k & 1] = turn.first() + atomicAdd(&a.bufs.counters[kCntHeads + kHeadStride * head], 1u);
+  for (int k = 0; t < cnt; k ^= 1) {
+    // the next row's place (read after the first barrier; two words, since a
+    // late wave may still read the other)
+    if (threadIdx.x == 0) L.tile[k] = q.take();
     const int64_t pb = uniform64(pr.pb);
     // core 2: a row without closed edges has nothing to do here
     const int np = a.core == 2 && !(pr.g & kRowClosed) ? 0 : uniform32((int)(pr.pe - pr.pb));
@@ -2328,7 +2386,7 @@ __global__ __launch_bounds__(64 * NW, 8) void core_kernel(LaunchArgs a, int bin0
     ListRef r0 = lane < per && j < np ? a.pci[pb + j] : (ListRef)0;
     for (int i = threadIdx.x; i < (1 << a.core_kb) / 16; i += T) ((w4*)s_bits)[i] = w4{0, 0, 0, 0};
     core_sync<NW>();
-    t = queued ? (int64_t)uniform32((int)L.tile[k & 1]) : k < turn.fixed ? turn.tile(blockIdx.x, k, batch) : cnt;
+    t = (int64_t)uniform32((int)L.tile[k]);
     const int64_t next_item = t < cnt ? (int64_t)items[t] : -1;
     auto put = [&](uint32_t x) {
       if (x != kNoCode) atomicOr(&s_bits[(x & 0x1FFFu) >> 2], 1u << (((x & 3u) << 3) | (x >> kCoreByteBits)));
@@ -2957,7 +3015,7 @@ hipError_t launch_zero(void* p, int64_t words32, hipStream_t s) {
 
 __global__ void rearm_kernel(uint32_t* counters, uint64_t* outs, int32_t nouts) {
   const int i = threadIdx.x;
-  if (i < kNumHeads) counters[kCntHeads + kHeadStride * i] = 0u;
+  if (i < 8 * kNumHeads) counters[kCntHeads + kHeadStride * i] = 0u;
   if (i == 0) counters[kCntFallback] = 0u;
   for (int j = i; j < nouts; j += blockDim.x) outs[j] = 0ull;
 }
@@ -2981,11 +3039,11 @@ hipError_t launch_plan(const LaunchArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int BIN, int kLocal, bool kWide>
-static int bin_blocks_per_cu() {
+template <bool kLight, int kLocal, bool kWide>
+static int hash_blocks_per_cu() {
   static const int n = [] {
     int k = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, count_kernel<BIN, kLocal, kWide>, kBlock, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, count_kernel<kLight, kLocal, kWide>, kBlock, 0) !=
         hipSuccess)
       k = 1;
     return k > 0 ? k : 1;
@@ -2993,25 +3051,37 @@ static int bin_blocks_per_cu() {
   return n;
 }
 
-// rows >= 0: the bin's row count is known on the host; the grid is then
-// capped at its tiles, and an empty bin is not launched.
-template <int BIN, int kLocal = kLocalNone>
-static void launch_bin(const LaunchArgs& a, int cus, int grid, hipStream_t s, int64_t rows = -1) {
-  if (rows == 0) return;
-  const bool wide = a.wide_ids != 0;
-  int64_t g = grid > 0 ? grid
-                       : (int64_t)(wide ? bin_blocks_per_cu<BIN, kLocal, true>() : bin_blocks_per_cu<BIN, kLocal, false>()) * cus;
-  int rounds = 0;
-  if (rows > 0) {
-    rounds = tile_rounds(BIN, rows, g, a.tune.rounds);
-    const int64_t piv = tile_pivots(BIN, rounds), tiles = (rows + piv - 1) / piv;
-    if (tiles < g) g = tiles;
+// The hash kernel over the bins of a mask; rows: per bin, null when the host
+// does not know them (full residency; else no more workgroups than tiles).
+template <bool kLight, int kLocal, bool kWide>
+static void launch_hash_as(const LaunchArgs& a, int cus, int grid, uint32_t bins, const int64_t* rows, hipStream_t s) {
+  int64_t g = grid > 0 ? grid : (int64_t)hash_blocks_per_cu<kLight, kLocal, kWide>() * cus;
+  if (rows) {
+    int64_t tiles = 0;
+    for (int b = 0; b < kNumBins; ++b) {
+      if (!(bins >> b & 1)) continue;
+      const int64_t piv = tile_pivots(b, tile_rounds(b, rows[b], g, a.tune.rounds));
+      tiles += (rows[b] + piv - 1) / piv;
+    }
+    if (tiles == 0) return;
+    g = min(g, (tiles + 7) & ~(int64_t)7);
   }
-  if (wide) count_kernel<BIN, kLocal, true><<<(unsigned)g, kBlock, 0, s>>>(a, rounds);
-  else count_kernel<BIN, kLocal, false><<<(unsigned)g, kBlock, 0, s>>>(a, rounds);
+  count_kernel<kLight, kLocal, kWide><<<(unsigned)g, kBlock, 0, s>>>(a, bins);
+}
+constexpr uint32_t kAllBins = (1u << kNumBins) - 1, kLightBins = 1u << BIN_G32 | 1u << BIN_G16 | 1u << BIN_G8;
+template <int kLocal = kLocalNone>
+static void launch_hash(const LaunchArgs& a, int cus, int grid, uint32_t bins, const int64_t* rows, hipStream_t s) {
+  if (kLocal == kLocalNone && (bins & ~kLightBins) == 0) {
+    if (a.wide_ids) launch_hash_as<true, kLocalNone, true>(a, cus, grid, bins, rows, s);
+    else launch_hash_as<true, kLocalNone, false>(a, cus, grid, bins, rows, s);
+  } else if (a.wide_ids) {
+    launch_hash_as<false, kLocal, true>(a, cus, grid, bins, rows, s);
+  } else {
+    launch_hash_as<false, kLocal, false>(a, cus, grid, bins, rows, s);
+  }
 }
 
-// The bitmap kernel of bins bin0..bin1, which use queue head `head`; rows as
+// The bitmap kernel of bins bin0..bin1,// The bitmap kernel of bins bin0..bin1, which use queue head `head`; rows as
 // for launch_bin.
 template <int NW>
 static int core_blocks_per_cu(int kb) {
@@ -3019,26 +3089,30 @@ static int core_blocks_per_cu(int kb) {
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, core_kernel<NW>, 64 * NW, (size_t)1 << kb) != hipSuccess) k = 1;
   return k > 0 ? k : 1;
 }
+// Workgroups per CU of the bitmap kernels where the hash kernel has rows of the
+// same count: they leave it 2 of a CU's 8 places from the start.  Workgroups
+// stay until the queue is empty, so at full residency the hash kernel's would
+// start when the bitmap kernels end, and work bound by memory would not run
+// beside work bound by latency (R-MAT-22: 3.45 ms; 5 and 4: 3.20; 4 and 4:
+// 3.22; 3 and 4: 3.54.  Part 0 of R-MAT-21 in four: 0.59 / 0.54 / 0.53 / 0.60).
+constexpr int kBlockBeside = 4, kWaveBeside = 3;
 template <int NW>
 static void launch_core(const LaunchArgs& a, int cus, int grid, hipStream_t s, int64_t rows, int bin0, int bin1,
-                        int head) {
+                        int head, bool beside) {
   if (rows == 0) return;
   int64_t g = grid > 0 ? grid : (int64_t)core_blocks_per_cu<NW>(a.core_kb) * cus;
-  if (rows > 0 && rows < g) g = rows;
+  if (grid <= 0 && beside) g = min(g, (int64_t)cus * (NW == 1 ? kWaveBeside : kBlockBeside));
+  if (rows > 0) g = min(g, (rows + 7) & ~(int64_t)7);
   core_kernel<NW><<<(unsigned)g, 64 * NW, (size_t)1 << a.core_kb, s>>>(a, bin0, bin1, head);
 }
 
 hipError_t launch_count(const LaunchArgs& a, int cus, int grid, hipStream_t s) {
-  launch_bin<BIN_GLOBAL>(a, cus, grid, s);
-  launch_bin<BIN_BLOCK>(a, cus, grid, s);
-  launch_bin<BIN_WAVE>(a, cus, grid, s);
-  launch_bin<BIN_G32>(a, cus, grid, s);
-  launch_bin<BIN_G16>(a, cus, grid, s);
-  launch_bin<BIN_G8>(a, cus, grid, s);
+  launch_hash(a, cus, grid, kAllBins, nullptr, s);
   return hipGetLastError();
 }
 
-int core_last_bin(const LaunchArgs& a, const int64_t* rows) {
+// Bins 0..core_last_bin are counted by the bitmap kernels (-1: none).
+static int core_last_bin(const LaunchArgs& a, const int64_t* rows) {
   if (a.core == 0) return -1;
   if (a.core != 1 || !rows) return BIN_WAVE;
   int64_t light = 0;
@@ -3046,60 +3120,52 @@ int core_last_bin(const LaunchArgs& a, const int64_t* rows) {
   return light <= kCoreLightRows ? BIN_G8 : BIN_WAVE;
 }
 
-hipError_t launch_count_order(const LaunchArgs& a, int cus, int grid, const int* order, int n,
-                              const int64_t* rows, hipStream_t s) {
+// Bins of a part of the count.
+static uint32_t part_bins(const LaunchArgs& a, int part, const int64_t* rows) {
   const int last = core_last_bin(a, rows);
-  for (int i = 0; i < n; ++i) {
-    const int b = order[i];
-    const int64_t r = rows ? rows[b] : -1;
-    if (b <= last) {
-      auto sum = [&](int b0, int b1) {
-        int64_t x = 0;
-        for (int y = b0; y <= b1; ++y) x += rows[y];
-        return x;
-      };
-      if (b == BIN_BLOCK)
-        launch_core<kWaves>(a, cus, grid, s, rows ? sum(BIN_GLOBAL, BIN_BLOCK) : -1, BIN_GLOBAL, BIN_BLOCK,
-                            kCoreHead);
-      if (b == BIN_WAVE) launch_core<1>(a, cus, grid, s, rows ? sum(BIN_WAVE, last) : -1, BIN_WAVE, last,
-                                           kCoreHead + 1);
-      if (a.core == 1) continue;
-    }
-    switch (b) {
-      case BIN_GLOBAL: launch_bin<BIN_GLOBAL>(a, cus, grid, s, r); break;
-      case BIN_BLOCK: launch_bin<BIN_BLOCK>(a, cus, grid, s, r); break;
-      case BIN_WAVE: launch_bin<BIN_WAVE>(a, cus, grid, s, r); break;
-      case BIN_G32: launch_bin<BIN_G32>(a, cus, grid, s, r); break;
-      case BIN_G16: launch_bin<BIN_G16>(a, cus, grid, s, r); break;
-      default: launch_bin<BIN_G8>(a, cus, grid, s, r); break;
-    }
+  const uint32_t block = 1u << BIN_GLOBAL | 1u << BIN_BLOCK, coded = (1u << (last + 1)) - 1;
+  if (part == kPartBlock) return coded & block;
+  if (part == kPartWave) return coded & ~block;
+  return a.core == 2 ? kAllBins : kAllBins & ~coded;
+}
+
+bool part_empty(const LaunchArgs& a, int part, const int64_t* rows) {
+  const uint32_t bins = part_bins(a, part, rows);
+  if (!rows) return bins == 0;
+  int64_t n = 0;
+  for (int b = 0; b < kNumBins; ++b) n += bins >> b & 1 ? rows[b] : 0;
+  return n == 0;
+}
+
+hipError_t launch_count_part(const LaunchArgs& a, int cus, int grid, int part, const int64_t* rows, hipStream_t s) {
+  if (part_empty(a, part, rows)) return hipSuccess;
+  const uint32_t bins = part_bins(a, part, rows);
+  if (part == kPartHash) {
+    launch_hash(a, cus, grid, bins, rows, s);
+  } else {
+    const int b0 = part == kPartBlock ? BIN_GLOBAL : BIN_WAVE, b1 = 31 - __builtin_clz(bins);
+    int64_t n = rows ? 0 : -1;
+    for (int b = b0; rows && b <= b1; ++b) n += rows[b];
+    const bool beside = !part_empty(a, kPartHash, rows);
+    if (part == kPartBlock) launch_core<kWaves>(a, cus, grid, s, n, b0, b1, kCoreHead, beside);
+    else launch_core<1>(a, cus, grid, s, n, b0, b1, kCoreHead + 1, beside);
   }
   return hipGetLastError();
 }
 
-template <int kLocal>
-static void launch_local_bins(const LaunchArgs& a, int cus, int first, int last, hipStream_t s) {
-  if (first <= BIN_GLOBAL && BIN_GLOBAL <= last) launch_bin<BIN_GLOBAL, kLocal>(a, cus, 0, s);
-  if (first <= BIN_BLOCK && BIN_BLOCK <= last) launch_bin<BIN_BLOCK, kLocal>(a, cus, 0, s);
-  if (first <= BIN_WAVE && BIN_WAVE <= last) launch_bin<BIN_WAVE, kLocal>(a, cus, 0, s);
-  if (first <= BIN_G32 && BIN_G32 <= last) launch_bin<BIN_G32, kLocal>(a, cus, 0, s);
-  if (first <= BIN_G16 && BIN_G16 <= last) launch_bin<BIN_G16, kLocal>(a, cus, 0, s);
-  if (first <= BIN_G8 && BIN_G8 <= last) launch_bin<BIN_G8, kLocal>(a, cus, 0, s);
-}
-
-hipError_t launch_count_local(const LaunchArgs& a, int cus, int first, int last, int mode, hipStream_t s) {
+hipError_t launch_count_local(const LaunchArgs& a, int cus, int mode, hipStream_t s) {
   if (a.ngraphs != 1 || !a.local.pown) return hipErrorInvalidValue;
   if (mode == kLocalParts) {
     if (!a.local.bounds || !a.local.pe || a.local.parts < 1 || a.local.parts > kMaxParts) return hipErrorInvalidValue;
-    launch_local_bins<kLocalParts>(a, cus, first, last, s);
+    launch_hash<kLocalParts>(a, cus, 0, kAllBins, nullptr, s);
     return hipGetLastError();
   }
   if (!a.local.pedge || !a.local.ecount) return hipErrorInvalidValue;
   if (mode == kLocalFull) {
     if (!a.local.pvid || !a.local.vcount) return hipErrorInvalidValue;
-    launch_local_bins<kLocalFull>(a, cus, first, last, s);
+    launch_hash<kLocalFull>(a, cus, 0, kAllBins, nullptr, s);
   } else if (mode == kLocalEdges) {
-    launch_local_bins<kLocalEdges>(a, cus, first, last, s);
+    launch_hash<kLocalEdges>(a, cus, 0, kAllBins, nullptr, s);
   } else {
     return hipErrorInvalidValue;
   }
@@ -3174,7 +3240,7 @@ hipError_t noalloc_scratch_address(void** ptr) { return hipGetSymbolAddress(ptr,
 
 int count_blocks_per_cu() {
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, count_kernel<BIN_WAVE, false, false>, kBlock, 0) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, count_kernel<false, kLocalNone, false>, kBlock, 0) !=
       hipSuccess)
     return 1;
   return n > 0 ? n : 1;

@@ -53,17 +53,17 @@ __host__ __device__ inline int tile_rounds(int bin, int64_t rows, int64_t grid, 
   return (int)(r < 1 ? 1 : most > 0 && r > most ? most : most < 1 ? 1 : r);
 }
 
-// Counter words of a plan (uint32).  The tile queue heads are a cache line
-// apart: the bins' kernels run side by side, and heads that share a line are
-// served one after another.
+// Counter words of a plan (uint32).  The tile queue heads, one per queue and
+// XCD, are a cache line apart: heads that share a line are served one after
+// another.
 constexpr int kCntBinCount = 0;                   // [kNumBins]
 constexpr int kCntFallback = kNumBins;            // hash builds that fell back to the tree
 constexpr int kPlanWords = 32;                    // words up to here are read back
-constexpr int kCntHeads = 32;                     // queue head i: word kCntHeads + kHeadStride * i
+constexpr int kCntHeads = 32;                     // queue i, eighth e: word kCntHeads + kHeadStride * (8 i + e)
 constexpr int kHeadStride = 32;
 constexpr int kNumHeads = kNumBins + 2;           // a bin's; then the bitmap kernels' two
 constexpr int kCoreHead = kNumBins;
-constexpr int kNumCounters = kCntHeads + kHeadStride * kNumHeads;
+constexpr int kNumCounters = kCntHeads + 8 * kHeadStride * kNumHeads;
 
 // Partner rows.  Every DAG edge (u, v) is counted from the endpoint whose
 // out-list is longer: its "owner" x keeps N+(x) as the LDS set and its
@@ -105,6 +105,13 @@ constexpr int64_t kCorePool = (int64_t)1 << 30;  // ids of a pool with codes: by
 __host__ __device__ inline uint32_t code_start(int64_t p, uint32_t n) {
   const uint32_t a = n >= 64 ? 64u : n >= 32 ? 32u : n >= 16 ? 16u : n >= 8 ? 8u : 1u;
   return ((uint32_t)p * 2u + a - 1u) & ~(a - 1u);
+}
+// Where a list of n ids at ci position p is in a pool of lists on lines: twice
+// p, or the next 128-byte line where it would straddle one -- less than n ids
+// further on, so lists stay inside [2p, 2p + 2n) and do not overlap.
+__host__ __device__ inline int64_t line_start(int64_t p, int32_t n) {
+  const int64_t s = 2 * p;
+  return (s & 31) + n > 32 ? (s + 31) & -32 : s;
 }
 constexpr uint32_t kCodeMul = 0x9E37u;      // odd, near 2^16 / phi
 __host__ __device__ constexpr uint32_t core_code(uint32_t i, int kb) {
@@ -255,6 +262,7 @@ struct LaunchArgs {
   int64_t P;            // partner-row slots = plan indices (sum of nv_max + 1)
   const int64_t* rp;    // DAG rowptr pool
   const int32_t* ci;    // DAG colidx pool
+  const int32_t* lines; // null, or the lists of ci on cache lines (line_start), for streaming
   const ListRef* pci;   // partner pool: each partner's list
   const int64_t* vrp;   // [P + 1] partner-row offsets into the partner pool
   const VRow* vrow;     // [P] partner rows
@@ -303,6 +311,7 @@ struct BuildBufs {
   int32_t* pvid;        // with pedge: [partner pool] partner vertex of each entry
   int32_t* pown;        // null, or (one graph) [P] owner vertex of each partner row
   uint16_t* codes;          // null, or where to write the codes of all ids (core_code, a.core_kb)
+  int32_t* lines;           // null, or where to write the lists at line_start
   const uint8_t* closed;    // null, or (one graph) per row kClosed | kOrdered
   const uint8_t* lpart;     // with closed: per DAG id e = (u, v), the part of u's codes that rank with v or above
   // Radix transpose (null when the scratch has no per-id part).  Build space:
@@ -416,6 +425,8 @@ hipError_t launch_stage_copy(const StageCopy* copies, int32_t n, int64_t chunks,
 // counter to 0 (bin counts kept), outs[0..nouts) to 0.
 hipError_t launch_rearm(uint32_t* counters, uint64_t* outs, int32_t nouts, hipStream_t s);
 hipError_t launch_plan(const LaunchArgs& a, hipStream_t s);
+// Bytes of a pool of ids with its lists on lines.
+inline size_t line_bytes(int64_t ids) { return sizeof(int32_t) * (size_t)(2 * ids + kCiPad); }
 // Bytes of the codes of a pool of ids.
 inline size_t code_bytes(int64_t ids) { return sizeof(uint16_t) * (size_t)(2 * ids + kCorePad); }
 // Codes for a graph of more than kCoreIds rows: the at most kCoreIds vertices
@@ -433,85 +444,35 @@ inline bool big_codes_fit(int64_t n, int64_t m) {
 int64_t big_codes_bytes(int64_t n, int64_t m);
 hipError_t launch_big_codes(const int64_t* rp, const int32_t* ci, int64_t n, int64_t m, char* scratch, uint16_t* c16,
                             uint8_t* closed, uint8_t* part, unsigned long long* closed_edges, int cus, hipStream_t s);
-// One full-residency persistent launch per bin (grid > 0 overrides the size).
+// The hash kernel over all bins at full residency (grid > 0 overrides the size).
 hipError_t launch_count(const LaunchArgs& a, int cus, int grid, hipStream_t s);
-// Bins order[0..n) in that order, each at full residency or, with rows per
-// bin known on the host (rows[kNumBins]), skipped when empty and with no more
-// workgroups than tiles.
-// Bins 0..core_last_bin are counted by the bitmap kernels (-1: none): those of
-// the rows that keep a wave busy, or all bins of a graph with few light rows
-// (rows: per bin, null if not known), where one more wide launch beats three
-// narrow ones (R-MAT n=30011 d=24: 0.17 -> 0.10 ms) -- a wave per light row
-// is slower from a few rows per resident wave on (the batch of 512 graphs,
-// 215 K rows of the 32-lane bin: 0.53 ms there, 0.64 ms here).
+// A count with codes has up to three parts, each one persistent launch; they
+// run side by side on streams of their own: the bitmap kernels of the rows
+// that take a workgroup (kPartBlock) and a wave (kPartWave), and the hash
+// kernel of all others (kPartHash; without codes of all rows, with codes of
+// some ids the other edges of the heavy rows as well).  rows: per bin, null
+// when the host does not know them; parts without rows launch nothing.
+// The bitmap kernels take the bins that keep a wave busy, or all bins of a
+// graph with few light rows (at most kCoreLightRows), where one more wide
+// launch beats narrow groups (R-MAT n=30011 d=24: 0.17 -> 0.10 ms) -- a wave
+// per light row is slower from a few rows per resident wave on (the batch of
+// 512 graphs, 215 K rows of the 32-lane bin: 0.53 ms there, 0.64 ms here).
 constexpr int64_t kCoreLightRows = 16384;
-int core_last_bin(const LaunchArgs& a, const int64_t* rows);
-hipError_t launch_count_order(const LaunchArgs& a, int cus, int grid, const int* order, int n,
-                              const int64_t* rows, hipStream_t s);
+constexpr int kPartBlock = 0, kPartWave = 1, kPartHash = 2, kCountParts = 3;
+bool part_empty(const LaunchArgs& a, int part, const int64_t* rows);
+hipError_t launch_count_part(const LaunchArgs& a, int cus, int grid, int part, const int64_t* rows, hipStream_t s);
 
-// Stream groups of the bins: the groups run side by side (group 0 on the
-// library stream, the others on side streams), each group's bins one after
-// another in the order written.  Persistent workgroups hold their CUs until
-// their bin drains, so a bin alone on the device at the end of a count runs
-// at its own issue rate: the groups start the sub-wave bins, whose waves
-// stall the most, beside the others and leave wave-wide work for last.
-#ifndef TC_BIN_ORDER
-#define TC_BIN_ORDER "01|2|3|45"
-#endif
-constexpr int kBinGroups = 4;
-struct BinGroups {
-  int n = 0;                        // groups in use
-  int len[kBinGroups] = {};         // bins per group
-  int bin[kBinGroups][kNumBins] = {};
-  bool ok = false;                  // every bin exactly once, at most kBinGroups groups
-};
-constexpr BinGroups parse_bin_groups(const char* t) {
-  BinGroups g{};
-  int seen = 0, cur = 0;
-  bool ok = true;
-  for (int i = 0; t[i] != 0; ++i) {
-    if (t[i] == '|') {
-      ok = ok && g.len[cur] > 0;
-      ++cur;
-      ok = ok && cur < kBinGroups;
-      if (!ok) break;
-      continue;
-    }
-    const int b = t[i] - '0';
-    ok = ok && b >= 0 && b < kNumBins && !(seen >> b & 1);
-    if (!ok) break;
-    seen |= 1 << b;
-    g.bin[cur][g.len[cur]++] = b;
-  }
-  g.n = cur + 1;
-  g.ok = ok && g.len[cur] > 0 && seen == (1 << kNumBins) - 1;
-  return g;
-}
-constexpr BinGroups kBinOrder = parse_bin_groups(TC_BIN_ORDER);
-static_assert(kBinOrder.ok, "TC_BIN_ORDER: bins 0-5 once each, in at most 4 '|'-separated groups");
-// The groups of the edges-only local count (without vertex counts).  The
-// workgroup bin goes first on its own: the wave bin then waits for CUs
-// behind it and the 32-/16-lane bins, and runs at the end with the whole
-// device, beside the short 8-lane bin (RMAT-22 edge and part counts on
-// MI355X: 11.8 ms, against 12.2-12.6 ms with TC_BIN_ORDER, 11.9 ms with the
-// 8-lane bin after the wave bin).  The full local count keeps TC_BIN_ORDER,
-// which measured ~0.25 ms faster for it.
-#ifndef TC_EDGES_BIN_ORDER
-#define TC_EDGES_BIN_ORDER "1|02|3|45"
-#endif
-constexpr BinGroups kEdgesBinOrder = parse_bin_groups(TC_EDGES_BIN_ORDER);
-static_assert(kEdgesBinOrder.ok, "TC_EDGES_BIN_ORDER: bins 0-5 once each, in at most 4 '|'-separated groups");
 // own: null, or per row 1 if it is a pivot row (rows outside
 // [row_begin, row_end) are never pivots).  out must hold 0; zero_next (null,
 // or another word) is set to 0 by the kernel.
 hipError_t launch_plain(const int64_t* rp, const int32_t* ci, int32_t row_begin, int32_t row_end,
                         const uint8_t* own, uint64_t* out, int grid, hipStream_t s, uint64_t* zero_next = nullptr);
-// Count of one graph that also fills a.local: same plan, local variants of
-// bins first..last.  mode kLocalFull: ecount and vcount (zeroed by the
+// Count of one graph that also fills a.local: same plan, the local variants
+// of the hash kernel over all bins.  mode kLocalFull: ecount and vcount (zeroed by the
 // caller); kLocalEdges: ecount only (the kernels keep no slot hit counters:
 // less LDS, more waves per SIMD); kLocalParts: pe only (bounds, parts, pe
 // set; the plain count's kernels, each row's hits added to its owner's part).
-hipError_t launch_count_local(const LaunchArgs& a, int cus, int first, int last, int mode, hipStream_t s);
+hipError_t launch_count_local(const LaunchArgs& a, int cus, int mode, hipStream_t s);
 // Per-graph table of launch_local_parts over rows [0, n): esrc[e] = the row
 // u of DAG edge e = (u, v); the local rebuild (launch_build with pedge and
 // esrc) then sets bit 31 where v owns the edge, i.e. d+(u) < d+(v).

@@ -241,7 +241,7 @@ void BuildScratch::release() {
 
 tc_status launch_build(const tck::LaunchArgs& a, int64_t RP, int64_t M, BuildScratch& bs, hipStream_t s,
                        const LocalBufs* loc, int32_t* pown, const uint8_t* closed,
-                       const uint8_t* part, uint16_t* codes) {
+                       const uint8_t* part, uint16_t* codes, int32_t* lines) {
   // The local rebuild also writes each entry's edge position and partner
   // vertex: the radix path carries the positions along (one graph, its
   // edges' rows in loc->esrc, filled before); the per-edge atomic path
@@ -252,6 +252,7 @@ tc_status launch_build(const tck::LaunchArgs& a, int64_t RP, int64_t M, BuildScr
   bs.b.pedge = loc ? loc->pedge : nullptr;
   bs.b.pvid = loc ? loc->pvid : nullptr;
   bs.b.codes = codes;
+  bs.b.lines = lines;
   bs.b.closed = closed;
   bs.b.lpart = part;
   bs.b.pown = pown;  // one graph: each partner row's owner
@@ -316,6 +317,14 @@ static tc_status check_dag(const tc_csr_view* dag, uint32_t check, int32_t* max_
 // flat ones have no set of 65535 vertices that most edges lead to.
 constexpr int32_t kCodesMinOut = 64;
 
+// Flat graphs (past tck::kCoreIds rows, no list of kCodesMinOut ids) of this
+// many ids on get their lists on lines as well: an edge's list is then read in
+// one 128-byte line instead of 1.5, and such a count is bound by the lines it
+// reads beyond L2 (ER n=2000003 d=33: 1.03 -> 0.90 ms, of a build 1.73 -> 1.81
+// ms).  With codes the other lists are few (R-MAT-22: 3.24, with lines 3.30
+// ms), and fewer ids stay in an XCD's L2 (4 MB).
+constexpr int64_t kLinesLeast = (int64_t)1 << 20;
+
 static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_begin, int32_t row_end,
                             const uint8_t* owned, int32_t max_out, tc_graph** out) {
   std::unique_ptr<tc_graph> g(new tc_graph);
@@ -332,6 +341,7 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
     dev_free(g->rp);
     dev_free(g->ci);
     g->drop_codes();
+    dev_free(g->lines);
     dev_free(g->d_desc);
     dev_free(g->own);
     dev_free(g->pown);
@@ -360,6 +370,10 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
     big = big && st == TC_OK;
     st = TC_OK;
   }
+  tck::RadixGeom geom;
+  if (g->n > tck::kCoreIds && max_out < kCodesMinOut && g->nnz >= kLinesLeast && tck::radix_geom((int64_t)g->n + 1, g->nnz, geom) &&
+      dev_alloc((void**)&g->lines, tck::line_bytes(g->nnz), "lists on lines") != TC_OK)
+    g->lines = nullptr;
   const tck::GraphDesc d{0, 0, 0, 0, 0, g->n, g->nv_max, row_begin, row_end, 0};
   hipError_t e = hipMemcpy(g->rp, dag->rowptr, sizeof(int64_t) * ((size_t)g->n + 1), hipMemcpyHostToDevice);
   if (e == hipSuccess && g->nnz > 0)
@@ -398,7 +412,7 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
       e = tck::launch_big_codes(g->rp, g->ci, g->n, g->nnz, bs.mem, g->c16, g->closed, g->part,
                                 (unsigned long long*)ctx->plain_out + 4, ctx->cus, s);
     if (e == hipSuccess) st = launch_build(a, (int64_t)g->n + 1, g->nnz, bs, s, nullptr, g->pown, g->closed, g->part,
-                                             big ? nullptr : g->c16);
+                                             big ? nullptr : g->c16, g->lines);
     if (st == TC_OK && e == hipSuccess) e = hipEventRecord(ctx->ev[1], s);
     if (st == TC_OK && e == hipSuccess)
       e = hipMemcpyAsync(ctx->pinned, g->partners.nv, sizeof(int32_t), hipMemcpyDeviceToHost, s);
@@ -418,7 +432,8 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
   g->nv = *(const int32_t*)ctx->pinned;
   g->coded = big ? 4 * (int64_t)ctx->pinned[1] >= g->nnz : g->c16 != nullptr;
   g->bytes = sizeof(int64_t) * ((int64_t)g->n + 1) + sizeof(int32_t) * g->nnz + sizeof(tck::GraphDesc) +
-             g->partners.bytes + (owned ? (int64_t)g->n : 0) + (g->c16 ? (int64_t)tck::code_bytes(g->nnz) : 0) +
+             g->partners.bytes + (owned ? (int64_t)g->n : 0) +
+             (g->lines ? (int64_t)tck::line_bytes(g->nnz) : 0) + (g->c16 ? (int64_t)tck::code_bytes(g->nnz) : 0) +
              (big ? (int64_t)g->n + g->nnz : 0) + sizeof(int32_t) * ((int64_t)g->nv_max + 1);
   *out = g.release();
   return TC_OK;
@@ -601,6 +616,7 @@ tc_status tc_graph_free(tc_ctx* ctx, tc_graph* g) try {
   dev_free(g->rp);
   dev_free(g->ci);
   g->drop_codes();
+  dev_free(g->lines);
   dev_free(g->d_desc);
   dev_free(g->own);
   dev_free(g->pown);
@@ -637,6 +653,7 @@ static tck::LaunchArgs count_args(tc_ctx* ctx, tc_graph* g) {
   a.P = (int64_t)g->nv_max + 1;
   a.rp = g->rp;
   a.ci = g->ci;
+  a.lines = g->lines;
   g->partners.into(a);
   a.tune = to_kernel_tune(ctx->tune);
   a.bufs = ctx->scratch.bufs();
@@ -652,13 +669,6 @@ static tck::LaunchArgs count_args(tc_ctx* ctx, tc_graph* g) {
 }  // extern "C"
 
 namespace tcr {
-
-// Index of the first group with work (it runs on the library stream).
-static int first_group(const bool* any, int n) {
-  for (int gi = 0; gi < n; ++gi)
-    if (any[gi]) return gi;
-  return 0;
-}
 
 // The binned count over plan buffers `bufs`.  kept: the plan in bufs is
 // already built for this graph and tune (its rows per bin in bins[]): re-arm
@@ -689,32 +699,20 @@ static tc_status binned_count(tc_ctx* ctx, tc_graph* g, const tck::PlanBufs& buf
     for (int b = 0; b < tck::kNumBins; ++b) bins[b] = c[tck::kCntBinCount + b];
   }
   TC_HIP_TRY(hipEventRecord(ctx->ev[1], s));
-  // The bin groups (tck::kBinOrder) run on separate streams (default
-  // priority): each group's persistent workgroups hold their CUs until its
-  // bins drain; the dispatcher interleaves the groups' workgroups from the
-  // start and the others take over the CUs a group's tail frees.  Groups
-  // with no tiles are skipped; one non-empty group runs on the library
-  // stream alone.
-  const tck::BinGroups& G = tck::kBinOrder;
-  bool any[tck::kBinGroups] = {};
-  const int last = tck::core_last_bin(a, bins);
-  for (int gi = 0; gi < G.n; ++gi)
-    for (int j = 0; j < G.len[gi]; ++j) {
-      const int b = G.bin[gi][j];
-      int64_t rows = b > tck::BIN_WAVE && b <= last ? 0 : bins[b];  // counted with the wave bin's
-      for (int x = tck::BIN_WAVE + 1; b == tck::BIN_WAVE && x <= last; ++x) rows += bins[x];
-      any[gi] = any[gi] || rows > 0;
-    }
-  const int g0 = first_group(any, G.n);
+  // The parts run side by side: their persistent workgroups share the CUs and
+  // take over those that another part's tail frees.  The first part with rows
+  // runs on the library stream.
+  bool first = true;
   int side = 0;
-  for (int gi = 0; gi < G.n; ++gi) {
-    if (!any[gi]) continue;
+  for (int p = 0; p < tck::kCountParts; ++p) {
+    if (tck::part_empty(a, p, bins)) continue;
     hipStream_t gs = s;
-    if (gi != g0) {
+    if (!first) {
       gs = ctx->side[side++];
-      TC_HIP_TRY(hipStreamWaitEvent(gs, ctx->ev[1], 0));  // timing starts before any group
+      TC_HIP_TRY(hipStreamWaitEvent(gs, ctx->ev[1], 0));  // timing starts before any part
     }
-    TC_HIP_TRY(tck::launch_count_order(a, ctx->cus, ctx->tune.grid, G.bin[gi], G.len[gi], bins, gs));
+    first = false;
+    TC_HIP_TRY(tck::launch_count_part(a, ctx->cus, ctx->tune.grid, p, bins, gs));
   }
   for (int i = 0; i < side; ++i) {
     TC_HIP_TRY(hipEventRecord(ctx->join[i], ctx->side[i]));
@@ -1046,17 +1044,7 @@ tc_status tc_count_local(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_local* ou
   TC_HIP_TRY(tck::launch_zero(L.pe, 2 * (int64_t)tck::kMaxParts, s));
   TC_HIP_TRY(tck::launch_plan(a, s));
   TC_HIP_TRY(hipEventRecord(ctx->ev[1], s));
-  {  // bin groups on the library stream and the side streams, as in tc_count
-    const tck::BinGroups& G = mode == tck::kLocalEdges ? tck::kEdgesBinOrder : tck::kBinOrder;
-    for (int gi = 0; gi < G.n; ++gi) {
-      hipStream_t gs = gi == 0 ? s : ctx->side[gi - 1];
-      if (gi > 0) TC_HIP_TRY(hipStreamWaitEvent(gs, ctx->ev[1], 0));
-      for (int j = 0; j < G.len[gi]; ++j)
-        TC_HIP_TRY(tck::launch_count_local(a, ctx->cus, G.bin[gi][j], G.bin[gi][j], mode, gs));
-      if (gi > 0) TC_HIP_TRY(hipEventRecord(ctx->join[gi - 1], gs));
-    }
-    for (int gi = 1; gi < G.n; ++gi) TC_HIP_TRY(hipStreamWaitEvent(s, ctx->join[gi - 1], 0));
-  }
+  TC_HIP_TRY(tck::launch_count_local(a, ctx->cus, mode, s));
   if (k > 0 && !parts_only)
     TC_HIP_TRY(tck::launch_local_parts(g->ci, L.esrc, g->n, g->edge_begin, g->edge_end, L.ecount, L.bounds, k, L.pe,
                                        ctx->cus, s));
