@@ -27,7 +27,7 @@ LIB = os.path.join(PKG, "lib")
 OBJ = os.path.join(PKG, "lib", "obj")
 
 HOST_SOURCES = ["host/csr.cpp", "host/gen.cpp", "host/partition.cpp", "host/metis.cpp", "host/arena.cpp"]
-HIP_SOURCES = ["hip/tc_kernels.hip", "hip/tc_runtime.cpp", "hip/tc_batch.cpp",
+HIP_SOURCES = ["hip/tc_kernels.hip", "hip/tc_runtime.cpp", "hip/tc_copy.cpp", "hip/tc_batch.cpp",
                "hip/tc_server.cpp", "hip/tc_tune.cpp"]
 
 HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-fopenmp", "-march=x86-64-v3",

@@ -515,6 +515,7 @@ void tc_ctx_destroy(tc_ctx* ctx) {
     DeviceGuard guard(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     ctx->scratch.release();
+    ctx->stager.release();
     dev_free(ctx->plain_out);
     dev_free(ctx->once_dev);
     for (auto& ev : ctx->ev)
@@ -1056,12 +1057,12 @@ tc_status tc_count_local(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_local* ou
   TC_HIP_TRY(hipStreamSynchronize(s));
   *total = sum_outs(ctx);
   const int64_t fallbacks = ((const uint32_t*)(ctx->pinned + 8))[tck::kCntFallback];
-  // pageable destinations: synchronous copies after the stream is done
+  // synchronous copies after the stream is done: the destinations are pageable
   if (out->edge_counts && g->edge_end > g->edge_begin)
-    TC_HIP_TRY(hipMemcpy(out->edge_counts, L.ecount + g->edge_begin,
-                         sizeof(uint32_t) * (size_t)(g->edge_end - g->edge_begin), hipMemcpyDeviceToHost));
+    TC_HIP_TRY(ctx->stager.to_host(out->edge_counts, L.ecount + g->edge_begin,
+                                   sizeof(uint32_t) * (size_t)(g->edge_end - g->edge_begin), s));
   if (out->vertex_counts && g->n > 0)
-    TC_HIP_TRY(hipMemcpy(out->vertex_counts, L.vcount, sizeof(uint64_t) * (size_t)g->n, hipMemcpyDeviceToHost));
+    TC_HIP_TRY(ctx->stager.to_host(out->vertex_counts, L.vcount, sizeof(uint64_t) * (size_t)g->n, s));
   if (k > 0)
     TC_HIP_TRY(hipMemcpy(out->part_counts, L.pe, sizeof(uint64_t) * (size_t)k, hipMemcpyDeviceToHost));
   if (parts_only) {  // every row's hits went to a part

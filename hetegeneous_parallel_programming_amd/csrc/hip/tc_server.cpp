@@ -53,10 +53,11 @@ struct Layout {
 // kMaxOutDegree, ids in [0, n).  One read of the caller's arrays, in plain
 // loops -- an OpenMP region per call, from several client threads at once,
 // costs far more than the loops themselves for graphs of a few thousand ids.
-// A large request is split over a few helper threads, since one thread
-// moves ~9 GB/s and an RMAT-20 request holds ~71 MB of CSR.
-constexpr size_t kCopySplit = (size_t)8 << 20;  // bytes per helper thread at least
-constexpr int kCopyThreads = 4;
+// A large request is split over helper threads, since one thread
+// moves ~9 GB/s and an RMAT-20 request holds ~71 MB of CSR (two of those among
+// 254 light ones: 4 threads of 8 MB and more 16.2 ms, these 15.3).
+constexpr size_t kCopySplit = (size_t)1 << 20;  // bytes per helper thread at least
+constexpr int kCopyThreads = 8;
 constexpr int64_t kMaxOutDegree = (int64_t)1 << 25;  // d * 64 < 2^31 in the plan's wedge-work field
 
 struct ShapeFlags {

@@ -90,3 +90,27 @@ def test_lines_of_owned_rows_and_partitions(ctx):
     pg = PartitionedGraph(g, 2, balance="partner")
     parts = [ctx.count_binned(ctx.upload_partition(pg.halo_partition(i)))[0] for i in range(2)]
     assert sum(parts) == oracle.tc_count(rp, ci)
+
+
+@pytest.mark.parametrize("m", [(1 << 21) - 1, 1 << 21, (1 << 21) + 1, (1 << 22) + 4099, (5 << 20) + 3])
+def test_large_edge_counts_reach_the_host(ctx, m):
+    # outputs around 8 MB and around the copies' chunks: triples of rows with
+    # three edges, four in five of them a triangle (only its first edge's ends
+    # share an out-neighbour), then one edge a row
+    k = m // 3 - 1
+    i = np.arange(k)
+    tri = i % 5 != 0
+    src = np.stack([3 * i, 3 * i, 3 * i + 1], 1)
+    dst = np.stack([np.where(tri, 3 * i + 1, 3 * i + 2), np.where(tri, 3 * i + 2, 3 * i + 3), 3 * i + 2], 1)
+    rest = m - 3 * k
+    n = 3 * k + rest + 1
+    src = np.concatenate([src.ravel(), 3 * k + np.arange(rest)])
+    ci = np.concatenate([dst.ravel(), 3 * k + 1 + np.arange(rest)]).astype(np.int32)
+    rp = np.zeros(n + 1, np.int64)
+    np.cumsum(np.bincount(src, minlength=n), out=rp[1:])
+    want = np.zeros(m, np.uint32)
+    want[3 * i[tri]] = 1
+    dg = ctx.upload_arrays(rp, ci)
+    for _ in range(2):
+        total, out = ctx.count_local(dg, vertices=False)
+        assert total == tri.sum() and (out["edge_counts"] == want).all()
