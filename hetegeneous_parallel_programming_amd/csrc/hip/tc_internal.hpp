@@ -177,12 +177,11 @@ struct tc_ctx {
   tcr::PlanScratch scratch;
   tcr::Stager stager;
   uint64_t* pinned = nullptr;  // 64 B count + 64 B bin counters
+  uint64_t* pinned_dev = nullptr;  // its device address
   void* noalloc = nullptr;     // device address of the static scratch of tc_count_noalloc
-  // device: the single-launch count's two words, used in turn; each launch
-  // clears the other one for the next call (plain_dirty: a call that did
-  // not finish left them unknown)
+  // device: the single-launch count's word, which every call leaves 0
+  // (plain_dirty: unless it did not finish)
   uint64_t* plain_out = nullptr;
-  int plain_turn = 0;
   bool plain_dirty = false;
   // tc_count_csr's copy of a small graph: rowptr, then colidx at the next
   // 256-byte boundary (grow-only, kept until destroy)
@@ -225,6 +224,7 @@ struct tc_graph {
   // rows per bin (which size the launches) on the host.
   tcr::PlanScratch plan;
   bool plan_valid = false;
+  bool plan_armed = false;  // its queue heads and sums are 0
   tc_tune plan_tune{};
   int64_t plan_bins[tck::kNumBins] = {};
 };

@@ -2894,11 +2894,9 @@ __global__ __launch_bounds__(kBlock, TC_COUNT_WAVES_PER_EU) void plain_kernel(co
                                                        const int32_t* __restrict__ ci,
                                                        int32_t row_begin, int32_t row_end,
                                                        const uint8_t* own, uint64_t* out,
-                                                       uint64_t* zero_next) {
+                                                       uint64_t* host) {
   __shared__ PlainLds L;
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  // the next call's word, cleared here instead of by a launch of its own
-  if (zero_next && blockIdx.x == 0 && threadIdx.x == 0) *zero_next = 0;
   const int64_t nw = (int64_t)gridDim.x * kWaves;
   uint64_t acc = 0;
   for (int64_t u = row_begin + (int64_t)blockIdx.x * kWaves + wid; u < row_end; u += nw) {
@@ -2921,7 +2919,20 @@ __global__ __launch_bounds__(kBlock, TC_COUNT_WAVES_PER_EU) void plain_kernel(co
     }
   }
   const uint64_t tot = block_sum(acc, L.red);
-  if (threadIdx.x == 0 && tot) atomicAdd(out, tot);
+  if (host) {
+    // one add carries the sum and, above bit 48, the workgroups that are
+    // done: the last one has the total, hands it over and clears the word
+    // (ER n=1000 d=32: 28.8 -> 22.4 us a call without the copy and its launch)
+    if (threadIdx.x == 0) {
+      const uint64_t old = atomicAdd((unsigned long long*)out, tot + (1ull << kDoneShift));
+      if (old >> kDoneShift == gridDim.x - 1) {
+        *host = (old + tot) & ((1ull << kDoneShift) - 1);
+        *out = 0;
+      }
+    }
+  } else if (threadIdx.x == 0 && tot) {
+    atomicAdd(out, tot);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -3022,6 +3033,27 @@ __global__ void rearm_kernel(uint32_t* counters, uint64_t* outs, int32_t nouts) 
 
 hipError_t launch_rearm(uint32_t* counters, uint64_t* outs, int32_t nouts, hipStream_t s) {
   rearm_kernel<<<1, kBlock, 0, s>>>(counters, outs, nouts);
+  return hipGetLastError();
+}
+
+__global__ __launch_bounds__(kBlock) void finish_kernel(uint32_t* counters, uint64_t* outs, uint64_t* host) {
+  const int i = threadIdx.x;
+  uint64_t x = i < kOutSlots ? outs[i * kOutStride] : 0;
+  const uint32_t fallbacks = counters[kCntFallback];
+#pragma unroll
+  for (int d = kOutSlots / 2; d >= 1; d >>= 1) x += shfl_down_u64(x, d);
+  __syncthreads();
+  if (i < kOutSlots) outs[i * kOutStride] = 0ull;
+  if (i < 8 * kNumHeads) counters[kCntHeads + kHeadStride * i] = 0u;
+  if (i == 0) {
+    counters[kCntFallback] = 0u;
+    host[0] = x;
+    host[1] = fallbacks;
+  }
+}
+
+hipError_t launch_finish(uint32_t* counters, uint64_t* outs, uint64_t* host, hipStream_t s) {
+  finish_kernel<<<1, kBlock, 0, s>>>(counters, outs, host);
   return hipGetLastError();
 }
 
@@ -3190,8 +3222,8 @@ hipError_t launch_local_parts(const int32_t* ci, const int32_t* esrc, int64_t n,
 }
 
 hipError_t launch_plain(const int64_t* rp, const int32_t* ci, int32_t row_begin, int32_t row_end,
-                        const uint8_t* own, uint64_t* out, int grid, hipStream_t s, uint64_t* zero_next) {
-  plain_kernel<<<grid, kBlock, 0, s>>>(rp, ci, row_begin, row_end, own, out, zero_next);
+                        const uint8_t* own, uint64_t* out, int grid, hipStream_t s, uint64_t* host) {
+  plain_kernel<<<grid, kBlock, 0, s>>>(rp, ci, row_begin, row_end, own, out, host);
   return hipGetLastError();
 }
 

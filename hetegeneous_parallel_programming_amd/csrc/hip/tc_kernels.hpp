@@ -424,6 +424,13 @@ hipError_t launch_stage_copy(const StageCopy* copies, int32_t n, int64_t chunks,
 // Re-arms a kept plan for another count: tile queue heads and the fallback
 // counter to 0 (bin counts kept), outs[0..nouts) to 0.
 hipError_t launch_rearm(uint32_t* counters, uint64_t* outs, int32_t nouts, hipStream_t s);
+// The end of a single graph's count: its sum (of kOutSlots words) to host[0]
+// and its hash fallbacks to host[1] (pinned memory, by its device address),
+// and a rearm on the way, so that another count with the plan needs none.
+// One launch instead of two copies and the next call's rearm, each ~5 us and
+// as much again between launches (R-MAT n=30011: 85 -> 72 us a call, R-MAT-18
+// 215 -> 200).
+hipError_t launch_finish(uint32_t* counters, uint64_t* outs, uint64_t* host, hipStream_t s);
 hipError_t launch_plan(const LaunchArgs& a, hipStream_t s);
 // Bytes of a pool of ids with its lists on lines.
 inline size_t line_bytes(int64_t ids) { return sizeof(int32_t) * (size_t)(2 * ids + kCiPad); }
@@ -454,19 +461,24 @@ hipError_t launch_count(const LaunchArgs& a, int cus, int grid, hipStream_t s);
 // when the host does not know them; parts without rows launch nothing.
 // The bitmap kernels take the bins that keep a wave busy, or all bins of a
 // graph with few light rows (at most kCoreLightRows), where one more wide
-// launch beats narrow groups (R-MAT n=30011 d=24: 0.17 -> 0.10 ms) -- a wave
-// per light row is slower from a few rows per resident wave on (the batch of
-// 512 graphs, 215 K rows of the 32-lane bin: 0.53 ms there, 0.64 ms here).
-constexpr int64_t kCoreLightRows = 16384;
+// launch beats narrow groups (R-MAT n=30011 d=24: 0.17 -> 0.10 ms, ER n=32000
+// d=16: 75 -> 45 us, R-MAT n=65003 d=32: 121 -> 82; ER n=40000 d=16 with all
+// rows so: 78 -> 131) -- a wave per light row is slower from a few rows per
+// resident wave on (the batch of 512 graphs, 215 K rows of the 32-lane bin:
+// 0.53 ms there, 0.64 ms here).
+constexpr int64_t kCoreLightRows = 32768;
 constexpr int kPartBlock = 0, kPartWave = 1, kPartHash = 2, kCountParts = 3;
 bool part_empty(const LaunchArgs& a, int part, const int64_t* rows);
 hipError_t launch_count_part(const LaunchArgs& a, int cus, int grid, int part, const int64_t* rows, hipStream_t s);
 
 // own: null, or per row 1 if it is a pivot row (rows outside
-// [row_begin, row_end) are never pivots).  out must hold 0; zero_next (null,
-// or another word) is set to 0 by the kernel.
+// [row_begin, row_end) are never pivots).  out must hold 0.  host: null, or
+// where the last workgroup stores the sum (pinned memory, by its device
+// address), leaving 0 in out; for sums below 2^kDoneShift and grids below
+// 2^(64 - kDoneShift).
+constexpr int kDoneShift = 48;
 hipError_t launch_plain(const int64_t* rp, const int32_t* ci, int32_t row_begin, int32_t row_end,
-                        const uint8_t* own, uint64_t* out, int grid, hipStream_t s, uint64_t* zero_next = nullptr);
+                        const uint8_t* own, uint64_t* out, int grid, hipStream_t s, uint64_t* host = nullptr);
 // Count of one graph that also fills a.local: same plan, the local variants
 // of the hash kernel over all bins.  mode kLocalFull: ecount and vcount (zeroed by the
 // caller); kLocalEdges: ecount only (the kernels keep no slot hit counters:

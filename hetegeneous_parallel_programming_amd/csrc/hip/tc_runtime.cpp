@@ -16,15 +16,9 @@ namespace tcr {
 
 static thread_local std::string g_err;
 // ctx->pinned layout (uint64 words): [0] count, [8..) plan counters,
-// [kPinnedFallback] the count's hash-fallback counter, [kPinnedOuts..) a
-// count's sum words.
-constexpr int kPinnedFallback = 24, kPinnedOuts = 64;
-constexpr size_t kPinnedBytes = sizeof(uint64_t) * (kPinnedOuts + tck::kOutWords);
-static uint64_t sum_outs(const tc_ctx* ctx) {
-  uint64_t t = 0;
-  for (int i = 0; i < tck::kOutSlots; ++i) t += ctx->pinned[kPinnedOuts + i * tck::kOutStride];
-  return t;
-}
+// [kPinnedSum] a count's sum and hash fallbacks.
+constexpr int kPinnedSum = 24;
+constexpr size_t kPinnedBytes = sizeof(uint64_t) * 32;
 
 tc_status fail(tc_status st, const std::string& msg) {
   g_err = msg;
@@ -493,6 +487,7 @@ tc_status tc_ctx_create(int32_t device, tc_ctx** out) try {
   TC_HIP_TRY(hipEventCreateWithFlags(&c->fork, hipEventDisableTiming));
   for (auto& ev : c->ev) TC_HIP_TRY(hipEventCreate(&ev));
   TC_HIP_TRY(hipHostMalloc((void**)&c->pinned, kPinnedBytes, hipHostMallocDefault));
+  TC_HIP_TRY(hipHostGetDevicePointer((void**)&c->pinned_dev, c->pinned, 0));
   {
     tc_status st = dev_alloc((void**)&c->plain_out, 256, "plain count word");
     if (st != TC_OK) return st;
@@ -673,18 +668,21 @@ namespace tcr {
 
 // The binned count over plan buffers `bufs`.  kept: the plan in bufs is
 // already built for this graph and tune (its rows per bin in bins[]): re-arm
-// the tile queues and count.  Otherwise plan first (one host round trip for
-// the rows per bin, which size the launches) and fill bins[].
+// the tile queues, unless the last count with it left them so, and count.
+// Otherwise plan first (one host round trip for the rows per bin, which size
+// the launches) and fill bins[].
 static tc_status binned_count(tc_ctx* ctx, tc_graph* g, const tck::PlanBufs& bufs, bool kept, int64_t* bins,
                               uint64_t* total, tc_stats* stats) {
   const double t0 = now_ms();
   tck::LaunchArgs a = count_args(ctx, g);
   a.bufs = bufs;
   hipStream_t s = ctx->stream;
-  TC_HIP_TRY(hipEventRecord(ctx->ev[0], s));
+  const bool armed = kept && g->plan_armed;
+  g->plan_armed = false;
+  if (!armed) TC_HIP_TRY(hipEventRecord(ctx->ev[0], s));
   if (kept) {
-    TC_HIP_TRY(tck::launch_rearm(a.bufs.counters, a.bufs.outs, tck::kOutWords, s));
-    TC_HIP_TRY(hipEventRecord(ctx->ev[3], s));
+    if (!armed) TC_HIP_TRY(tck::launch_rearm(a.bufs.counters, a.bufs.outs, tck::kOutWords, s));
+    if (!armed) TC_HIP_TRY(hipEventRecord(ctx->ev[3], s));
   } else {
     TC_HIP_TRY(tck::launch_zero(a.bufs.counters, tck::kNumCounters, s));
     TC_HIP_TRY(tck::launch_zero(a.bufs.outs, 2 * tck::kOutWords, s));
@@ -702,13 +700,17 @@ static tc_status binned_count(tc_ctx* ctx, tc_graph* g, const tck::PlanBufs& buf
   TC_HIP_TRY(hipEventRecord(ctx->ev[1], s));
   // The parts run side by side: their persistent workgroups share the CUs and
   // take over those that another part's tail frees.  The first part with rows
-  // runs on the library stream.
+  // runs on the library stream.  Two bitmap kernels alone (a graph with few
+  // light rows) go one after the other: a wait for another stream's event
+  // takes ~15 us, twice, more than they gain by it (R-MAT n=30011: 72 -> 55
+  // us; with the hash kernel's part R-MAT-18 would go from 200 to 309 us).
+  const bool beside = !tck::part_empty(a, tck::kPartHash, bins);
   bool first = true;
   int side = 0;
   for (int p = 0; p < tck::kCountParts; ++p) {
     if (tck::part_empty(a, p, bins)) continue;
     hipStream_t gs = s;
-    if (!first) {
+    if (!first && beside) {
       gs = ctx->side[side++];
       TC_HIP_TRY(hipStreamWaitEvent(gs, ctx->ev[1], 0));  // timing starts before any part
     }
@@ -720,23 +722,20 @@ static tc_status binned_count(tc_ctx* ctx, tc_graph* g, const tck::PlanBufs& buf
     TC_HIP_TRY(hipStreamWaitEvent(s, ctx->join[i], 0));
   }
   TC_HIP_TRY(hipEventRecord(ctx->ev[2], s));
-  TC_HIP_TRY(hipMemcpyAsync(ctx->pinned + kPinnedOuts, a.bufs.outs, sizeof(uint64_t) * tck::kOutWords,
-                            hipMemcpyDeviceToHost, s));
-  TC_HIP_TRY(hipMemcpyAsync(ctx->pinned + kPinnedFallback, a.bufs.counters + tck::kCntFallback, sizeof(uint32_t),
-                            hipMemcpyDeviceToHost, s));
+  TC_HIP_TRY(tck::launch_finish(a.bufs.counters, a.bufs.outs, ctx->pinned_dev + kPinnedSum, s));
   TC_HIP_TRY(hipStreamSynchronize(s));
-  *total = sum_outs(ctx);
+  *total = ctx->pinned[kPinnedSum];
   if (stats) {
     std::memset(stats, 0, sizeof(*stats));
     stats->total_ms = now_ms() - t0;
     float ms = 0;
-    TC_HIP_TRY(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[3]));
+    if (!armed) TC_HIP_TRY(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[3]));
     stats->plan_ms = ms;
     TC_HIP_TRY(hipEventElapsedTime(&ms, ctx->ev[1], ctx->ev[2]));
     stats->count_ms = ms;
     stats->pivots = g->nv;
     for (int b = 0; b < TC_NUM_BINS; ++b) stats->bin_pivots[b] = bins[b];
-    stats->hash_fallbacks = *(const uint32_t*)(ctx->pinned + kPinnedFallback);
+    stats->hash_fallbacks = (int64_t)ctx->pinned[kPinnedSum + 1];
     stats->plan_kept = kept ? 1 : 0;
   }
   return TC_OK;
@@ -744,9 +743,9 @@ static tc_status binned_count(tc_ctx* ctx, tc_graph* g, const tck::PlanBufs& buf
 
 // The binned count with the plan kept in the graph.  The plan (rows per bin,
 // bin-major item lists) depends only on the graph's partner rows and the
-// launch setting, so it is built on the first call: later calls re-arm the
-// tile queues and launch the sized bins directly -- no planning kernels and
-// no host round trip before the count.
+// launch setting, so it is built on the first call: later calls launch the
+// sized kernels directly -- no planning kernels and no host round trip before
+// the count, whose last kernel leaves the plan ready for the next.
 static tc_status count_binned(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_stats* stats) {
   const int64_t P = (int64_t)g->nv_max + 1;
   const bool kept = g->plan_valid && std::memcmp(&g->plan_tune, &ctx->tune, sizeof(tc_tune)) == 0;
@@ -758,6 +757,7 @@ static tc_status count_binned(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_stat
     g->plan_valid = false;
   }
   tc_status st = binned_count(ctx, g, g->plan.bufs(), kept, g->plan_bins, total, stats);
+  g->plan_armed = st == TC_OK;
   if (st == TC_OK && !kept) {
     g->plan_tune = ctx->tune;
     g->plan_valid = true;
@@ -765,38 +765,30 @@ static tc_status count_binned(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_stat
   return st;
 }
 
+static bool small_graph(const tc_graph* g);
+
 // The plain kernel's single launch, its u64 sum at `out` on the device.
-// kept_zero: `out` is the context's plain-count word, zero between calls:
-// no zero launch before the kernel; it is cleared again after the result is
-// read, off the caller's critical path (the next launch on the stream waits
-// for it).
+// kept_zero: `out` is the context's plain-count word, zero between calls: no
+// zero launch before the kernel.
 static tc_status plain_count(tc_ctx* ctx, tc_graph* g, uint64_t* out, uint64_t* total, tc_stats* stats,
                              bool kept_zero = false) {
   const double t0 = now_ms();
   const int64_t P = (int64_t)g->row_end - g->row_begin;
   hipStream_t s = ctx->stream;
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(ctx->plain_grid, (P + tck::kWaves - 1) / tck::kWaves));
-  // kept_zero: out is the context's pair of words, one per call in turn
-  uint64_t* word = out;
-  uint64_t* next = nullptr;
-  if (kept_zero) {
-    if (ctx->plain_dirty) TC_HIP_TRY(tck::launch_zero(out, 4, s));
-    ctx->plain_dirty = true;
-    word = out + ctx->plain_turn;
-    next = out + (1 - ctx->plain_turn);
-  } else {
-    TC_HIP_TRY(tck::launch_zero(out, 2, s));
-  }
+  // A small graph's sum (at most ids * kCapWave) leaves room for the count of
+  // finished workgroups above it.
+  const bool direct = small_graph(g) && grid < 1 << (64 - tck::kDoneShift);
+  if (!kept_zero || ctx->plain_dirty || !direct) TC_HIP_TRY(tck::launch_zero(out, 2, s));
+  if (kept_zero) ctx->plain_dirty = true;
   TC_HIP_TRY(hipEventRecord(ctx->ev[1], s));
-  TC_HIP_TRY(tck::launch_plain(g->rp, g->ci, g->row_begin, g->row_end, g->own, word, grid, s, next));
+  TC_HIP_TRY(tck::launch_plain(g->rp, g->ci, g->row_begin, g->row_end, g->own, out, grid, s,
+                               direct ? ctx->pinned_dev : nullptr));
   TC_HIP_TRY(hipEventRecord(ctx->ev[2], s));
-  TC_HIP_TRY(hipMemcpyAsync(ctx->pinned, word, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+  if (!direct) TC_HIP_TRY(hipMemcpyAsync(ctx->pinned, out, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
   TC_HIP_TRY(hipStreamSynchronize(s));
   *total = ctx->pinned[0];
-  if (kept_zero) {
-    ctx->plain_turn = 1 - ctx->plain_turn;
-    ctx->plain_dirty = false;
-  }
+  if (kept_zero && direct) ctx->plain_dirty = false;
   tc_status st = finish_stats(ctx, stats, t0, false, P);
   if (st == TC_OK && stats) stats->single_launch = 1;
   return st;
@@ -1050,13 +1042,12 @@ tc_status tc_count_local(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_local* ou
     TC_HIP_TRY(tck::launch_local_parts(g->ci, L.esrc, g->n, g->edge_begin, g->edge_end, L.ecount, L.bounds, k, L.pe,
                                        ctx->cus, s));
   TC_HIP_TRY(hipEventRecord(ctx->ev[2], s));
-  TC_HIP_TRY(hipMemcpyAsync(ctx->pinned + kPinnedOuts, a.bufs.outs, sizeof(uint64_t) * tck::kOutWords,
-                            hipMemcpyDeviceToHost, s));
+  TC_HIP_TRY(tck::launch_finish(a.bufs.counters, a.bufs.outs, ctx->pinned_dev + kPinnedSum, s));
   TC_HIP_TRY(hipMemcpyAsync(ctx->pinned + 8, a.bufs.counters, sizeof(uint32_t) * tck::kPlanWords,
                             hipMemcpyDeviceToHost, s));
   TC_HIP_TRY(hipStreamSynchronize(s));
-  *total = sum_outs(ctx);
-  const int64_t fallbacks = ((const uint32_t*)(ctx->pinned + 8))[tck::kCntFallback];
+  *total = ctx->pinned[kPinnedSum];
+  const int64_t fallbacks = (int64_t)ctx->pinned[kPinnedSum + 1];
   // synchronous copies after the stream is done: the destinations are pageable
   if (out->edge_counts && g->edge_end > g->edge_begin)
     TC_HIP_TRY(ctx->stager.to_host(out->edge_counts, L.ecount + g->edge_begin,
