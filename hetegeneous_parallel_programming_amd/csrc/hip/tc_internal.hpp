@@ -179,8 +179,8 @@ struct tc_ctx {
   uint64_t* pinned = nullptr;  // 64 B count + 64 B bin counters
   uint64_t* pinned_dev = nullptr;  // its device address
   void* noalloc = nullptr;     // device address of the static scratch of tc_count_noalloc
-  // device: the single-launch count's word, which every call leaves 0
-  // (plain_dirty: unless it did not finish)
+  // device: the single-launch count's kOutWords words, which every call
+  // leaves 0 (plain_dirty: unless it did not finish); then an upload's word
   uint64_t* plain_out = nullptr;
   bool plain_dirty = false;
   // tc_count_csr's copy of a small graph: rowptr, then colidx at the next

@@ -2920,14 +2920,25 @@ __global__ __launch_bounds__(kBlock, TC_COUNT_WAVES_PER_EU) void plain_kernel(co
   }
   const uint64_t tot = block_sum(acc, L.red);
   if (host) {
-    // one add carries the sum and, above bit 48, the workgroups that are
-    // done: the last one has the total, hands it over and clears the word
-    // (ER n=1000 d=32: 28.8 -> 22.4 us a call without the copy and its launch)
+    // One add carries a sum and, above bit kDoneShift, how many workgroups it
+    // has: the last of a word adds the word to the root, the last of those has
+    // the total, hands it over, and all words are 0 again (ER n=1000 d=32:
+    // 28.8 -> 22 us a call without the copy and its launch).  32 words, since
+    // one serves an add per ~12 ns (2048 workgroups: 25 us).
     if (threadIdx.x == 0) {
-      const uint64_t old = atomicAdd((unsigned long long*)out, tot + (1ull << kDoneShift));
-      if (old >> kDoneShift == gridDim.x - 1) {
-        *host = (old + tot) & ((1ull << kDoneShift) - 1);
-        *out = 0;
+      constexpr uint64_t one = 1ull << kDoneShift;
+      const uint32_t s = blockIdx.x % kOutSlots, words = min(gridDim.x, (uint32_t)kOutSlots);
+      unsigned long long* w = (unsigned long long*)out + s * kOutStride;
+      unsigned long long* root = (unsigned long long*)out + kOutStride / 2;
+      const uint64_t old = atomicAdd(w, tot + one);
+      if (old >> kDoneShift == (gridDim.x - s + kOutSlots - 1) / kOutSlots - 1) {
+        const uint64_t sum = (old + tot) & (one - 1);
+        *w = 0;
+        const uint64_t before = atomicAdd(root, sum + one);
+        if (before >> kDoneShift == words - 1) {
+          *host = (before + sum) & (one - 1);
+          *root = 0;
+        }
       }
     }
   } else if (threadIdx.x == 0 && tot) {

@@ -474,8 +474,8 @@ hipError_t launch_count_part(const LaunchArgs& a, int cus, int grid, int part, c
 // own: null, or per row 1 if it is a pivot row (rows outside
 // [row_begin, row_end) are never pivots).  out must hold 0.  host: null, or
 // where the last workgroup stores the sum (pinned memory, by its device
-// address), leaving 0 in out; for sums below 2^kDoneShift and grids below
-// 2^(64 - kDoneShift).
+// address); out is then kOutWords words, left 0.  For sums below 2^kDoneShift
+// and grids below 2^(64 - kDoneShift).
 constexpr int kDoneShift = 48;
 hipError_t launch_plain(const int64_t* rp, const int32_t* ci, int32_t row_begin, int32_t row_end,
                         const uint8_t* own, uint64_t* out, int grid, hipStream_t s, uint64_t* host = nullptr);

@@ -19,6 +19,7 @@ static thread_local std::string g_err;
 // [kPinnedSum] a count's sum and hash fallbacks.
 constexpr int kPinnedSum = 24;
 constexpr size_t kPinnedBytes = sizeof(uint64_t) * 32;
+constexpr size_t kPlainBytes = sizeof(uint64_t) * (tck::kOutWords + 1);
 
 tc_status fail(tc_status st, const std::string& msg) {
   g_err = msg;
@@ -404,14 +405,14 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
     a.core_kb = tck::core_bits(g->n);
     if (big)  // (the build's scratch is free until the build)
       e = tck::launch_big_codes(g->rp, g->ci, g->n, g->nnz, bs.mem, g->c16, g->closed, g->part,
-                                (unsigned long long*)ctx->plain_out + 4, ctx->cus, s);
+                                (unsigned long long*)ctx->plain_out + tck::kOutWords, ctx->cus, s);
     if (e == hipSuccess) st = launch_build(a, (int64_t)g->n + 1, g->nnz, bs, s, nullptr, g->pown, g->closed, g->part,
                                              big ? nullptr : g->c16, g->lines);
     if (st == TC_OK && e == hipSuccess) e = hipEventRecord(ctx->ev[1], s);
     if (st == TC_OK && e == hipSuccess)
       e = hipMemcpyAsync(ctx->pinned, g->partners.nv, sizeof(int32_t), hipMemcpyDeviceToHost, s);
     if (big && st == TC_OK && e == hipSuccess)
-      e = hipMemcpyAsync(ctx->pinned + 1, ctx->plain_out + 4, sizeof(uint64_t), hipMemcpyDeviceToHost, s);
+      e = hipMemcpyAsync(ctx->pinned + 1, ctx->plain_out + tck::kOutWords, sizeof(uint64_t), hipMemcpyDeviceToHost, s);
     if (st == TC_OK && e == hipSuccess) e = hipStreamSynchronize(s);
   }
   bs.release();
@@ -489,9 +490,9 @@ tc_status tc_ctx_create(int32_t device, tc_ctx** out) try {
   TC_HIP_TRY(hipHostMalloc((void**)&c->pinned, kPinnedBytes, hipHostMallocDefault));
   TC_HIP_TRY(hipHostGetDevicePointer((void**)&c->pinned_dev, c->pinned, 0));
   {
-    tc_status st = dev_alloc((void**)&c->plain_out, 256, "plain count word");
+    tc_status st = dev_alloc((void**)&c->plain_out, kPlainBytes, "plain count words");
     if (st != TC_OK) return st;
-    TC_HIP_TRY(hipMemset(c->plain_out, 0, 256));
+    TC_HIP_TRY(hipMemset(c->plain_out, 0, kPlainBytes));
   }
   // device address of the allocation-free count's static scratch (this device's copy)
   TC_HIP_TRY(tck::noalloc_scratch_address(&c->noalloc));
@@ -767,9 +768,9 @@ static tc_status count_binned(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_stat
 
 static bool small_graph(const tc_graph* g);
 
-// The plain kernel's single launch, its u64 sum at `out` on the device.
-// kept_zero: `out` is the context's plain-count word, zero between calls: no
-// zero launch before the kernel.
+// The plain kernel's single launch, summing in the tck::kOutWords words at
+// `out` on the device.  kept_zero: those are the context's, zero between
+// calls: no zero launch before the kernel.
 static tc_status plain_count(tc_ctx* ctx, tc_graph* g, uint64_t* out, uint64_t* total, tc_stats* stats,
                              bool kept_zero = false) {
   const double t0 = now_ms();
@@ -779,7 +780,7 @@ static tc_status plain_count(tc_ctx* ctx, tc_graph* g, uint64_t* out, uint64_t* 
   // A small graph's sum (at most ids * kCapWave) leaves room for the count of
   // finished workgroups above it.
   const bool direct = small_graph(g) && grid < 1 << (64 - tck::kDoneShift);
-  if (!kept_zero || ctx->plain_dirty || !direct) TC_HIP_TRY(tck::launch_zero(out, 2, s));
+  if (!kept_zero || ctx->plain_dirty || !direct) TC_HIP_TRY(tck::launch_zero(out, 2 * tck::kOutWords, s));
   if (kept_zero) ctx->plain_dirty = true;
   TC_HIP_TRY(hipEventRecord(ctx->ev[1], s));
   TC_HIP_TRY(tck::launch_plain(g->rp, g->ci, g->row_begin, g->row_end, g->own, out, grid, s,
