@@ -143,8 +143,9 @@ tc_status tc_count_binned(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_stats* s
 /* tc_count on a graph whose every list is under 1024 ids and whose counted
  * rows hold at most 2^18 DAG ids -- or, for a flat graph, at most 2^21 ids
  * in at most 2^17 rows with lists of at most 64 -- runs tc_count_plain's
- * single launch instead (stats->single_launch = 1): there one launch is
- * faster than planning plus the binned kernels' launches.  Both are exact.
+ * single launch instead (stats->single_launch = 1), which needs no plan.
+ * Both are exact.  stats->plan_ms of a binned count is 0 when the count
+ * before it with the kept plan left the plan ready.
  * tc_count_plain: one launch of the plain kernel, one wave64 per pivot,
  * grid-stride over pivots at full residency -- the direct restatement of
  * warp_vertex (bs_warp_vertex.cuh:2-35, grid a17 of
