@@ -2291,8 +2291,8 @@ struct __align__(16) CoreLds {
 // where lists start, so the list of each of 64 consecutive chunks is one
 // broadcast LDS read and two mbcnt, whatever the lists' lengths.  Codes past
 // a list's end do not count, and a load may run past the pool's end
-// (kCorePad).
-__device__ __forceinline__ uint32_t core_batch(const char* __restrict__ pool, const uint8_t* B, CoreWave& W,
+// (kCorePad).  kb: 2^kb bytes of B are the bitmap.
+__device__ __forceinline__ uint32_t core_batch(const char* __restrict__ pool, const uint8_t* B, int kb, CoreWave& W,
                                                uint32_t len, uint32_t off, int lane) {
   constexpr int NC = kCoreInFlight, CH = kCoreChunk;
   static_assert(kCoreSpan % (64 * NC) == 0 && kCoreSpan / 64 <= 64, "spans are whole iterations");
@@ -2335,7 +2335,7 @@ __device__ __forceinline__ uint32_t core_batch(const char* __restrict__ pool, co
 #pragma unroll
         for (int i = 0; i < CH / 2; ++i) {
           const uint32_t w = d[q][i];
-          const uint32_t lo = B[w & 0x1FFFu], hi = B[(w >> 16) & 0x1FFFu];
+          const uint32_t lo = B[code_byte(w, 0, kb)], hi = B[code_byte(w, 1, kb)];
           r = __builtin_amdgcn_alignbit(lo >> ((w >> kCoreByteBits) & 7u), r, 1);
           r = __builtin_amdgcn_alignbit(hi >> (w >> 29), r, 1);
         }
@@ -2402,7 +2402,7 @@ __global__ __launch_bounds__(64 * NW, 8) void core_kernel(LaunchArgs a, int bin0
       r0 = lane < per && j < np ? a.pci[pb + j] : (ListRef)0;  // the next batch's
       const uint32_t full = (uint32_t)list_len(r);
       const uint32_t len = ref_marks(r, kMarkClosed) ? closed_len(r) : all ? full : 0u;
-      hits += core_batch(pool, B, L.w[wid], len, code_start(list_start(r), full) * 2u, lane);
+      hits += core_batch(pool, B, a.core_kb, L.w[wid], len, code_start(list_start(r), full) * 2u, lane);
     }
     if (batch) {  // one atomic per wave and row
       uint32_t h = hits;

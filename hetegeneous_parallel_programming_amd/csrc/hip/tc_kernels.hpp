@@ -124,6 +124,13 @@ __host__ __device__ constexpr uint32_t core_code(uint32_t i, int kb) {
   return (r >> kb) << kCoreByteBits | (r & ((1u << kb) - 1u));
 }
 constexpr uint16_t kNoCode = (uint16_t)core_code(65535, kCoreByteBits);
+// The bitmap byte of the code in half `half` of a word: below 2^kb whatever the
+// 16 bits are.  A load may hold what no list owns (the room between lists, what
+// is past the pool's last), which is looked up like any code and not counted;
+// with the 13 bits of the largest bitmap it would read past a smaller one.
+__host__ __device__ inline uint32_t code_byte(uint32_t word, int half, int kb) {
+  return (word >> (16 * half)) & ((1u << kb) - 1u);
+}
 // Smallest kb for n vertices (the bitmap is cleared 16 bytes per lane of a wave).
 inline int core_bits(int64_t n) {
   int kb = 10;
