@@ -84,7 +84,7 @@ static uint64_t count_metis(const std::string& spec) {
       tch_csr_view(sub, &v);
       tc_graph* dg = nullptr;
       uint64_t cnt = 0;
-      tc_status st = tc_graph_upload_rows(dev.get(), &v, owned.data(), TC_CHECK_SHAPE, &dg);
+      tc_status st = tc_graph_upload_rows(dev.get(), &v, owned.data(), TC_CHECK_SHAPE | TC_UPLOAD_ONCE, &dg);
       if (st == TC_OK) st = tc_count(dev.get(), dg, &cnt, nullptr);
       tc_graph_free(dev.get(), dg);
       tch_csr_free(sub);

@@ -296,15 +296,24 @@ tck::Tune to_kernel_tune(const tc_tune& t) {
 
 // Host-side checks shared by every upload: shape (and more when asked), and
 // the per-batch int32 element total (64 lists of at most max_out ids).
-static tc_status check_dag(const tc_csr_view* dag, uint32_t check, int32_t* max_out) {
+struct DagShape {
+  int32_t max_out = 0;
+  uint64_t squares = 0;  // sum over rows of out-degree squared: bounds the ids a count streams
+};
+static tc_status check_dag(const tc_csr_view* dag, uint32_t check, DagShape* shape) {
   if (!dag) return fail(TC_EINVAL, "null csr view");
   tc_status st = tch_validate(dag, check | TC_CHECK_SHAPE);
   if (st != TC_OK) return fail(st, tch_last_error());
   int64_t mo = 0;
-  for (int64_t v = 0; v < dag->n_rows; ++v) mo = std::max<int64_t>(mo, dag->rowptr[v + 1] - dag->rowptr[v]);
+  uint64_t squares = 0;  // (below 2^64 for any graph that passes)
+  for (int64_t v = 0; v < dag->n_rows; ++v) {
+    const int64_t d = dag->rowptr[v + 1] - dag->rowptr[v];
+    mo = std::max<int64_t>(mo, d);
+    squares += (uint64_t)d * (uint64_t)d;
+  }
   if (mo * 64 >= ((int64_t)1 << 31))
     return fail(TC_ERANGE, "DAG out-degree too large (max_out * 64 must fit in int32)");
-  *max_out = (int32_t)mo;
+  *shape = DagShape{(int32_t)mo, squares};
   return TC_OK;
 }
 
@@ -312,16 +321,34 @@ static tc_status check_dag(const tc_csr_view* dag, uint32_t check, int32_t* max_
 // flat ones have no set of 65535 vertices that most edges lead to.
 constexpr int32_t kCodesMinOut = 64;
 
+// Whether the codes of a graph past tck::kCoreIds rows repay in one count.
+// They shorten it by a share of its time, which goes with the ids it streams
+// (at most `squares`), and cost an allocation and a pass per id: so only where
+// there is much to stream, much of it per id, and by a few long lists (at
+// 4 times the squares of a graph of equal lists; flat graphs have about 1.25).
+// One-shot calls on MI355X, without / with codes, ms: R-MAT n=333333 of 8 M
+// ids (165 squares an id) 4.07 / 4.59, n=1000000 of 15 M (151) 7.05 / 7.49,
+// n=6000000 of 30 M (80) 17.4 / 18.4; n=2000000 of 30 M (179) 13.5 / 13.0,
+// n=500000 of 30 M (419) 13.4 / 11.0, n=4266666 of 64 M (218) 28.7 / 26.1; ER
+// n=1250000 of 60 M (60, lists to 86) 16.6 / 18.8.
+constexpr uint64_t kOnceSquares = (uint64_t)1 << 32, kOnceSquaresPerId = 128;
+static bool once_repays_codes(int64_t n, int64_t nnz, uint64_t squares) {
+  return squares >= kOnceSquares && squares >= kOnceSquaresPerId * (uint64_t)nnz &&
+         (double)squares * (double)n >= 4.0 * (double)nnz * (double)nnz;
+}
+
 // Flat graphs (past tck::kCoreIds rows, no list of kCodesMinOut ids) of this
 // many ids on get their lists on lines as well: an edge's list is then read in
 // one 128-byte line instead of 1.5, and such a count is bound by the lines it
 // reads beyond L2 (ER n=2000003 d=33: 1.03 -> 0.90 ms, of a build 1.73 -> 1.81
 // ms).  With codes the other lists are few (R-MAT-22: 3.24, with lines 3.30
-// ms), and fewer ids stay in an XCD's L2 (4 MB).
+// ms), and fewer ids stay in an XCD's L2 (4 MB).  A graph counted once gets
+// none: the buffer alone costs more than a count gains (one-shot ER n=437500 of
+// 3.5 M ids 2.19 ms, with lines 2.97).
 constexpr int64_t kLinesLeast = (int64_t)1 << 20;
 
 static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_begin, int32_t row_end,
-                            const uint8_t* owned, int32_t max_out, tc_graph** out) {
+                            const uint8_t* owned, DagShape shape, bool once, tc_graph** out) {
   std::unique_ptr<tc_graph> g(new tc_graph);
   g->ctx = ctx;
   g->n = dag->n_rows;
@@ -330,7 +357,7 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
   g->row_end = row_end;
   g->edge_begin = dag->rowptr[row_begin];
   g->edge_end = dag->rowptr[row_end];
-  g->max_out = max_out;
+  g->max_out = shape.max_out;
   g->nv_max = tck::partner_rows_max(g->n, g->nnz);
   auto cleanup = [&]() {
     dev_free(g->rp);
@@ -356,7 +383,8 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
   }
   // The bitmap kernels' codes, which a count can do without: none where there
   // is no memory for them.
-  bool big = max_out >= kCodesMinOut && tck::big_codes_fit(g->n, g->nnz);
+  bool big = shape.max_out >= kCodesMinOut && tck::big_codes_fit(g->n, g->nnz) &&
+             (!once || once_repays_codes(g->n, g->nnz, shape.squares));
   if (big || (g->n <= tck::kCoreIds && g->nnz < tck::kCorePool)) {
     st = dev_alloc((void**)&g->c16, tck::code_bytes(g->nnz), "id codes");
     if (st == TC_OK && big) st = dev_alloc((void**)&g->closed, (size_t)g->n, "closed rows");
@@ -366,7 +394,8 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
     st = TC_OK;
   }
   tck::RadixGeom geom;
-  if (g->n > tck::kCoreIds && max_out < kCodesMinOut && g->nnz >= kLinesLeast && tck::radix_geom((int64_t)g->n + 1, g->nnz, geom) &&
+  if (!once && g->n > tck::kCoreIds && shape.max_out < kCodesMinOut && g->nnz >= kLinesLeast &&
+      tck::radix_geom((int64_t)g->n + 1, g->nnz, geom) &&
       dev_alloc((void**)&g->lines, tck::line_bytes(g->nnz), "lists on lines") != TC_OK)
     g->lines = nullptr;
   const tck::GraphDesc d{0, 0, 0, 0, 0, g->n, g->nv_max, row_begin, row_end, 0};
@@ -559,12 +588,12 @@ tc_status tc_device_name(tc_ctx* ctx, char* buf, int32_t len) try {
 
 tc_status tc_graph_upload(tc_ctx* ctx, const tc_csr_view* dag, uint32_t check, tc_graph** out) try {
   if (!ctx || !out) return fail(TC_EINVAL, "null argument");
-  int32_t max_out = 0;
-  tc_status st = check_dag(dag, check, &max_out);
+  DagShape shape;
+  tc_status st = check_dag(dag, check, &shape);
   if (st != TC_OK) return st;
   std::lock_guard<std::recursive_mutex> lk(ctx->mu);
   DeviceGuard guard(ctx->device);
-  return upload_csr(ctx, dag, 0, dag->n_rows, nullptr, max_out, out);
+  return upload_csr(ctx, dag, 0, dag->n_rows, nullptr, shape, (check & TC_UPLOAD_ONCE) != 0, out);
 } catch (...) {
   return tcr::caught();
 }
@@ -572,12 +601,12 @@ tc_status tc_graph_upload(tc_ctx* ctx, const tc_csr_view* dag, uint32_t check, t
 tc_status tc_graph_upload_rows(tc_ctx* ctx, const tc_csr_view* dag, const uint8_t* owned, uint32_t check,
                                tc_graph** out) try {
   if (!ctx || !out) return fail(TC_EINVAL, "null argument");
-  int32_t max_out = 0;
-  tc_status st = check_dag(dag, check, &max_out);
+  DagShape shape;
+  tc_status st = check_dag(dag, check, &shape);
   if (st != TC_OK) return st;
   std::lock_guard<std::recursive_mutex> lk(ctx->mu);
   DeviceGuard guard(ctx->device);
-  return upload_csr(ctx, dag, 0, dag->n_rows, owned, max_out, out);
+  return upload_csr(ctx, dag, 0, dag->n_rows, owned, shape, (check & TC_UPLOAD_ONCE) != 0, out);
 } catch (...) {
   return tcr::caught();
 }
@@ -590,12 +619,12 @@ tc_status tc_partition_upload(tc_ctx* ctx, const tch_partition_view* part, uint3
   if (st != TC_OK) return fail(st, tch_last_error());
   tc_csr_view v;
   tch_csr_view(full, &v);
-  int32_t max_out = 0;
-  st = check_dag(&v, check, &max_out);
+  DagShape shape;
+  st = check_dag(&v, check, &shape);
   if (st == TC_OK) {
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     DeviceGuard guard(ctx->device);
-    st = upload_csr(ctx, &v, part->row_begin, part->row_end, nullptr, max_out, out);
+    st = upload_csr(ctx, &v, part->row_begin, part->row_end, nullptr, shape, (check & TC_UPLOAD_ONCE) != 0, out);
   }
   tch_csr_free(full);
   return st;
@@ -841,11 +870,11 @@ tc_status tc_count(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_stats* stats) t
 tc_status tc_count_csr(tc_ctx* ctx, const tc_csr_view* dag, uint32_t check, uint64_t* total, tc_stats* stats) try {
   if (!ctx || !total) return fail(TC_EINVAL, "null argument");
   if (!dag) return fail(TC_EINVAL, "null csr view");
-  int32_t max_out = 0;
+  DagShape shape;
   tc_status st;
   auto whole = [&]() {  // upload + tc_count + free
     tc_graph* g = nullptr;
-    tc_status s2 = upload_csr(ctx, dag, 0, dag->n_rows, nullptr, max_out, &g);
+    tc_status s2 = upload_csr(ctx, dag, 0, dag->n_rows, nullptr, shape, true, &g);
     if (s2 != TC_OK) return s2;
     s2 = tc_count(ctx, g, total, stats);
     tc_graph_free(ctx, g);
@@ -861,12 +890,12 @@ tc_status tc_count_csr(tc_ctx* ctx, const tc_csr_view* dag, uint32_t check, uint
   const bool small = dag->n_rows >= 0 && dag->nnz >= 0 && dag->nnz <= tcr::kPlainMaxIds && dag->rowptr &&
                      (dag->nnz == 0 || dag->colidx);
   if (!small) {
-    st = check_dag(dag, check, &max_out);
+    st = check_dag(dag, check, &shape);
     if (st != TC_OK) return st;
   }
   std::lock_guard<std::recursive_mutex> lk(ctx->mu);
   DeviceGuard guard(ctx->device);
-  if (!small && !tcr::plain_fits(dag->n_rows, dag->nnz, max_out)) return whole();
+  if (!small && !tcr::plain_fits(dag->n_rows, dag->nnz, shape.max_out)) return whole();
   const size_t rp_bytes = sizeof(int64_t) * ((size_t)dag->n_rows + 1);
   const size_t ci_off = (rp_bytes + 255) & ~(size_t)255;
   const size_t bytes = ci_off + sizeof(int32_t) * (size_t)(dag->nnz + tck::kCiPad);
@@ -888,8 +917,8 @@ tc_status tc_count_csr(tc_ctx* ctx, const tc_csr_view* dag, uint32_t check, uint
     return fail(TC_EDEVICE, std::string("one-shot copy: ") + hipGetErrorString(ce));
   }
   if (small) {
-    st = check_dag(dag, check, &max_out);
-    if (st != TC_OK || !tcr::plain_fits(dag->n_rows, dag->nnz, max_out)) {
+    st = check_dag(dag, check, &shape);
+    if (st != TC_OK || !tcr::plain_fits(dag->n_rows, dag->nnz, shape.max_out)) {
       TC_HIP_TRY(hipStreamSynchronize(s));  // the copies read the caller's arrays
       return st != TC_OK ? st : whole();
     }
@@ -903,7 +932,7 @@ tc_status tc_count_csr(tc_ctx* ctx, const tc_csr_view* dag, uint32_t check, uint
   g.row_begin = 0;
   g.row_end = dag->n_rows;
   g.edge_end = dag->nnz;
-  g.max_out = max_out;
+  g.max_out = shape.max_out;
   return tcr::plain_count(ctx, &g, ctx->plain_out, total, stats, true);
 } catch (...) {
   return tcr::caught();

@@ -79,7 +79,8 @@ tc_status tc_device_name(tc_ctx* ctx, char* buf, int32_t len);
 /* ---- graphs on the device ----------------------------------------------
  * Replaces GraphGPU::init (successful_push_pull/graph_gpu.h:84-137: device
  * rowptr/colidx + H2D).  `dag` must be the oriented DAG (tch_orient);
- * `check` (TC_CHECK_*) validates it on the host first. */
+ * `check` (TC_CHECK_*) validates it on the host first; with TC_UPLOAD_ONCE
+ * the upload leaves out what repays only over several counts. */
 tc_status tc_graph_upload(tc_ctx* ctx, const tc_csr_view* dag, uint32_t check, tc_graph** out);
 /* Same, counting only the rows u with owned[u] != 0 (n_rows bytes, copied):
  * a PE's share when its rows are an arbitrary vertex set, as with METIS

@@ -325,7 +325,7 @@ class Device {
   // Count only the rows u of `g` with owned[u] != 0 (tc_graph_upload_rows).
   AccType count_rows(const Graph& g, const uint8_t* owned, tc_stats* st = nullptr) {
     tc_graph* dg = nullptr;
-    dev_check(tc_graph_upload_rows(ctx_, &g.view(), owned, TC_CHECK_SHAPE, &dg));
+    dev_check(tc_graph_upload_rows(ctx_, &g.view(), owned, TC_CHECK_SHAPE | TC_UPLOAD_ONCE, &dg));
     uint64_t total = 0;
     tc_status s = tc_count(ctx_, dg, &total, st);
     tc_graph_free(ctx_, dg);
@@ -355,7 +355,7 @@ class Device {
       lo.part_counts = part_counts->data();
     }
     tc_graph* dg = nullptr;
-    dev_check(tc_graph_upload(ctx_, &g.view(), TC_CHECK_SHAPE, &dg));
+    dev_check(tc_graph_upload(ctx_, &g.view(), TC_CHECK_SHAPE | TC_UPLOAD_ONCE, &dg));
     uint64_t total = 0;
     tc_status s = tc_count_local(ctx_, dg, &total, &lo, nullptr);
     tc_graph_free(ctx_, dg);

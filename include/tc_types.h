@@ -49,6 +49,9 @@ typedef struct tc_csr_view {
 #define TC_CHECK_SORTED  2u  /* every row strictly increasing (sorted, no duplicates) */
 #define TC_CHECK_NOSELF  4u  /* no self-loops                                         */
 #define TC_CHECK_ALL     7u
+/* With the checks of an upload, a hint: the graph is counted once and freed.
+ * What repays only over several counts is then not prepared. */
+#define TC_UPLOAD_ONCE   8u
 
 #ifdef __cplusplus
 }

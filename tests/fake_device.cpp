@@ -1,0 +1,193 @@
+// A stand-in for the GPU behind the device library's host code: device memory
+// is host memory under a budget, copies are memcpy, streams run at once, and
+// the kernel launches do nothing but note what they were given.  Linked with
+// csrc/hip's .cpp files, so that their allocation order, fallbacks and routes
+// can be tested on the CPU.  Counts are 0 throughout.
+//
+//   fake_device SCENARIO [arguments]   exits 0 when the scenario holds
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <mutex>
+#include <thread>
+
+#include "tc_internal.hpp"
+
+// ---- device memory -----------------------------------------------------------
+static std::mutex g_mu;
+static std::map<void*, size_t> g_size;
+static size_t g_used = 0, g_peak = 0, g_budget = ~(size_t)0;
+static int g_allocs = 0;
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  if (g_used + n > g_budget) return hipErrorOutOfMemory;
+  *p = std::calloc(1, n + 64);
+  g_size[*p] = n;
+  g_used += n;
+  g_peak = std::max(g_peak, g_used);
+  ++g_allocs;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  auto it = g_size.find(p);
+  if (it == g_size.end()) std::abort();  // freed twice, or never allocated
+  g_used -= it->second;
+  g_size.erase(it);
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return (*p = std::calloc(1, n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostFree(void* p) { return std::free(p), hipSuccess; }
+hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) { return *d = h, hipSuccess; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return std::memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) { return std::memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemset(void* d, int v, size_t n) { return std::memset(d, v, n), hipSuccess; }
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return std::memset(d, v, n), hipSuccess; }
+// ---- streams, events, graphs, devices ------------------------------------------
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = (hipStream_t)std::malloc(1), hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { return std::free(s), hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return *e = (hipEvent_t)std::malloc(1), hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t e) { return std::free(e), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 0, hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { return *g = (hipGraph_t)std::malloc(1), hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t* x, hipGraph_t, hipGraphNode_t*, char*, size_t) { return *x = (hipGraphExec_t)std::malloc(1), hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t x) { return std::free(x), hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t g) { return std::free(g), hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) { return std::memset(p, 0, sizeof *p), p->multiProcessorCount = 256, hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
+}
+
+// ---- launches -----------------------------------------------------------------
+static tck::BuildBufs g_build;           // of the last partner build
+static unsigned long long g_closed = 0;  // what launch_big_codes reports
+static int g_big_codes = 0;              // its launches
+static tck::LaunchArgs g_args;           // of the last count
+namespace tck {
+int64_t scan_partials(int64_t n) { return n / 1024 + 2; }
+int64_t big_codes_bytes(int64_t n, int64_t m) { return 12 * n + 2 * m; }
+hipError_t launch_big_codes(const int64_t*, const int32_t*, int64_t, int64_t, char*, uint16_t*, uint8_t*, uint8_t*,
+                            unsigned long long* closed, int, hipStream_t) {
+  return *closed = g_closed, ++g_big_codes, hipSuccess;
+}
+hipError_t launch_partners(const LaunchArgs&, int64_t, int64_t, const BuildBufs& b, hipStream_t) { return g_build = b, hipSuccess; }
+hipError_t launch_zero(void* p, int64_t n, hipStream_t) { return std::memset(p, 0, 4 * (size_t)n), hipSuccess; }
+hipError_t launch_stage_copy(const StageCopy*, int32_t, int64_t, hipStream_t) { return hipSuccess; }
+hipError_t launch_rearm(uint32_t*, uint64_t*, int32_t, hipStream_t) { return hipSuccess; }
+hipError_t launch_finish(uint32_t*, uint64_t*, uint64_t* host, hipStream_t) { return host[0] = host[1] = 0, hipSuccess; }
+hipError_t launch_plan(const LaunchArgs& a, hipStream_t) { return g_args = a, hipSuccess; }
+hipError_t launch_count(const LaunchArgs& a, int, int, hipStream_t) { return g_args = a, hipSuccess; }
+bool part_empty(const LaunchArgs&, int, const int64_t*) { return false; }
+hipError_t launch_count_part(const LaunchArgs& a, int, int, int, const int64_t*, hipStream_t) { return g_args = a, hipSuccess; }
+hipError_t launch_plain(const int64_t*, const int32_t*, int32_t, int32_t, const uint8_t*, uint64_t*, int, hipStream_t, uint64_t*) { return hipSuccess; }
+hipError_t launch_count_local(const LaunchArgs& a, int, int, hipStream_t) { return g_args = a, hipSuccess; }
+hipError_t launch_local_prep(const int64_t*, int64_t, int32_t*, hipStream_t) { return hipSuccess; }
+hipError_t launch_local_parts(const int32_t*, const int32_t*, int64_t, int64_t, int64_t, const uint32_t*, const int32_t*, int32_t, unsigned long long*, int, hipStream_t) { return hipSuccess; }
+hipError_t launch_copy(const void*, void*, int64_t, int, hipStream_t) { return hipSuccess; }
+hipError_t launch_read(const void*, int64_t, uint32_t*, int, hipStream_t) { return hipSuccess; }
+int count_blocks_per_cu() { return 4; }
+int plain_blocks_per_cu() { return 4; }
+hipError_t noalloc_scratch_address(void** p) { return *p = nullptr, hipSuccess; }
+PlanBufs noalloc_plan_bufs(void*) { return PlanBufs{}; }
+}  // namespace tck
+
+// ---- graphs ---------------------------------------------------------------------
+struct Dag {
+  std::vector<int64_t> rp;
+  std::vector<int32_t> ci;
+  tc_csr_view view() const { return tc_csr_view{rp.data(), ci.data(), (int32_t)rp.size() - 1, (int64_t)ci.size()}; }
+};
+// n rows; the first `rows` have `d` ids each.
+static Dag make(int32_t n, int32_t rows, int32_t d) {
+  Dag g;
+  g.rp.assign((size_t)n + 1, 0);
+  for (int32_t v = 0; v < n; ++v) {
+    if (v < rows)
+      for (int32_t k = 0; k < d; ++k) g.ci.push_back(n - d + k);
+    g.rp[(size_t)v + 1] = (int64_t)g.ci.size();
+  }
+  return g;
+}
+
+#define CHECK(x)                                                              \
+  do {                                                                        \
+    if (!(x)) {                                                               \
+      std::printf("line %d: %s (%s)\n", __LINE__, #x, tc_last_error(nullptr)); \
+      std::exit(1);                                                           \
+    }                                                                         \
+  } while (0)
+
+struct Ctx {
+  tc_ctx* c = nullptr;
+  Ctx() { CHECK(tc_ctx_create(0, &c) == TC_OK); }
+  ~Ctx() { tc_ctx_destroy(c); }
+  operator tc_ctx*() const { return c; }
+};
+
+// ---- scenarios --------------------------------------------------------------------
+
+// A graph counted once gets no lines, and codes only where one count repays
+// them; a resident graph gets both.
+static void one_shot(int, char**) {
+  Ctx ctx;
+  uint64_t total;
+  const Dag flat = make(140000, 139000, 17), skewed = make(140000, 20000, 120), heavy = make(140000, 6000, 2000);
+  g_closed = ~0ull >> 3;
+  auto once = [&](const Dag& g) {
+    const tc_csr_view v = g.view();
+    g_big_codes = 0;
+    CHECK(tc_count_csr(ctx, &v, TC_CHECK_SHAPE, &total, nullptr) == TC_OK);
+    return g_big_codes;
+  };
+  CHECK(once(flat) == 0 && !g_build.lines && !g_build.codes && !g_args.c16);
+  CHECK(once(skewed) == 0 && !g_build.lines && !g_args.c16 && g_args.core == 0);
+  CHECK(once(heavy) == 1 && g_args.c16 && g_args.core == 2);
+  const Dag few = make(60000, 50000, 70);  // every id has a code: written on the way, in one shot too
+  CHECK(once(few) == 0 && g_build.codes && g_args.core == 1);
+  for (uint32_t hint : {0u, (uint32_t)TC_UPLOAD_ONCE}) {
+    const std::vector<uint8_t> owned(140000, 1);
+    for (int kind = 0; kind < 2; ++kind) {
+      auto upload = [&](const Dag& g, tc_graph** dg) {
+        const tc_csr_view v = g.view();
+        return kind ? tc_graph_upload_rows(ctx, &v, owned.data(), TC_CHECK_SHAPE | hint, dg)
+                    : tc_graph_upload(ctx, &v, TC_CHECK_SHAPE | hint, dg);
+      };
+      tc_graph* dg = nullptr;
+      CHECK(upload(flat, &dg) == TC_OK && (g_build.lines != nullptr) == (hint == 0));
+      tc_graph_free(ctx, dg);
+      g_big_codes = 0;
+      CHECK(upload(skewed, &dg) == TC_OK && g_big_codes == (hint ? 0 : 1));
+      tc_graph_free(ctx, dg);
+      CHECK(upload(heavy, &dg) == TC_OK && g_build.closed);
+      tc_graph_free(ctx, dg);
+    }
+  }
+}
+
+int main(int argc, char** argv) {
+  static const std::map<std::string, std::function<void(int, char**)>> all = {
+      {"one_shot", one_shot},
+  };
+  const auto it = argc > 1 ? all.find(argv[1]) : all.end();
+  if (it == all.end()) return 2;
+  it->second(argc - 2, argv + 2);
+  if (!g_size.empty()) return std::printf("%zu device allocations never freed\n", g_size.size()), 1;
+  return 0;
+}
