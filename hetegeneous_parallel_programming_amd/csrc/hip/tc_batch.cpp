@@ -12,7 +12,7 @@
 
 using namespace tcr;
 
-struct tc_batch {
+struct tc_batch final : tcr::Spare {
   tc_ctx* ctx = nullptr;
   int32_t n = 0;
   int64_t* rp = nullptr;
@@ -35,11 +35,20 @@ struct tc_batch {
   tc_tune captured{};
   int64_t bytes = 0;
 
-  void release() {
+  void drop_graph() {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
     exec = nullptr;
     graph = nullptr;
+  }
+  void shed() override {  // the next count captures again
+    drop_graph();
+    dev_free(c16);
+    c16 = nullptr;
+    bytes -= (int64_t)tck::code_bytes(cio);
+  }
+  void release() {
+    drop_graph();
     dev_free(rp);
     dev_free(ci);
     dev_free(c16);
@@ -52,10 +61,7 @@ struct tc_batch {
 };
 
 static tc_status capture(tc_ctx* ctx, tc_batch* b) {
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
-  b->exec = nullptr;
-  b->graph = nullptr;
+  b->drop_graph();
   tck::LaunchArgs a{};
   a.descs = b->d_descs;
   a.ngraphs = b->n;
@@ -106,24 +112,8 @@ static tc_status capture(tc_ctx* ctx, tc_batch* b) {
   return TC_OK;
 }
 
-extern "C" {
-
-tc_status tc_batch_create(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_graphs, uint32_t check,
-                          tc_batch** out) try {
-  if (!ctx || !out || n_graphs < 0 || (n_graphs > 0 && !dags)) return fail(TC_EINVAL, "bad arguments");
-  for (int32_t i = 0; i < n_graphs; ++i) {
-    const tc_csr_view& d = dags[i];
-    tc_status st = tch_validate(&d, check | TC_CHECK_SHAPE);
-    if (st != TC_OK) return fail(st, "graph " + std::to_string(i) + ": " + tch_last_error());
-    for (int64_t v = 0; v < d.n_rows; ++v)
-      if ((d.rowptr[v + 1] - d.rowptr[v]) * 64 >= ((int64_t)1 << 31))
-        return fail(TC_ERANGE, "graph " + std::to_string(i) + ": DAG out-degree too large");
-  }
-  int64_t tot_slots = 0;
-  for (int32_t i = 0; i < n_graphs; ++i) tot_slots += (int64_t)tck::partner_rows_max(dags[i].n_rows, dags[i].nnz) + 1;
-  if (tot_slots >= ((int64_t)1 << 31)) return fail(TC_ERANGE, "batch has 2^31 or more pivots");
-  std::lock_guard<std::recursive_mutex> lk(ctx->mu);
-  DeviceGuard guard(ctx->device);
+// tc_batch_create after its checks, with ctx->mu held.
+static tc_status build_batch(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_graphs, tc_batch** out) {
   std::unique_ptr<tc_batch> b(new tc_batch);
   b->ctx = ctx;
   b->n = n_graphs;
@@ -154,8 +144,6 @@ tc_status tc_batch_create(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_graphs
     b->release();
     return st;
   }
-  // the bitmap kernels' codes, which a count can do without
-  if (coded && dev_alloc((void**)&b->c16, tck::code_bytes(cio), "batch id codes") != TC_OK) b->c16 = nullptr;
   hipError_t e = hipHostMalloc((void**)&b->pinned, sizeof(uint64_t) * ((size_t)n_graphs + 16), hipHostMallocDefault);
   if (e != hipSuccess) {
     b->pinned = nullptr;
@@ -276,6 +264,10 @@ tc_status tc_batch_create(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_graphs
     BuildScratch bs;
     e = hipMemcpy(d_seg, rebased.data(), sizeof(tck::GraphDesc) * (size_t)n_graphs, hipMemcpyHostToDevice);
     if (e == hipSuccess) st = bs.ensure(max_rows, max_ids);  // once: the segments reuse it in stream order
+    // the bitmap kernels' codes, which a count can do without: taken last
+    if (coded && e == hipSuccess && st == TC_OK &&
+        dev_alloc((void**)&b->c16, tck::code_bytes(cio), "batch id codes") != TC_OK)
+      b->c16 = nullptr;
     if (e == hipSuccess && st == TC_OK) e = hipEventRecord(ctx->ev[0], ctx->stream);
     for (const Seg& sg : segs) {
       if (e != hipSuccess || st != TC_OK) break;
@@ -316,8 +308,36 @@ tc_status tc_batch_create(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_graphs
   }
   b->bytes = sizeof(int64_t) * rpo + sizeof(int32_t) * cio + (int64_t)sizeof(tck::GraphDesc) * n_graphs +
              b->partners.bytes + PlanScratch::bytes_for(b->P) + 8 * (int64_t)n_graphs + (b->c16 ? (int64_t)tck::code_bytes(cio) : 0);
+  if (b->c16) {
+    try {
+      ctx->spares.insert(b.get());
+    } catch (...) {
+      b->shed();
+    }
+  }
   *out = b.release();
   return TC_OK;
+}
+
+extern "C" {
+
+tc_status tc_batch_create(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_graphs, uint32_t check,
+                          tc_batch** out) try {
+  if (!ctx || !out || n_graphs < 0 || (n_graphs > 0 && !dags)) return fail(TC_EINVAL, "bad arguments");
+  for (int32_t i = 0; i < n_graphs; ++i) {
+    const tc_csr_view& d = dags[i];
+    tc_status st = tch_validate(&d, check | TC_CHECK_SHAPE);
+    if (st != TC_OK) return fail(st, "graph " + std::to_string(i) + ": " + tch_last_error());
+    for (int64_t v = 0; v < d.n_rows; ++v)
+      if ((d.rowptr[v + 1] - d.rowptr[v]) * 64 >= ((int64_t)1 << 31))
+        return fail(TC_ERANGE, "graph " + std::to_string(i) + ": DAG out-degree too large");
+  }
+  int64_t tot_slots = 0;
+  for (int32_t i = 0; i < n_graphs; ++i) tot_slots += (int64_t)tck::partner_rows_max(dags[i].n_rows, dags[i].nnz) + 1;
+  if (tot_slots >= ((int64_t)1 << 31)) return fail(TC_ERANGE, "batch has 2^31 or more pivots");
+  std::lock_guard<std::recursive_mutex> lk(ctx->mu);
+  DeviceGuard guard(ctx->device);
+  return with_room(ctx, [&] { return build_batch(ctx, dags, n_graphs, out); });
 } catch (...) {
   return tcr::caught();
 }
@@ -396,6 +416,7 @@ tc_status tc_batch_free(tc_ctx* ctx, tc_batch* b) try {
   std::lock_guard<std::recursive_mutex> lk(b->ctx->mu);
   DeviceGuard guard(b->ctx->device);
   (void)hipStreamSynchronize(b->ctx->stream);
+  b->ctx->spares.erase(b);
   b->release();
   delete b;
   return TC_OK;

@@ -8,6 +8,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <unordered_set>
 #include <vector>
 
 #include "tc.h"
@@ -155,6 +156,26 @@ tck::Tune to_kernel_tune(const tc_tune& t);
 tc_status check_tune(const tc_tune& t);
 tc_tune default_tune();
 
+// A graph or a batch that holds device memory its counts can do without: the
+// 16-bit codes and the lists on lines.  Such memory is taken last, and when a
+// context runs out it gives all of it back and tries again, so that it never
+// takes the place of what a call needs.
+struct Spare {
+  // Gives it back; the context's streams are idle.
+  virtual void shed() = 0;
+
+ protected:
+  ~Spare() = default;
+};
+bool shed_spares(tc_ctx* ctx);  // all of ctx's; whether there were any
+// f's status; when f ran out of memory and spares could be shed, that of
+// another try.  f leaves nothing behind when it fails.
+template <class F>
+tc_status with_room(tc_ctx* ctx, F f) {
+  const tc_status st = f();
+  return st == TC_ENOMEM && shed_spares(ctx) ? f() : st;
+}
+
 }  // namespace tcr
 
 struct tc_ctx {
@@ -176,6 +197,7 @@ struct tc_ctx {
   std::string name;
   tcr::PlanScratch scratch;
   tcr::Stager stager;
+  std::unordered_set<tcr::Spare*> spares;  // the graphs and batches that hold any
   uint64_t* pinned = nullptr;  // 64 B count + 64 B bin counters
   uint64_t* pinned_dev = nullptr;  // its device address
   void* noalloc = nullptr;     // device address of the static scratch of tc_count_noalloc
@@ -190,7 +212,7 @@ struct tc_ctx {
   int grid() const { return tune.grid > 0 ? tune.grid : count_grid; }
 };
 
-struct tc_graph {
+struct tc_graph final : tcr::Spare {
   tc_ctx* ctx = nullptr;
   int64_t* rp = nullptr;
   int32_t* ci = nullptr;
@@ -204,12 +226,21 @@ struct tc_graph {
   uint8_t* closed = nullptr;  // with c16, over kCoreIds rows: tck::BuildBufs::closed
   uint8_t* part = nullptr;    // with closed: tck::BuildBufs::lpart
   bool coded = false;         // whether enough edges can use the codes
+  int64_t spare_bytes = 0;    // of those four
   void drop_codes() {
     tcr::dev_free(c16);
     tcr::dev_free(closed);
     tcr::dev_free(part);
     c16 = nullptr;
     closed = part = nullptr;
+    coded = false;
+  }
+  void shed() override {
+    drop_codes();
+    tcr::dev_free(lines);
+    lines = nullptr;
+    bytes -= spare_bytes;
+    spare_bytes = 0;
   }
   int32_t* pown = nullptr;  // [nv_max + 1] owner vertex of each partner row, written by every build
   int32_t max_out = 0;

@@ -61,6 +61,15 @@ void dev_free(void* p) {
   if (p) (void)hipFree(p);
 }
 
+bool shed_spares(tc_ctx* ctx) {
+  std::lock_guard<std::recursive_mutex> lk(ctx->mu);
+  if (ctx->spares.empty()) return false;
+  (void)hipStreamSynchronize(ctx->stream);
+  for (Spare* x : ctx->spares) x->shed();
+  ctx->spares.clear();
+  return true;
+}
+
 tc_status PlanScratch::ensure(int64_t pivots, int64_t nouts) {
   if (!counters) {
     tc_status st = dev_alloc((void**)&counters, sizeof(uint32_t) * tck::kNumCounters, "plan counters");
@@ -347,8 +356,8 @@ static bool once_repays_codes(int64_t n, int64_t nnz, uint64_t squares) {
 // 3.5 M ids 2.19 ms, with lines 2.97).
 constexpr int64_t kLinesLeast = (int64_t)1 << 20;
 
-static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_begin, int32_t row_end,
-                            const uint8_t* owned, DagShape shape, bool once, tc_graph** out) {
+static tc_status build_graph(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_begin, int32_t row_end,
+                             const uint8_t* owned, DagShape shape, bool once, tc_graph** out) {
   std::unique_ptr<tc_graph> g(new tc_graph);
   g->ctx = ctx;
   g->n = dag->n_rows;
@@ -381,23 +390,6 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
     cleanup();
     return st;
   }
-  // The bitmap kernels' codes, which a count can do without: none where there
-  // is no memory for them.
-  bool big = shape.max_out >= kCodesMinOut && tck::big_codes_fit(g->n, g->nnz) &&
-             (!once || once_repays_codes(g->n, g->nnz, shape.squares));
-  if (big || (g->n <= tck::kCoreIds && g->nnz < tck::kCorePool)) {
-    st = dev_alloc((void**)&g->c16, tck::code_bytes(g->nnz), "id codes");
-    if (st == TC_OK && big) st = dev_alloc((void**)&g->closed, (size_t)g->n, "closed rows");
-    if (st == TC_OK && big) st = dev_alloc((void**)&g->part, (size_t)g->nnz, "code parts");
-    if (st != TC_OK) g->drop_codes();
-    big = big && st == TC_OK;
-    st = TC_OK;
-  }
-  tck::RadixGeom geom;
-  if (!once && g->n > tck::kCoreIds && shape.max_out < kCodesMinOut && g->nnz >= kLinesLeast &&
-      tck::radix_geom((int64_t)g->n + 1, g->nnz, geom) &&
-      dev_alloc((void**)&g->lines, tck::line_bytes(g->nnz), "lists on lines") != TC_OK)
-    g->lines = nullptr;
   const tck::GraphDesc d{0, 0, 0, 0, 0, g->n, g->nv_max, row_begin, row_end, 0};
   hipError_t e = hipMemcpy(g->rp, dag->rowptr, sizeof(int64_t) * ((size_t)g->n + 1), hipMemcpyHostToDevice);
   if (e == hipSuccess && g->nnz > 0)
@@ -421,14 +413,28 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
   hipStream_t s = ctx->stream;
   // the scratch is allocated before the timed span: build_ms is the device's build
   st = bs.ensure((int64_t)g->n + 1, g->nnz);
-  if (big && tck::big_codes_bytes(g->n, g->nnz) > bs.cap) {
-    g->drop_codes();
-    big = false;
-  }
   if (st != TC_OK) {
     cleanup();
     return st;
   }
+  // The bitmap kernels' codes and the lists on lines, which a count can do
+  // without: taken last, none where there is no memory for them.
+  bool big = shape.max_out >= kCodesMinOut && tck::big_codes_fit(g->n, g->nnz) &&
+             (!once || once_repays_codes(g->n, g->nnz, shape.squares)) &&
+             tck::big_codes_bytes(g->n, g->nnz) <= bs.cap;
+  if (big || (g->n <= tck::kCoreIds && g->nnz < tck::kCorePool)) {
+    st = dev_alloc((void**)&g->c16, tck::code_bytes(g->nnz), "id codes");
+    if (st == TC_OK && big) st = dev_alloc((void**)&g->closed, (size_t)g->n, "closed rows");
+    if (st == TC_OK && big) st = dev_alloc((void**)&g->part, (size_t)g->nnz, "code parts");
+    if (st != TC_OK) g->drop_codes();
+    big = big && st == TC_OK;
+    st = TC_OK;
+  }
+  tck::RadixGeom geom;
+  if (!once && g->n > tck::kCoreIds && shape.max_out < kCodesMinOut && g->nnz >= kLinesLeast &&
+      tck::radix_geom((int64_t)g->n + 1, g->nnz, geom) &&
+      dev_alloc((void**)&g->lines, tck::line_bytes(g->nnz), "lists on lines") != TC_OK)
+    g->lines = nullptr;
   e = hipEventRecord(ctx->ev[0], s);
   if (e == hipSuccess) {
     a.core_kb = tck::core_bits(g->n);
@@ -455,12 +461,24 @@ static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_beg
   g->build_ms = ms;
   g->nv = *(const int32_t*)ctx->pinned;
   g->coded = big ? 4 * (int64_t)ctx->pinned[1] >= g->nnz : g->c16 != nullptr;
+  g->spare_bytes = (g->lines ? (int64_t)tck::line_bytes(g->nnz) : 0) + (g->c16 ? (int64_t)tck::code_bytes(g->nnz) : 0) +
+                   (big ? (int64_t)g->n + g->nnz : 0);
   g->bytes = sizeof(int64_t) * ((int64_t)g->n + 1) + sizeof(int32_t) * g->nnz + sizeof(tck::GraphDesc) +
-             g->partners.bytes + (owned ? (int64_t)g->n : 0) +
-             (g->lines ? (int64_t)tck::line_bytes(g->nnz) : 0) + (g->c16 ? (int64_t)tck::code_bytes(g->nnz) : 0) +
-             (big ? (int64_t)g->n + g->nnz : 0) + sizeof(int32_t) * ((int64_t)g->nv_max + 1);
+             g->partners.bytes + (owned ? (int64_t)g->n : 0) + g->spare_bytes + sizeof(int32_t) * ((int64_t)g->nv_max + 1);
+  if (g->spare_bytes) {
+    try {
+      ctx->spares.insert(g.get());
+    } catch (...) {
+      g->shed();
+    }
+  }
   *out = g.release();
   return TC_OK;
+}
+
+static tc_status upload_csr(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_begin, int32_t row_end,
+                            const uint8_t* owned, DagShape shape, bool once, tc_graph** out) {
+  return with_room(ctx, [&] { return build_graph(ctx, dag, row_begin, row_end, owned, shape, once, out); });
 }
 
 // plan_ms = ev[0] -> ev[plan_end]; count_ms = ev[1] -> ev[2].
@@ -639,6 +657,7 @@ tc_status tc_graph_free(tc_ctx* ctx, tc_graph* g) try {
   std::lock_guard<std::recursive_mutex> lk(c->mu);
   DeviceGuard guard(c->device);
   (void)hipStreamSynchronize(c->stream);
+  c->spares.erase(g);
   dev_free(g->rp);
   dev_free(g->ci);
   g->drop_codes();
@@ -781,7 +800,7 @@ static tc_status count_binned(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_stat
   const bool kept = g->plan_valid && std::memcmp(&g->plan_tune, &ctx->tune, sizeof(tc_tune)) == 0;
   if (!kept) {
     const int64_t had = g->plan.cap;
-    tc_status st = g->plan.ensure(P, tck::kOutWords);
+    tc_status st = with_room(ctx, [&] { return g->plan.ensure(P, tck::kOutWords); });
     if (st != TC_OK) return st;
     if (g->plan.cap != had) g->bytes += PlanScratch::bytes_for(g->plan.cap) - (had ? PlanScratch::bytes_for(had) : 0);
     g->plan_valid = false;
@@ -903,7 +922,7 @@ tc_status tc_count_csr(tc_ctx* ctx, const tc_csr_view* dag, uint32_t check, uint
     dev_free(ctx->once_dev);
     ctx->once_dev = nullptr;
     ctx->once_cap = 0;
-    st = dev_alloc((void**)&ctx->once_dev, bytes, "one-shot graph");
+    st = with_room(ctx, [&] { return dev_alloc((void**)&ctx->once_dev, bytes, "one-shot graph"); });
     if (st != TC_OK) return st;
     ctx->once_cap = bytes;
   }
@@ -1047,8 +1066,8 @@ tc_status tc_count_local(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_local* ou
   const bool vertices = out->vertex_counts != nullptr;
   const bool parts_only = k > 0 && !vertices && !out->edge_counts;
   const int mode = vertices ? tck::kLocalFull : parts_only ? tck::kLocalParts : tck::kLocalEdges;
-  tc_status st = ctx->scratch.ensure(P, tck::kOutWords);
-  if (st == TC_OK) st = parts_only ? ensure_split(g->local) : ensure_local(ctx, g);
+  tc_status st = with_room(ctx, [&] { return ctx->scratch.ensure(P, tck::kOutWords); });
+  if (st == TC_OK) st = with_room(ctx, [&] { return parts_only ? ensure_split(g->local) : ensure_local(ctx, g); });
   if (st != TC_OK) return st;
   LocalBufs& L = g->local;
   tck::LaunchArgs a = count_args(ctx, g);
@@ -1102,8 +1121,8 @@ tc_status tc_probe_copy(tc_ctx* ctx, int64_t bytes, int32_t iters, double* ms_pe
   std::lock_guard<std::recursive_mutex> lk(ctx->mu);
   DeviceGuard guard(ctx->device);
   void *src = nullptr, *dst = nullptr;
-  tc_status st = dev_alloc(&src, (size_t)bytes, "copy src");
-  if (st == TC_OK) st = dev_alloc(&dst, (size_t)bytes, "copy dst");
+  tc_status st = with_room(ctx, [&] { return dev_alloc(&src, (size_t)bytes, "copy src"); });
+  if (st == TC_OK) st = with_room(ctx, [&] { return dev_alloc(&dst, (size_t)bytes, "copy dst"); });
   if (st != TC_OK) {
     dev_free(src);
     return st;
@@ -1134,8 +1153,9 @@ tc_status tc_probe_read(tc_ctx* ctx, int64_t bytes, int32_t iters, double* ms_pe
   DeviceGuard guard(ctx->device);
   const int grid = ctx->cus * 32;
   void *src = nullptr, *sink = nullptr;
-  tc_status st = dev_alloc(&src, (size_t)bytes, "read src");
-  if (st == TC_OK) st = dev_alloc(&sink, sizeof(uint32_t) * (size_t)grid * tck::kBlock, "read sink");
+  tc_status st = with_room(ctx, [&] { return dev_alloc(&src, (size_t)bytes, "read src"); });
+  if (st == TC_OK)
+    st = with_room(ctx, [&] { return dev_alloc(&sink, sizeof(uint32_t) * (size_t)grid * tck::kBlock, "read sink"); });
   if (st != TC_OK) {
     dev_free(src);
     return st;

@@ -543,7 +543,7 @@ tc_status tc_server_create(tc_ctx* ctx, const tc_server_config* cfg, tc_server**
   s->fill_graphs = cfg->fill_graphs > 0 ? cfg->fill_graphs : kDefaultFillGraphs;
   s->fill_wait_us = cfg->fill_wait_us > 0 ? cfg->fill_wait_us : kDefaultFillWaitUs;
   DeviceGuard guard(ctx->device);
-  tc_status st = dev_alloc((void**)&s->pool, cfg->hbm_budget, "server pool");
+  tc_status st = with_room(ctx, [&] { return dev_alloc((void**)&s->pool, cfg->hbm_budget, "server pool"); });
   if (st != TC_OK) return st;
   st = tch_arena_create(cfg->hbm_budget, kAlign, &s->arena);
   if (st != TC_OK) {
@@ -586,8 +586,8 @@ tc_status tc_server_create(tc_ctx* ctx, const tc_server_config* cfg, tc_server**
       s->release();
       return fail(TC_EDEVICE, std::string("server slot: ") + hipGetErrorString(e));
     }
-    st = dev_alloc(&sl.plan, total, "slot plan scratch");
-    if (st == TC_OK) st = sl.build.ensure(R, s->max_ids);
+    st = with_room(ctx, [&] { return dev_alloc(&sl.plan, total, "slot plan scratch"); });
+    if (st == TC_OK) st = with_room(ctx, [&] { return sl.build.ensure(R, s->max_ids); });
     if (st != TC_OK) {
       s->release();
       return st;

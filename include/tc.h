@@ -113,7 +113,10 @@ typedef struct tc_graph_info {
   int64_t nnz;            /* DAG ids                                            */
   int64_t partner_rows;   /* partner rows built (units of work of the count)    */
   double build_ms;        /* device time of the partner build                   */
-  int64_t bytes;          /* device bytes held                                  */
+  int64_t bytes;          /* device bytes held; some of them (16-bit codes, a
+                             second copy of short lists) only make counts faster:
+                             a call that would run out of memory frees those of
+                             all graphs and batches of the context first        */
 } tc_graph_info;
 tc_status tc_graph_get_info(const tc_graph* g, tc_graph_info* out);
 

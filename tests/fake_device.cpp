@@ -20,17 +20,16 @@
 static std::mutex g_mu;
 static std::map<void*, size_t> g_size;
 static size_t g_used = 0, g_peak = 0, g_budget = ~(size_t)0;
-static int g_allocs = 0;
+static std::function<bool(size_t)> g_deny;  // sizes that are never to be had
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
   std::lock_guard<std::mutex> lk(g_mu);
-  if (g_used + n > g_budget) return hipErrorOutOfMemory;
+  if (g_used + n > g_budget || (g_deny && g_deny(n))) return hipErrorOutOfMemory;
   *p = std::calloc(1, n + 64);
   g_size[*p] = n;
   g_used += n;
   g_peak = std::max(g_peak, g_used);
-  ++g_allocs;
   return hipSuccess;
 }
 hipError_t hipFree(void* p) {
@@ -181,9 +180,98 @@ static void one_shot(int, char**) {
   }
 }
 
+// What a program does with one graph, at a budget of device memory; the first
+// status that is not TC_OK.
+static tc_status use_graph(const Dag& g, size_t budget, int64_t* bytes = nullptr) {
+  Ctx ctx;
+  g_budget = budget;
+  const tc_csr_view v = g.view();
+  tc_graph* dg = nullptr;
+  uint64_t total;
+  tc_status st = tc_graph_upload(ctx, &v, TC_CHECK_SHAPE, &dg);
+  for (int i = 0; i < 2 && st == TC_OK; ++i) st = tc_count_binned(ctx, dg, &total, nullptr);
+  std::vector<uint32_t> edges(g.ci.size());
+  tc_local out{};
+  out.edge_counts = edges.data();
+  if (st == TC_OK) st = tc_count_local(ctx, dg, &total, &out, nullptr);
+  if (st == TC_OK) st = tc_count_binned(ctx, dg, &total, nullptr);
+  if (bytes && dg) *bytes = tc_graph_bytes(dg);
+  tc_graph_free(ctx, dg);
+  g_budget = ~(size_t)0;
+  return st;
+}
+static tc_status use_batch(const Dag& g, size_t budget, int64_t* bytes = nullptr) {
+  Ctx ctx;
+  g_budget = budget;
+  const tc_csr_view v[2] = {g.view(), g.view()};
+  tc_batch* b = nullptr;
+  uint64_t counts[2];
+  tc_status st = tc_batch_create(ctx, v, 2, TC_CHECK_SHAPE, &b);
+  if (st == TC_OK) st = tc_batch_count(ctx, b, counts, nullptr);
+  if (bytes && b) *bytes = tc_batch_bytes(b);
+  tc_batch_free(ctx, b);
+  g_budget = ~(size_t)0;
+  return st;
+}
+
+// Codes and lines never take the place of what a call needs: whatever memory
+// holds the calls without them holds the calls.
+static void memory(int, char**) {
+  const Dag flat = make(140000, 139000, 17), skewed = make(140000, 20000, 120), few = make(60000, 50000, 70);
+  g_closed = ~0ull >> 3;
+  for (const Dag* g : {&flat, &skewed, &few})
+    for (const auto& use : {use_graph, use_batch}) {
+      const size_t n = g->rp.size() - 1, m = g->ci.size();
+      int64_t least = 0, most = 0;
+      g_peak = 0;
+      CHECK(use(*g, ~(size_t)0, &most) == TC_OK);
+      const size_t with = g_peak;
+      const bool batch = use == use_batch;
+      g_deny = [=](size_t b) {
+        return batch ? b == tck::code_bytes(2 * m) : b == tck::code_bytes(m) || b == tck::line_bytes(m) || b == n || b == m;
+      };
+      g_peak = 0;
+      CHECK(use(*g, ~(size_t)0, &least) == TC_OK);
+      const size_t without = g_peak;
+      g_deny = nullptr;
+      CHECK(most >= least && with >= without);
+      CHECK(use(*g, without - 1, nullptr) == TC_ENOMEM);
+      int64_t bytes = 0;
+      CHECK(use(*g, without, &bytes) == TC_OK && bytes == least);
+      for (int i = 1; i < 16; ++i) CHECK(use(*g, without + (with - without) * i / 16, &bytes) == TC_OK);
+      CHECK(use(*g, with, &bytes) == TC_OK && bytes == most);
+    }
+  // beside others: a graph and a batch with codes give them up for a third
+  Ctx ctx;
+  const tc_csr_view v = skewed.view(), w = few.view(), x = flat.view();
+  tc_graph *a = nullptr, *c = nullptr;
+  tc_batch* b = nullptr;
+  uint64_t total;
+  CHECK(tc_graph_upload(ctx, &v, TC_CHECK_SHAPE, &a) == TC_OK && tc_batch_create(ctx, &w, 1, TC_CHECK_SHAPE, &b) == TC_OK);
+  CHECK(tc_batch_count(ctx, b, &total, nullptr) == TC_OK);
+  const int64_t had_a = tc_graph_bytes(a), had_b = tc_batch_bytes(b);
+  g_peak = g_used;
+  CHECK(tc_graph_upload(ctx, &x, TC_CHECK_SHAPE | TC_UPLOAD_ONCE, &c) == TC_OK);
+  const size_t need = g_peak;
+  tc_graph_free(ctx, c);
+  g_budget = need;
+  CHECK(tc_graph_upload(ctx, &x, TC_CHECK_SHAPE, &c) == TC_OK && tc_graph_bytes(a) == had_a);
+  tc_graph_free(ctx, c);
+  g_budget = need - 1;
+  CHECK(tc_graph_upload(ctx, &x, TC_CHECK_SHAPE, &c) == TC_OK);
+  CHECK(tc_graph_bytes(a) < had_a && tc_batch_bytes(b) < had_b);
+  CHECK(tc_count_binned(ctx, a, &total, nullptr) == TC_OK && g_args.core == 0 && !g_args.c16);
+  CHECK(tc_batch_count(ctx, b, &total, nullptr) == TC_OK && g_args.core == 0 && !g_args.c16);
+  tc_graph_free(ctx, c);
+  tc_graph_free(ctx, a);
+  tc_batch_free(ctx, b);
+  g_budget = ~(size_t)0;
+}
+
 int main(int argc, char** argv) {
   static const std::map<std::string, std::function<void(int, char**)>> all = {
       {"one_shot", one_shot},
+      {"memory", memory},
   };
   const auto it = argc > 1 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;

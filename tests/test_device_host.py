@@ -40,3 +40,7 @@ def fake(tmp_path_factory):
 
 def test_one_shot_calls_prepare_for_one_count(fake):
     fake("one_shot")
+
+
+def test_codes_and_lines_take_no_memory_that_is_needed(fake):
+    fake("memory")
