@@ -308,6 +308,9 @@ tck::Tune to_kernel_tune(const tc_tune& t) {
 struct DagShape {
   int32_t max_out = 0;
   uint64_t squares = 0;  // sum over rows of out-degree squared: bounds the ids a count streams
+  // squares against those of lists of equal length: 1.1 to 1.3 in flat graphs
+  // (ER of mean out-degree 4 to 50), 3.5 and more in R-MAT graphs
+  double skew = 0;
 };
 static tc_status check_dag(const tc_csr_view* dag, uint32_t check, DagShape* shape) {
   if (!dag) return fail(TC_EINVAL, "null csr view");
@@ -315,45 +318,55 @@ static tc_status check_dag(const tc_csr_view* dag, uint32_t check, DagShape* sha
   if (st != TC_OK) return fail(st, tch_last_error());
   int64_t mo = 0;
   uint64_t squares = 0;  // (below 2^64 for any graph that passes)
+  int64_t lists = 0;
   for (int64_t v = 0; v < dag->n_rows; ++v) {
     const int64_t d = dag->rowptr[v + 1] - dag->rowptr[v];
     mo = std::max<int64_t>(mo, d);
     squares += (uint64_t)d * (uint64_t)d;
+    lists += d > 0;
   }
   if (mo * 64 >= ((int64_t)1 << 31))
     return fail(TC_ERANGE, "DAG out-degree too large (max_out * 64 must fit in int32)");
-  *shape = DagShape{(int32_t)mo, squares};
+  *shape = DagShape{(int32_t)mo, squares, lists ? (double)squares * (double)lists / ((double)dag->nnz * (double)dag->nnz) : 0.0};
   return TC_OK;
 }
 
-// Graphs past tck::kCoreIds rows get codes only when some list is this long:
-// flat ones have no set of 65535 vertices that most edges lead to.
+// Graphs past tck::kCoreIds rows get codes when some list is kCodesMinOut long
+// and lists are uneven.  Flat ones have no set of 65535 vertices that most
+// edges lead to, and their codes are no shorter to stream (ER n=400009 of 40 M
+// ids, lists to 180: 2.75 ms with codes, 2.44 without, 2.21 with lists on
+// lines; n=80001 of 4 M, 97% of the edges coded: 0.252, 0.212, 0.215).
 constexpr int32_t kCodesMinOut = 64;
+constexpr double kCodesSkew = 2.0;
+static bool wants_codes(const DagShape& shape) { return shape.max_out >= kCodesMinOut && shape.skew >= kCodesSkew; }
+// They are kept and counted with only when one edge in kCodedShare can use
+// them: that much repays the bitmap kernels' launches.  The line is not a sharp
+// one (without / with codes: at 43% 0.509 / 0.507 ms, at 73% 0.287 / 0.288, of
+// R-MAT n=4000000 of 8 M ids, 90%, 0.382 / 0.328); below it lie rows that are
+// not ordered by degree (a symmetric R-MAT graph: 12%).
+constexpr int64_t kCodedShare = 4;
 
 // Whether the codes of a graph past tck::kCoreIds rows repay in one count.
 // They shorten it by a share of its time, which goes with the ids it streams
 // (at most `squares`), and cost an allocation and a pass per id: so only where
-// there is much to stream, much of it per id, and by a few long lists (at
-// 4 times the squares of a graph of equal lists; flat graphs have about 1.25).
+// there is much to stream, in all and per id.
 // One-shot calls on MI355X, without / with codes, ms: R-MAT n=333333 of 8 M
 // ids (165 squares an id) 4.07 / 4.59, n=1000000 of 15 M (151) 7.05 / 7.49,
 // n=6000000 of 30 M (80) 17.4 / 18.4; n=2000000 of 30 M (179) 13.5 / 13.0,
-// n=500000 of 30 M (419) 13.4 / 11.0, n=4266666 of 64 M (218) 28.7 / 26.1; ER
-// n=1250000 of 60 M (60, lists to 86) 16.6 / 18.8.
+// n=500000 of 30 M (419) 13.4 / 11.0, n=4266666 of 64 M (218) 28.7 / 26.1.
 constexpr uint64_t kOnceSquares = (uint64_t)1 << 32, kOnceSquaresPerId = 128;
-static bool once_repays_codes(int64_t n, int64_t nnz, uint64_t squares) {
-  return squares >= kOnceSquares && squares >= kOnceSquaresPerId * (uint64_t)nnz &&
-         (double)squares * (double)n >= 4.0 * (double)nnz * (double)nnz;
+static bool once_repays_codes(int64_t nnz, uint64_t squares) {
+  return squares >= kOnceSquares && squares >= kOnceSquaresPerId * (uint64_t)nnz;
 }
 
-// Flat graphs (past tck::kCoreIds rows, no list of kCodesMinOut ids) of this
-// many ids on get their lists on lines as well: an edge's list is then read in
-// one 128-byte line instead of 1.5, and such a count is bound by the lines it
-// reads beyond L2 (ER n=2000003 d=33: 1.03 -> 0.90 ms, of a build 1.73 -> 1.81
-// ms).  With codes the other lists are few (R-MAT-22: 3.24, with lines 3.30
-// ms), and fewer ids stay in an XCD's L2 (4 MB).  A graph counted once gets
-// none: the buffer alone costs more than a count gains (one-shot ER n=437500 of
-// 3.5 M ids 2.19 ms, with lines 2.97).
+// Graphs past tck::kCoreIds rows that want no codes, of this many ids on, get
+// their lists on lines: an edge's list is then read in one 128-byte line
+// instead of 1.5, and such a count is bound by the lines it reads beyond L2 (ER
+// n=2000003 d=33: 1.03 -> 0.90 ms, of a build 1.73 -> 1.81 ms; n=1000003 d=80
+// of 40 M ids: 1.45 -> 1.25).  With codes the other lists are few (R-MAT-22:
+// 3.24, with lines 3.30 ms), and fewer ids stay in an XCD's L2 (4 MB).  A graph
+// counted once gets none: the buffer alone costs more than a count gains
+// (one-shot ER n=437500 of 3.5 M ids 2.19 ms, with lines 2.97).
 constexpr int64_t kLinesLeast = (int64_t)1 << 20;
 
 static tc_status build_graph(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_begin, int32_t row_end,
@@ -419,8 +432,8 @@ static tc_status build_graph(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_be
   }
   // The bitmap kernels' codes and the lists on lines, which a count can do
   // without: taken last, none where there is no memory for them.
-  bool big = shape.max_out >= kCodesMinOut && tck::big_codes_fit(g->n, g->nnz) &&
-             (!once || once_repays_codes(g->n, g->nnz, shape.squares)) &&
+  bool big = wants_codes(shape) && tck::big_codes_fit(g->n, g->nnz) &&
+             (!once || once_repays_codes(g->nnz, shape.squares)) &&
              tck::big_codes_bytes(g->n, g->nnz) <= bs.cap;
   if (big || (g->n <= tck::kCoreIds && g->nnz < tck::kCorePool)) {
     st = dev_alloc((void**)&g->c16, tck::code_bytes(g->nnz), "id codes");
@@ -431,7 +444,7 @@ static tc_status build_graph(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_be
     st = TC_OK;
   }
   tck::RadixGeom geom;
-  if (!once && g->n > tck::kCoreIds && shape.max_out < kCodesMinOut && g->nnz >= kLinesLeast &&
+  if (!once && g->n > tck::kCoreIds && !wants_codes(shape) && g->nnz >= kLinesLeast &&
       tck::radix_geom((int64_t)g->n + 1, g->nnz, geom) &&
       dev_alloc((void**)&g->lines, tck::line_bytes(g->nnz), "lists on lines") != TC_OK)
     g->lines = nullptr;
@@ -460,7 +473,11 @@ static tc_status build_graph(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_be
   (void)hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]);
   g->build_ms = ms;
   g->nv = *(const int32_t*)ctx->pinned;
-  g->coded = big ? 4 * (int64_t)ctx->pinned[1] >= g->nnz : g->c16 != nullptr;
+  g->coded = big ? kCodedShare * (int64_t)ctx->pinned[1] >= g->nnz : g->c16 != nullptr;
+  if (big && !g->coded) {  // no count reads them
+    g->drop_codes();
+    big = false;
+  }
   g->spare_bytes = (g->lines ? (int64_t)tck::line_bytes(g->nnz) : 0) + (g->c16 ? (int64_t)tck::code_bytes(g->nnz) : 0) +
                    (big ? (int64_t)g->n + g->nnz : 0);
   g->bytes = sizeof(int64_t) * ((int64_t)g->n + 1) + sizeof(int32_t) * g->nnz + sizeof(tck::GraphDesc) +

@@ -113,13 +113,13 @@ struct Dag {
   std::vector<int32_t> ci;
   tc_csr_view view() const { return tc_csr_view{rp.data(), ci.data(), (int32_t)rp.size() - 1, (int64_t)ci.size()}; }
 };
-// n rows; the first `rows` have `d` ids each.
-static Dag make(int32_t n, int32_t rows, int32_t d) {
+// n rows; the first `rows` have `d` ids each, the next `hubs` have `long_d`.
+static Dag make(int32_t n, int32_t rows, int32_t d, int32_t hubs = 0, int32_t long_d = 0) {
   Dag g;
   g.rp.assign((size_t)n + 1, 0);
   for (int32_t v = 0; v < n; ++v) {
-    if (v < rows)
-      for (int32_t k = 0; k < d; ++k) g.ci.push_back(n - d + k);
+    const int32_t k = v < rows ? d : v < rows + hubs ? long_d : 0;
+    for (int32_t i = 0; i < k; ++i) g.ci.push_back(n - k + i);
     g.rp[(size_t)v + 1] = (int64_t)g.ci.size();
   }
   return g;
@@ -147,7 +147,8 @@ struct Ctx {
 static void one_shot(int, char**) {
   Ctx ctx;
   uint64_t total;
-  const Dag flat = make(140000, 139000, 17), skewed = make(140000, 20000, 120), heavy = make(140000, 6000, 2000);
+  const Dag flat = make(140000, 139000, 17), skewed = make(140000, 20000, 10, 2000, 500),
+            heavy = make(140000, 40000, 20, 600, 10000);
   g_closed = ~0ull >> 3;
   auto once = [&](const Dag& g) {
     const tc_csr_view v = g.view();
@@ -217,7 +218,7 @@ static tc_status use_batch(const Dag& g, size_t budget, int64_t* bytes = nullptr
 // Codes and lines never take the place of what a call needs: whatever memory
 // holds the calls without them holds the calls.
 static void memory(int, char**) {
-  const Dag flat = make(140000, 139000, 17), skewed = make(140000, 20000, 120), few = make(60000, 50000, 70);
+  const Dag flat = make(140000, 139000, 17), skewed = make(140000, 20000, 10, 2000, 500), few = make(60000, 50000, 70);
   g_closed = ~0ull >> 3;
   for (const Dag* g : {&flat, &skewed, &few})
     for (const auto& use : {use_graph, use_batch}) {
@@ -268,10 +269,45 @@ static void memory(int, char**) {
   g_budget = ~(size_t)0;
 }
 
+// Which graphs get codes and which lines; codes that too few edges can use go.
+static void choice(int, char**) {
+  Ctx ctx;
+  uint64_t total;
+  struct Got {
+    bool codes, lines;
+    int64_t bytes;
+  };
+  auto got = [&](const Dag& g) {
+    const tc_csr_view v = g.view();
+    tc_graph* dg = nullptr;
+    g_big_codes = 0;
+    CHECK(tc_graph_upload(ctx, &v, TC_CHECK_SHAPE, &dg) == TC_OK);
+    CHECK(tc_count_binned(ctx, dg, &total, nullptr) == TC_OK);
+    const Got x{g_args.c16 != nullptr, g_args.lines != nullptr, tc_graph_bytes(dg)};
+    CHECK((g_args.core != 0) == x.codes);
+    tc_graph_free(ctx, dg);
+    return x;
+  };
+  g_closed = ~0ull >> 3;
+  const Dag skewed = make(140000, 20000, 10, 2000, 500);
+  const int64_t m = (int64_t)skewed.ci.size();
+  const Got with = got(skewed);
+  CHECK(with.codes && !with.lines && g_big_codes == 1);
+  g_closed = (unsigned long long)m / 4 - 1;
+  const Got without = got(skewed);
+  CHECK(!without.codes && g_big_codes == 1 && with.bytes - without.bytes == (int64_t)tck::code_bytes(m) + m + 140000);
+  g_closed = ~0ull >> 3;
+  for (const Dag& flat : {make(140000, 60000, 80), make(140000, 139000, 17, 1, 64), make(140000, 139000, 17, 3, 600)}) {
+    const Got x = got(flat);
+    CHECK(!x.codes && x.lines && g_big_codes == 0);
+  }
+}
+
 int main(int argc, char** argv) {
   static const std::map<std::string, std::function<void(int, char**)>> all = {
       {"one_shot", one_shot},
       {"memory", memory},
+      {"choice", choice},
   };
   const auto it = argc > 1 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;

@@ -44,3 +44,7 @@ def test_one_shot_calls_prepare_for_one_count(fake):
 
 def test_codes_and_lines_take_no_memory_that_is_needed(fake):
     fake("memory")
+
+
+def test_which_graphs_get_codes_and_lines(fake):
+    fake("choice")
