@@ -22,6 +22,7 @@ struct tc_batch final : tcr::Spare {
   tck::GraphDesc* d_descs = nullptr;
   std::vector<tck::GraphDesc> descs;
   std::vector<int32_t> rows;
+  std::vector<uint8_t> short_lists;  // per graph, DagShape::short_lists
   int64_t P = 0;        // plan indices (partner-row slots over all graphs)
   int64_t RP = 0;       // rowptr pool slots
   int64_t cio = 0;      // colidx pool slots
@@ -119,11 +120,13 @@ static tc_status build_batch(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_gra
   b->n = n_graphs;
   b->descs.resize(n_graphs);
   b->rows.resize(n_graphs);
+  b->short_lists.resize(n_graphs);
   int64_t rpo = 0, cio = 0, pro = 0;
   for (int32_t i = 0; i < n_graphs; ++i) {
     const int32_t nvm = tck::partner_rows_max(dags[i].n_rows, dags[i].nnz);
     b->descs[i] = tck::GraphDesc{rpo, cio, cio, rpo, pro, dags[i].n_rows, nvm, 0, dags[i].n_rows, cio};
     b->rows[i] = dags[i].n_rows;
+    b->short_lists[i] = DagShape(dags[i]).short_lists();
     rpo += dags[i].n_rows + 1;
     cio += dags[i].nnz;
     pro += (int64_t)nvm + 1;
@@ -389,7 +392,8 @@ tc_status tc_batch_count_each(tc_ctx* ctx, tc_batch* b, uint64_t* counts, double
     const int64_t P = b->rows[i];
     const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(ctx->plain_grid, (P + tck::kWaves - 1) / tck::kWaves));
     TC_HIP_TRY(hipMemsetAsync(d_out + i, 0, sizeof(uint64_t), s));
-    TC_HIP_TRY(tck::launch_plain(b->rp + d.rp_off, b->ci + d.ci_off, 0, b->rows[i], nullptr, d_out + i, grid, s));
+    TC_HIP_TRY(tck::launch_plain(b->rp + d.rp_off, b->ci + d.ci_off, 0, b->rows[i], nullptr, d_out + i, grid,
+                                 b->short_lists[i] != 0, s));
     TC_HIP_TRY(hipMemcpyAsync(b->pinned + i, d_out + i, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
     TC_HIP_TRY(hipStreamSynchronize(s));
     counts[i] = b->pinned[i];

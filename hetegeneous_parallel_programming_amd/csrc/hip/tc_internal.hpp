@@ -139,6 +139,24 @@ struct Stager {
   hipError_t ring();
 };
 
+// What an upload's choices go by: one pass over the row offsets.
+struct DagShape {
+  int64_t max_out = 0;
+  uint64_t squares = 0;  // sum of the out-degrees' squares: bounds the ids a count streams
+  double mean = 0;       // squares per id: the mean length of the list an id is in
+  double skew = 0;       // squares against those of lists of equal length
+  DagShape() = default;
+  explicit DagShape(const tc_csr_view& dag);  // (rowptr checked; squares stay below 2^64 where max_out passes)
+  // ER graphs of mean out-degree 2 to 100 have 1.1 to 1.5, R-MAT graphs 3.5 and more.
+  bool flat() const { return skew < 2.0; }
+  // The plain kernel's loads of four ids waste much of themselves on short
+  // lists; in uneven graphs most ids streamed are in longer ones (us, ids
+  // loaded four at a time / singly: ER of mean 5.9, n=1000000 590 / 519, of
+  // 9.5, n=1500000 930 / 852, of 14.3, n=1000000 687 / 689, of 24.1, n=600000
+  // 554 / 623; R-MAT of 8.3, n=10000 25.6 / 27.0).
+  bool short_lists() const { return flat() && mean < 12.0; }
+};
+
 // Makes ctx's device current for the scope of one API call.
 struct DeviceGuard {
   int prev = -1;
@@ -244,6 +262,7 @@ struct tc_graph final : tcr::Spare {
   }
   int32_t* pown = nullptr;  // [nv_max + 1] owner vertex of each partner row, written by every build
   int32_t max_out = 0;
+  bool short_lists = false;  // DagShape::short_lists
   tcr::Partners partners;
   tcr::LocalBufs local;
   int32_t nv_max = 0;   // partner rows it may need (nv_max + 1 slots = plan indices)

@@ -160,10 +160,13 @@ struct PivotSet {
 // values; typing them as global keeps the element loads global_load (a
 // generic pointer would make them flat loads, which also wait on LDS).
 typedef __attribute__((address_space(1))) const int32_t gint32;
-// kChunk consecutive ids anywhere in a list: only int32-aligned, which global
+// CH consecutive ids anywhere in a list: only int32-aligned, which global
 // loads of any width allow.
-typedef int32_t chunk_ids __attribute__((ext_vector_type(kChunk), aligned(4)));
-typedef __attribute__((address_space(1))) const chunk_ids gchunk;
+template <int CH>
+struct IdLoad {
+  typedef int32_t ids __attribute__((ext_vector_type(CH), aligned(4)));
+  typedef __attribute__((address_space(1))) const ids gids;
+};
 
 constexpr int32_t kEmpty = -1;
 constexpr uint32_t kHashA0 = 0x9E3779u;  // odd 24-bit multipliers: 2^24 / phi,
@@ -375,8 +378,8 @@ __device__ __forceinline__ uint32_t group_sum(uint32_t x) {
 // bucket of each table) and four compares per id.  Only the first rem[c] ids
 // of chunk c count.  kLocal: a chunk's hits also go to the hit counter of its
 // batch edge kq[] and (kLocalFull) each hit to that of its slot.
-template <int G, int NC, int kLocal, bool kWide>
-__device__ __forceinline__ void hash_probe(const PivotSet& S, const int (&w)[NC * kChunk], const int (&rem)[NC],
+template <int G, int NC, int kLocal, bool kWide, int CH>
+__device__ __forceinline__ void hash_probe(const PivotSet& S, const int (&w)[NC * CH], const int (&rem)[NC],
                                            const int (&kq)[NC], uint32_t& hits, const LocalSink& ls) {
   const char* Tb = (const char*)S.A;
   const int lb = S.p0;
@@ -384,8 +387,8 @@ __device__ __forceinline__ void hash_probe(const PivotSet& S, const int (&w)[NC 
   for (int c = 0; c < NC; ++c) {
     uint32_t h = 0;
 #pragma unroll
-    for (int i = 0; i < kChunk; ++i) {
-      const int q = c * kChunk + i;
+    for (int i = 0; i < CH; ++i) {
+      const int q = c * CH + i;
       const int hk = hash_key<kWide>(w[q]);
       const uint32_t b0 = hash_bucket(hk, kHashA0, lb), b1 = hash_bucket(hk, kHashA1, lb);
       const int2 x = *(const int2*)(Tb + (b0 << 3));
@@ -448,7 +451,7 @@ struct RefEdges {
 
 // kWide: hash sets hold keys folded for ids past 2^24 (kSetHashWide); one
 // instantiation per hash kind keeps a single lookup path in the loop.
-template <int G, int kModes, int NC = kInFlight, int kLocal = kLocalNone, bool kWide = false, class Src>
+template <int G, int kModes, int NC = kInFlight, int kLocal = kLocalNone, bool kWide = false, int CH = kChunk, class Src>
 __device__ __forceinline__ uint32_t pivot_edges(const int32_t* __restrict__ ci, const Src src, int da,
                                                 const PivotSet S, int jfirst, int jstride,
                                                 uint32_t* sEnd, gint32** sBase, int gl,
@@ -473,7 +476,7 @@ __device__ __forceinline__ uint32_t pivot_edges(const int32_t* __restrict__ ci, 
     // flat indexes are unsigned: 64 lists of almost 2^25 ids, in whole
     // chunks, reach 2^31
     int sum;
-    const uint32_t excl = (uint32_t)group_excl_scan<G>((c + kChunk - 1) & -kChunk, gl, sum);
+    const uint32_t excl = (uint32_t)group_excl_scan<G>((c + CH - 1) & -CH, gl, sum);
     const uint32_t total = (uint32_t)sum;
     sEnd[gl] = excl + (uint32_t)c;
     sBase[gl] = base - excl;
@@ -519,68 +522,71 @@ __device__ __forceinline__ uint32_t pivot_edges(const int32_t* __restrict__ ci, 
       cur_end = e;
       cur_base = sBase[k];
     };
-    constexpr int NF = NC * kChunk;
+    constexpr int NF = NC * CH;
     for (uint32_t t0 = 0; t0 < total; t0 += G * NF) {
       int w[NF];
       int rem[NC];  // ids of each chunk that count
       int kq[NC];   // kLocal: batch edge of each chunk
       auto load = [&](int c, uint32_t t) {
         if (t >= cur_end) step_to(t);
-        const chunk_ids x = *(gchunk*)(cur_base + t);
+        const typename IdLoad<CH>::ids x = *(typename IdLoad<CH>::gids*)(cur_base + t);
 #pragma unroll
-        for (int i = 0; i < kChunk; ++i) w[c * kChunk + i] = x[i];
+        for (int i = 0; i < CH; ++i) w[c * CH + i] = x[i];
         rem[c] = (int)(cur_end - t);
         if constexpr (kLocal) kq[c] = cur_k;
       };
       if ((TC_SPLIT_FULL & (G == 64 ? 1 : 2)) && t0 + G * NF <= total) {  // every lane has NC chunks
 #pragma unroll
-        for (int c = 0; c < NC; ++c) load(c, t0 + (c * G + gl) * kChunk);
+        for (int c = 0; c < NC; ++c) load(c, t0 + (c * G + gl) * CH);
       } else {
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-          const uint32_t t = t0 + (c * G + gl) * kChunk;
+          const uint32_t t = t0 + (c * G + gl) * CH;
 #pragma unroll
-          for (int i = 0; i < kChunk; ++i) w[c * kChunk + i] = 0;
+          for (int i = 0; i < CH; ++i) w[c * CH + i] = 0;
           rem[c] = 0;
           if constexpr (kLocal) kq[c] = 0;
           if (t < total) load(c, t);
         }
       }
       if ((kModes & kModeHash) && S.mode == (kWide ? kSetHashWide : kSetHash)) {
-        hash_probe<G, NC, kLocal, kWide>(S, w, rem, kq, hits, ls);
+        hash_probe<G, NC, kLocal, kWide, CH>(S, w, rem, kq, hits, ls);
       } else if ((kModes & kModeTree) && ((kModes == kModeTree) || S.mode == kSetTree)) {
         // h descent steps; then the lower bound is k with its trailing one
         // bits and the following zero shifted out (0 = past the end -> -1).
         // The node index is carried as a byte offset (4k): one compare, one
         // select and one shift-add per step.  ~k is never 0 (k < 2^h).
         // (One chunk at a time: a set is rarely a tree, and the hash lookups'
-        // loop should not pay registers for it.)
+        // loop should not pay registers for it; single ids all together.)
         const int h = S.p0;
         const char* Ab = (const char*)A;
+        constexpr int kAt = CH > 1 ? CH : NC;
+        static_assert(!kLocal || kAt == CH, "hits are attributed by chunk");
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          int kb[kChunk];
+        for (int q0 = 0; q0 < NF; q0 += kAt) {
+          int kb[kAt];
 #pragma unroll
-          for (int i = 0; i < kChunk; ++i) kb[i] = 4;
+          for (int i = 0; i < kAt; ++i) kb[i] = 4;
           for (int s = 0; s < h; ++s) {
-            int val[kChunk];
+            int val[kAt];
 #pragma unroll
-            for (int i = 0; i < kChunk; ++i) val[i] = *(const int32_t*)(Ab + kb[i]);
+            for (int i = 0; i < kAt; ++i) val[i] = *(const int32_t*)(Ab + kb[i]);
 #pragma unroll
-            for (int i = 0; i < kChunk; ++i) kb[i] = 2 * kb[i] + (val[i] < w[c * kChunk + i] ? 4 : 0);
+            for (int i = 0; i < kAt; ++i) kb[i] = 2 * kb[i] + (val[i] < w[q0 + i] ? 4 : 0);
           }
           uint32_t hc = 0;
 #pragma unroll
-          for (int i = 0; i < kChunk; ++i) {
+          for (int i = 0; i < kAt; ++i) {
+            const int q = q0 + i;
             const unsigned k = (unsigned)kb[i] >> 2;
             const unsigned lo = (k >> __builtin_ctz(~k)) >> 1;
-            const bool f = (A[lo] == w[c * kChunk + i]) & (i < rem[c]);
+            const bool f = (A[lo] == w[q]) & (q % CH < rem[q / CH]);
             hc += f ? 1u : 0u;
             if constexpr (kLocal == kLocalFull)
               if (f) count_slot_hit(ls.C, (int)lo);
           }
           hits += hc;
-          if constexpr (kLocal) edge_hits<G, kLocal>(ls.EC, kq[c], hc);
+          if constexpr (kLocal) edge_hits<G, kLocal>(ls.EC, kq[q0 / CH], hc);
         }
       } else if (kModes & kModeHbm) {
         int lo[NF];
@@ -596,8 +602,8 @@ __device__ __forceinline__ uint32_t pivot_edges(const int32_t* __restrict__ ci, 
         for (int c = 0; c < NC; ++c) {
           uint32_t hc = 0;
 #pragma unroll
-          for (int i = 0; i < kChunk; ++i) {
-            const int q = c * kChunk + i;
+          for (int i = 0; i < CH; ++i) {
+            const int q = c * CH + i;
             const bool f = (A[lo[q]] == w[q]) & (i < rem[c]);
             hc += f ? 1u : 0u;
             if constexpr (kLocal == kLocalFull)
@@ -2890,6 +2896,8 @@ struct __align__(16) PlainLds {
   uint64_t red[kWaves];
 };
 
+// CH: ids per load.
+template <int CH>
 __global__ __launch_bounds__(kBlock, TC_COUNT_WAVES_PER_EU) void plain_kernel(const int64_t* __restrict__ rp,
                                                        const int32_t* __restrict__ ci,
                                                        int32_t row_begin, int32_t row_end,
@@ -2904,17 +2912,17 @@ __global__ __launch_bounds__(kBlock, TC_COUNT_WAVES_PER_EU) void plain_kernel(co
     const int da = (int)(rp[u + 1] - rb);
     if (da < 2 || (own && !own[u])) continue;
     constexpr int kModes = kModeTree | kModeHbm;
-    constexpr int kPlainInFlight = 2;
+    constexpr int kPlainInFlight = CH > 1 ? 2 : 6;
     if (da <= kCapWave - 1) {
       stage_tree(L.A[wid], ci + rb, da, lane, 64);
       wave_sync();
       const PivotSet S{L.A[wid], kSetTree, tree_levels(da), 0};
-      acc += pivot_edges<64, kModes, kPlainInFlight>(ci, DagEdges{rp, ci + rb}, da, S, 0, 64, L.End + wid * 64,
+      acc += pivot_edges<64, kModes, kPlainInFlight, kLocalNone, false, CH>(ci, DagEdges{rp, ci + rb}, da, S, 0, 64, L.End + wid * 64,
                                                      L.Base + wid * 64, lane);
       wave_sync();
     } else {
       const PivotSet S{ci + rb, kSetHbm, da, 0};
-      acc += pivot_edges<64, kModes, kPlainInFlight>(ci, DagEdges{rp, ci + rb}, da, S, 0, 64, L.End + wid * 64,
+      acc += pivot_edges<64, kModes, kPlainInFlight, kLocalNone, false, CH>(ci, DagEdges{rp, ci + rb}, da, S, 0, 64, L.End + wid * 64,
                                                      L.Base + wid * 64, lane);
     }
   }
@@ -3233,8 +3241,9 @@ hipError_t launch_local_parts(const int32_t* ci, const int32_t* esrc, int64_t n,
 }
 
 hipError_t launch_plain(const int64_t* rp, const int32_t* ci, int32_t row_begin, int32_t row_end,
-                        const uint8_t* own, uint64_t* out, int grid, hipStream_t s, uint64_t* host) {
-  plain_kernel<<<grid, kBlock, 0, s>>>(rp, ci, row_begin, row_end, own, out, host);
+                        const uint8_t* own, uint64_t* out, int grid, bool single, hipStream_t s, uint64_t* host) {
+  if (single) plain_kernel<1><<<grid, kBlock, 0, s>>>(rp, ci, row_begin, row_end, own, out, host);
+  else plain_kernel<kChunk><<<grid, kBlock, 0, s>>>(rp, ci, row_begin, row_end, own, out, host);
   return hipGetLastError();
 }
 
@@ -3291,7 +3300,7 @@ int count_blocks_per_cu() {
 
 int plain_blocks_per_cu() {
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, plain_kernel, kBlock, 0) != hipSuccess) return 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, plain_kernel<kChunk>, kBlock, 0) != hipSuccess) return 1;
   return n > 0 ? n : 1;
 }
 

@@ -484,8 +484,10 @@ hipError_t launch_count_part(const LaunchArgs& a, int cus, int grid, int part, c
 // address); out is then kOutWords words, left 0.  For sums below 2^kDoneShift
 // and grids below 2^(64 - kDoneShift).
 constexpr int kDoneShift = 48;
+// single: ids are loaded one at a time, not kChunk (see tcr::DagShape::short_lists).
 hipError_t launch_plain(const int64_t* rp, const int32_t* ci, int32_t row_begin, int32_t row_end,
-                        const uint8_t* own, uint64_t* out, int grid, hipStream_t s, uint64_t* host = nullptr);
+                        const uint8_t* own, uint64_t* out, int grid, bool single, hipStream_t s,
+                        uint64_t* host = nullptr);
 // Count of one graph that also fills a.local: same plan, the local variants
 // of the hash kernel over all bins.  mode kLocalFull: ecount and vcount (zeroed by the
 // caller); kLocalEdges: ecount only (the kernels keep no slot hit counters:

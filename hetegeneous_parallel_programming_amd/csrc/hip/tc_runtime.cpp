@@ -303,31 +303,29 @@ tck::Tune to_kernel_tune(const tc_tune& t) {
   return tck::Tune{t.t_g8, t.t_g16, t.t_g32, t.t_wave, t.rounds, t.pivot_set, t.hash_kicks};
 }
 
+DagShape::DagShape(const tc_csr_view& dag) {
+  int64_t lists = 0;
+  for (int64_t v = 0; v < dag.n_rows; ++v) {
+    const int64_t d = dag.rowptr[v + 1] - dag.rowptr[v];
+    max_out = std::max(max_out, d);
+    squares += (uint64_t)d * (uint64_t)d;
+    lists += d > 0;
+  }
+  if (lists) {
+    mean = (double)squares / (double)dag.nnz;
+    skew = mean * (double)lists / (double)dag.nnz;
+  }
+}
+
 // Host-side checks shared by every upload: shape (and more when asked), and
 // the per-batch int32 element total (64 lists of at most max_out ids).
-struct DagShape {
-  int32_t max_out = 0;
-  uint64_t squares = 0;  // sum over rows of out-degree squared: bounds the ids a count streams
-  // squares against those of lists of equal length: 1.1 to 1.3 in flat graphs
-  // (ER of mean out-degree 4 to 50), 3.5 and more in R-MAT graphs
-  double skew = 0;
-};
 static tc_status check_dag(const tc_csr_view* dag, uint32_t check, DagShape* shape) {
   if (!dag) return fail(TC_EINVAL, "null csr view");
   tc_status st = tch_validate(dag, check | TC_CHECK_SHAPE);
   if (st != TC_OK) return fail(st, tch_last_error());
-  int64_t mo = 0;
-  uint64_t squares = 0;  // (below 2^64 for any graph that passes)
-  int64_t lists = 0;
-  for (int64_t v = 0; v < dag->n_rows; ++v) {
-    const int64_t d = dag->rowptr[v + 1] - dag->rowptr[v];
-    mo = std::max<int64_t>(mo, d);
-    squares += (uint64_t)d * (uint64_t)d;
-    lists += d > 0;
-  }
-  if (mo * 64 >= ((int64_t)1 << 31))
+  *shape = DagShape(*dag);
+  if (shape->max_out * 64 >= ((int64_t)1 << 31))
     return fail(TC_ERANGE, "DAG out-degree too large (max_out * 64 must fit in int32)");
-  *shape = DagShape{(int32_t)mo, squares, lists ? (double)squares * (double)lists / ((double)dag->nnz * (double)dag->nnz) : 0.0};
   return TC_OK;
 }
 
@@ -337,8 +335,7 @@ static tc_status check_dag(const tc_csr_view* dag, uint32_t check, DagShape* sha
 // ids, lists to 180: 2.75 ms with codes, 2.44 without, 2.21 with lists on
 // lines; n=80001 of 4 M, 97% of the edges coded: 0.252, 0.212, 0.215).
 constexpr int32_t kCodesMinOut = 64;
-constexpr double kCodesSkew = 2.0;
-static bool wants_codes(const DagShape& shape) { return shape.max_out >= kCodesMinOut && shape.skew >= kCodesSkew; }
+static bool wants_codes(const DagShape& shape) { return shape.max_out >= kCodesMinOut && !shape.flat(); }
 // They are kept and counted with only when one edge in kCodedShare can use
 // them: that much repays the bitmap kernels' launches.  The line is not a sharp
 // one (without / with codes: at 43% 0.509 / 0.507 ms, at 73% 0.287 / 0.288, of
@@ -354,9 +351,10 @@ constexpr int64_t kCodedShare = 4;
 // ids (165 squares an id) 4.07 / 4.59, n=1000000 of 15 M (151) 7.05 / 7.49,
 // n=6000000 of 30 M (80) 17.4 / 18.4; n=2000000 of 30 M (179) 13.5 / 13.0,
 // n=500000 of 30 M (419) 13.4 / 11.0, n=4266666 of 64 M (218) 28.7 / 26.1.
-constexpr uint64_t kOnceSquares = (uint64_t)1 << 32, kOnceSquaresPerId = 128;
-static bool once_repays_codes(int64_t nnz, uint64_t squares) {
-  return squares >= kOnceSquares && squares >= kOnceSquaresPerId * (uint64_t)nnz;
+constexpr uint64_t kOnceSquares = (uint64_t)1 << 32;
+constexpr double kOnceMean = 128;
+static bool once_repays_codes(const DagShape& shape) {
+  return shape.squares >= kOnceSquares && shape.mean >= kOnceMean;
 }
 
 // Graphs past tck::kCoreIds rows that want no codes, of this many ids on, get
@@ -379,7 +377,8 @@ static tc_status build_graph(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_be
   g->row_end = row_end;
   g->edge_begin = dag->rowptr[row_begin];
   g->edge_end = dag->rowptr[row_end];
-  g->max_out = shape.max_out;
+  g->max_out = (int32_t)shape.max_out;
+  g->short_lists = shape.short_lists();
   g->nv_max = tck::partner_rows_max(g->n, g->nnz);
   auto cleanup = [&]() {
     dev_free(g->rp);
@@ -433,7 +432,7 @@ static tc_status build_graph(tc_ctx* ctx, const tc_csr_view* dag, int32_t row_be
   // The bitmap kernels' codes and the lists on lines, which a count can do
   // without: taken last, none where there is no memory for them.
   bool big = wants_codes(shape) && tck::big_codes_fit(g->n, g->nnz) &&
-             (!once || once_repays_codes(g->nnz, shape.squares)) &&
+             (!once || once_repays_codes(shape)) &&
              tck::big_codes_bytes(g->n, g->nnz) <= bs.cap;
   if (big || (g->n <= tck::kCoreIds && g->nnz < tck::kCorePool)) {
     st = dev_alloc((void**)&g->c16, tck::code_bytes(g->nnz), "id codes");
@@ -848,7 +847,7 @@ static tc_status plain_count(tc_ctx* ctx, tc_graph* g, uint64_t* out, uint64_t* 
   if (!kept_zero || ctx->plain_dirty || !direct) TC_HIP_TRY(tck::launch_zero(out, 2 * tck::kOutWords, s));
   if (kept_zero) ctx->plain_dirty = true;
   TC_HIP_TRY(hipEventRecord(ctx->ev[1], s));
-  TC_HIP_TRY(tck::launch_plain(g->rp, g->ci, g->row_begin, g->row_end, g->own, out, grid, s,
+  TC_HIP_TRY(tck::launch_plain(g->rp, g->ci, g->row_begin, g->row_end, g->own, out, grid, g->short_lists, s,
                                direct ? ctx->pinned_dev : nullptr));
   TC_HIP_TRY(hipEventRecord(ctx->ev[2], s));
   if (!direct) TC_HIP_TRY(hipMemcpyAsync(ctx->pinned, out, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
@@ -879,7 +878,7 @@ constexpr int64_t kPlainFlatMaxIds = (int64_t)1 << 21;
 constexpr int64_t kPlainFlatMaxRows = (int64_t)1 << 17;
 constexpr int32_t kPlainFlatMaxOut = 64;
 
-static bool plain_fits(int64_t rows, int64_t ids, int32_t max_out) {
+static bool plain_fits(int64_t rows, int64_t ids, int64_t max_out) {
   if (max_out >= tck::kCapWave) return false;
   return ids <= kPlainMaxIds ||
          (ids <= kPlainFlatMaxIds && rows <= kPlainFlatMaxRows && max_out <= kPlainFlatMaxOut);
@@ -968,7 +967,8 @@ tc_status tc_count_csr(tc_ctx* ctx, const tc_csr_view* dag, uint32_t check, uint
   g.row_begin = 0;
   g.row_end = dag->n_rows;
   g.edge_end = dag->nnz;
-  g.max_out = shape.max_out;
+  g.max_out = (int32_t)shape.max_out;
+  g.short_lists = shape.short_lists();
   return tcr::plain_count(ctx, &g, ctx->plain_out, total, stats, true);
 } catch (...) {
   return tcr::caught();

@@ -79,6 +79,7 @@ static tck::BuildBufs g_build;           // of the last partner build
 static unsigned long long g_closed = 0;  // what launch_big_codes reports
 static int g_big_codes = 0;              // its launches
 static tck::LaunchArgs g_args;           // of the last count
+static bool g_single = false;            // of the last plain launch
 namespace tck {
 int64_t scan_partials(int64_t n) { return n / 1024 + 2; }
 int64_t big_codes_bytes(int64_t n, int64_t m) { return 12 * n + 2 * m; }
@@ -95,7 +96,7 @@ hipError_t launch_plan(const LaunchArgs& a, hipStream_t) { return g_args = a, hi
 hipError_t launch_count(const LaunchArgs& a, int, int, hipStream_t) { return g_args = a, hipSuccess; }
 bool part_empty(const LaunchArgs&, int, const int64_t*) { return false; }
 hipError_t launch_count_part(const LaunchArgs& a, int, int, int, const int64_t*, hipStream_t) { return g_args = a, hipSuccess; }
-hipError_t launch_plain(const int64_t*, const int32_t*, int32_t, int32_t, const uint8_t*, uint64_t*, int, hipStream_t, uint64_t*) { return hipSuccess; }
+hipError_t launch_plain(const int64_t*, const int32_t*, int32_t, int32_t, const uint8_t*, uint64_t*, int, bool single, hipStream_t, uint64_t*) { return g_single = single, hipSuccess; }
 hipError_t launch_count_local(const LaunchArgs& a, int, int, hipStream_t) { return g_args = a, hipSuccess; }
 hipError_t launch_local_prep(const int64_t*, int64_t, int32_t*, hipStream_t) { return hipSuccess; }
 hipError_t launch_local_parts(const int32_t*, const int32_t*, int64_t, int64_t, int64_t, const uint32_t*, const int32_t*, int32_t, unsigned long long*, int, hipStream_t) { return hipSuccess; }
@@ -300,6 +301,27 @@ static void choice(int, char**) {
   for (const Dag& flat : {make(140000, 60000, 80), make(140000, 139000, 17, 1, 64), make(140000, 139000, 17, 3, 600)}) {
     const Got x = got(flat);
     CHECK(!x.codes && x.lines && g_big_codes == 0);
+  }
+  // the plain kernel's loads: one id where lists are short and even
+  const struct {
+    Dag g;
+    bool single;
+  } plain[] = {{make(9000, 8000, 11), true}, {make(9000, 8000, 12), false}, {make(9000, 8000, 1, 100, 300), false}, {make(9, 0, 0), true}};
+  for (const auto& p : plain) {
+    const tc_csr_view v = p.g.view();
+    double ms;
+    g_single = !p.single;
+    CHECK(tc_count_csr(ctx, &v, TC_CHECK_SHAPE, &total, nullptr) == TC_OK && g_single == p.single);
+    tc_graph* dg = nullptr;
+    g_single = !p.single;
+    CHECK(tc_graph_upload(ctx, &v, TC_CHECK_SHAPE, &dg) == TC_OK && tc_count_plain(ctx, dg, &total, nullptr) == TC_OK);
+    CHECK(g_single == p.single);
+    tc_graph_free(ctx, dg);
+    tc_batch* b = nullptr;
+    g_single = !p.single;
+    CHECK(tc_batch_create(ctx, &v, 1, TC_CHECK_SHAPE, &b) == TC_OK && tc_batch_count_each(ctx, b, &total, &ms, nullptr) == TC_OK);
+    CHECK(g_single == p.single);
+    tc_batch_free(ctx, b);
   }
 }
 
