@@ -830,8 +830,6 @@ static tc_status count_binned(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_stat
   return st;
 }
 
-static bool small_graph(const tc_graph* g);
-
 // The plain kernel's single launch, summing in the tck::kOutWords words at
 // `out` on the device.  kept_zero: those are the context's, zero between
 // calls: no zero launch before the kernel.
@@ -841,9 +839,11 @@ static tc_status plain_count(tc_ctx* ctx, tc_graph* g, uint64_t* out, uint64_t* 
   const int64_t P = (int64_t)g->row_end - g->row_begin;
   hipStream_t s = ctx->stream;
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(ctx->plain_grid, (P + tck::kWaves - 1) / tck::kWaves));
-  // A small graph's sum (at most ids * kCapWave) leaves room for the count of
-  // finished workgroups above it.
-  const bool direct = small_graph(g) && grid < 1 << (64 - tck::kDoneShift);
+  // The last workgroup hands the sum over where the most that it can be (every
+  // id of the list of every edge) leaves room for the count of finished
+  // workgroups above it: all but graphs of many ids and a very long list.
+  const bool direct = (double)(g->edge_end - g->edge_begin) * (double)g->max_out < (double)(1ull << tck::kDoneShift) &&
+                      grid < 1 << (64 - tck::kDoneShift);
   if (!kept_zero || ctx->plain_dirty || !direct) TC_HIP_TRY(tck::launch_zero(out, 2 * tck::kOutWords, s));
   if (kept_zero) ctx->plain_dirty = true;
   TC_HIP_TRY(hipEventRecord(ctx->ev[1], s));

@@ -79,7 +79,8 @@ static tck::BuildBufs g_build;           // of the last partner build
 static unsigned long long g_closed = 0;  // what launch_big_codes reports
 static int g_big_codes = 0;              // its launches
 static tck::LaunchArgs g_args;           // of the last count
-static bool g_single = false;            // of the last plain launch
+static bool g_single = false, g_direct = false;  // of the last plain launch
+static int g_launches = 0;               // plain, zero and rearm launches
 namespace tck {
 int64_t scan_partials(int64_t n) { return n / 1024 + 2; }
 int64_t big_codes_bytes(int64_t n, int64_t m) { return 12 * n + 2 * m; }
@@ -88,7 +89,7 @@ hipError_t launch_big_codes(const int64_t*, const int32_t*, int64_t, int64_t, ch
   return *closed = g_closed, ++g_big_codes, hipSuccess;
 }
 hipError_t launch_partners(const LaunchArgs&, int64_t, int64_t, const BuildBufs& b, hipStream_t) { return g_build = b, hipSuccess; }
-hipError_t launch_zero(void* p, int64_t n, hipStream_t) { return std::memset(p, 0, 4 * (size_t)n), hipSuccess; }
+hipError_t launch_zero(void* p, int64_t n, hipStream_t) { return ++g_launches, std::memset(p, 0, 4 * (size_t)n), hipSuccess; }
 hipError_t launch_stage_copy(const StageCopy*, int32_t, int64_t, hipStream_t) { return hipSuccess; }
 hipError_t launch_rearm(uint32_t*, uint64_t*, int32_t, hipStream_t) { return hipSuccess; }
 hipError_t launch_finish(uint32_t*, uint64_t*, uint64_t* host, hipStream_t) { return host[0] = host[1] = 0, hipSuccess; }
@@ -96,7 +97,9 @@ hipError_t launch_plan(const LaunchArgs& a, hipStream_t) { return g_args = a, hi
 hipError_t launch_count(const LaunchArgs& a, int, int, hipStream_t) { return g_args = a, hipSuccess; }
 bool part_empty(const LaunchArgs&, int, const int64_t*) { return false; }
 hipError_t launch_count_part(const LaunchArgs& a, int, int, int, const int64_t*, hipStream_t) { return g_args = a, hipSuccess; }
-hipError_t launch_plain(const int64_t*, const int32_t*, int32_t, int32_t, const uint8_t*, uint64_t*, int, bool single, hipStream_t, uint64_t*) { return g_single = single, hipSuccess; }
+hipError_t launch_plain(const int64_t*, const int32_t*, int32_t, int32_t, const uint8_t*, uint64_t*, int, bool single, hipStream_t, uint64_t* host) {
+  return g_single = single, g_direct = host != nullptr, ++g_launches, hipSuccess;
+}
 hipError_t launch_count_local(const LaunchArgs& a, int, int, hipStream_t) { return g_args = a, hipSuccess; }
 hipError_t launch_local_prep(const int64_t*, int64_t, int32_t*, hipStream_t) { return hipSuccess; }
 hipError_t launch_local_parts(const int32_t*, const int32_t*, int64_t, int64_t, int64_t, const uint32_t*, const int32_t*, int32_t, unsigned long long*, int, hipStream_t) { return hipSuccess; }
@@ -325,11 +328,36 @@ static void choice(int, char**) {
   }
 }
 
+// A plain count is one launch, whatever the graph's size, unless its sum might
+// not fit beside the count of workgroups; the one after such a count clears
+// the words first.
+static void plain(int, char**) {
+  Ctx ctx;
+  for (const Dag& g : {make(9000, 8000, 11), make(300000, 200000, 20), make(9000, 8000, 1, 1, 4000)}) {
+    const tc_csr_view v = g.view();
+    tc_graph* dg = nullptr;
+    uint64_t total;
+    CHECK(tc_graph_upload(ctx, &v, TC_CHECK_SHAPE, &dg) == TC_OK);
+    for (int i = 0; i < 3; ++i) {
+      g_launches = 0;
+      CHECK(tc_count_plain(ctx, dg, &total, nullptr) == TC_OK && g_direct && (g_launches == 1 || i == 0));
+    }
+    dg->max_out = 1 << 25;  // as if of a list that long: 2^25 * ids may pass 2^48
+    const bool fits = (uint64_t)dg->max_out * g.ci.size() < 1ull << tck::kDoneShift;
+    g_launches = 0;
+    CHECK(tc_count_plain(ctx, dg, &total, nullptr) == TC_OK && g_direct == fits && g_launches == (fits ? 1 : 2));
+    dg->edge_end = (int64_t)1 << 30;
+    CHECK(tc_count_plain(ctx, dg, &total, nullptr) == TC_OK && !g_direct);
+    tc_graph_free(ctx, dg);
+  }
+}
+
 int main(int argc, char** argv) {
   static const std::map<std::string, std::function<void(int, char**)>> all = {
       {"one_shot", one_shot},
       {"memory", memory},
       {"choice", choice},
+      {"plain", plain},
   };
   const auto it = argc > 1 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;

@@ -48,3 +48,7 @@ def test_codes_and_lines_take_no_memory_that_is_needed(fake):
 
 def test_which_graphs_get_codes_and_lines(fake):
     fake("choice")
+
+
+def test_a_plain_count_is_one_launch(fake):
+    fake("plain")
