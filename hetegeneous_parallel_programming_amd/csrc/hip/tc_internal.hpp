@@ -157,6 +157,22 @@ struct DagShape {
   bool short_lists() const { return flat() && mean < 12.0; }
 };
 
+// Threads that copy a server request of `bytes`, of `clients` that are copying
+// one (this one among them).  One thread moves ~9 GB/s, so a request is split
+// from 1 MB a thread on; but the clients share kCopyThreads, since more threads
+// than that only cost their start (8 clients with requests of 1.2 M ids on
+// MI355X: a thread per MB each 0.60 ms a submit, one each 0.31; one client
+// 0.25 -> 0.18).  Requests of 16 MB and more have up to 4 whatever the others
+// do: their copies outlast that.
+constexpr size_t kCopySplit = (size_t)1 << 20, kCopySplitLarge = (size_t)8 << 20;
+constexpr int kCopyThreads = 8, kCopyThreadsLarge = 4;
+inline int copy_threads(size_t bytes, int clients) {
+  const int64_t by_size = (int64_t)(bytes / kCopySplit), large = (int64_t)(bytes / kCopySplitLarge);
+  const int64_t share = by_size < kCopyThreads / clients ? by_size : kCopyThreads / clients;
+  const int64_t n = large < kCopyThreadsLarge ? large : kCopyThreadsLarge;
+  return (int)(n > share ? n : share > 1 ? share : 1);
+}
+
 // Makes ctx's device current for the scope of one API call.
 struct DeviceGuard {
   int prev = -1;

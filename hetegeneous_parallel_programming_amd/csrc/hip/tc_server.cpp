@@ -53,11 +53,7 @@ struct Layout {
 // kMaxOutDegree, ids in [0, n).  One read of the caller's arrays, in plain
 // loops -- an OpenMP region per call, from several client threads at once,
 // costs far more than the loops themselves for graphs of a few thousand ids.
-// A large request is split over helper threads, since one thread
-// moves ~9 GB/s and an RMAT-20 request holds ~71 MB of CSR (two of those among
-// 254 light ones: 4 threads of 8 MB and more 16.2 ms, these 15.3).
-constexpr size_t kCopySplit = (size_t)1 << 20;  // bytes per helper thread at least
-constexpr int kCopyThreads = 8;
+// A large request is split over helper threads (copy_threads).
 constexpr int64_t kMaxOutDegree = (int64_t)1 << 25;  // d * 64 < 2^31 in the plan's wedge-work field
 
 struct ShapeFlags {
@@ -86,12 +82,19 @@ void check_copy(const tc_csr_view& g, int64_t* rp_dst, int32_t* ci_dst, int64_t 
 }
 
 // Copies g (rowptr[0] == 0 and rowptr[n] == nnz already checked) to rp_dst /
-// ci_dst; returns null, or what is wrong with its shape.
-const char* stage_checked(const tc_csr_view& g, int64_t* rp_dst, int32_t* ci_dst) {
+// ci_dst; returns null, or what is wrong with its shape.  copying: requests
+// that are in here.
+const char* stage_checked(const tc_csr_view& g, int64_t* rp_dst, int32_t* ci_dst, std::atomic<int>& copying) {
   const int64_t n = g.n_rows, m = g.nnz;
   rp_dst[0] = 0;
   const size_t bytes = sizeof(int64_t) * (size_t)n + sizeof(int32_t) * (size_t)m;
-  const int nt = (int)std::max<size_t>(1, std::min<size_t>(kCopyThreads, bytes / kCopySplit));
+  struct Copying {
+    std::atomic<int>& n;
+    const int clients;
+    explicit Copying(std::atomic<int>& c) : n(c), clients(c.fetch_add(1, std::memory_order_relaxed) + 1) {}
+    ~Copying() { n.fetch_sub(1, std::memory_order_relaxed); }
+  } me(copying);
+  const int nt = copy_threads(bytes, me.clients);
   ShapeFlags f[kCopyThreads];
   auto part = [&](int t) {
     check_copy(g, rp_dst, ci_dst, n * t / nt, n * (t + 1) / nt, m * t / nt, m * (t + 1) / nt, f[t]);
@@ -176,6 +179,7 @@ struct tc_server {
   std::deque<Req*> waiting, ready;
   std::deque<tc_request_result> results;
   int64_t outstanding = 0, submitted = 0, completed = 0, rejected = 0, launches = 0, launched_graphs = 0;
+  std::atomic<int> copying{0};  // requests being copied by their clients
   int64_t max_ids = 0;  // DAG ids per launch (cfg.max_batch_ids or its default)
   int64_t heavy_ids = 0;  // cfg.heavy_ids or its default
   int32_t fill_graphs = 0, fill_wait_us = 0;  // cfg's, or their defaults
@@ -675,7 +679,7 @@ static tc_status submit_request(tc_server* s, const tc_csr_view* dag, uint64_t t
     rp_dst = r->rp.data();
     ci_dst = r->ci.data();
   }
-  if (const char* bad = stage_checked(g, rp_dst, ci_dst)) {
+  if (const char* bad = stage_checked(g, rp_dst, ci_dst, s->copying)) {
     if (r->staged) tch_arena_free(s->stage_arena, r->stage_off);
     std::lock_guard<std::mutex> lk(s->mu);
     --s->outstanding;

@@ -352,12 +352,56 @@ static void plain(int, char**) {
   }
 }
 
+// Threads that copy a request: never more than the clients' share, never fewer
+// than a large request's own; concurrent submits all arrive.
+static void clients(int, char**) {
+  constexpr size_t MB = (size_t)1 << 20;
+  for (int c = 1; c <= 64; ++c)
+    for (size_t mb : {0, 1, 2, 3, 5, 8, 15, 16, 24, 31, 32, 70, 1000}) {
+      const int n = tcr::copy_threads(mb * MB, c), large = (int)std::min<size_t>(4, mb / 8);
+      CHECK(n >= 1 && n <= 8 && (n == 1 || n <= (int)mb) && n >= large);
+      if (mb < 16) CHECK(n * std::min(c, 8) <= 8);      // 8 threads for all that copy at once
+      if (c == 1) CHECK(n == (int)std::min<size_t>(8, std::max<size_t>(1, mb)));
+    }
+  Ctx ctx;
+  tc_server_config cfg{};
+  cfg.hbm_budget = (uint64_t)1 << 30;
+  cfg.host_staging = (uint64_t)64 << 20;  // some requests fit it, others go pageable
+  cfg.slots = 2;
+  cfg.max_batch_graphs = 64;
+  cfg.max_batch_rows = 1 << 22;
+  cfg.max_queue = 1024;
+  tc_server* s = nullptr;
+  CHECK(tc_server_create(ctx, &cfg, &s) == TC_OK);
+  const Dag big = make(60000, 50000, 70), small = make(3000, 2000, 9);
+  Dag bad = make(60000, 50000, 70);
+  bad.ci[bad.ci.size() - 5] = 60000;  // in the last thread's share
+  std::atomic<int> refused{0};
+  std::vector<std::thread> all;
+  for (int c = 0; c < 8; ++c)
+    all.emplace_back([&, c] {
+      for (int i = 0; i < 6; ++i) {
+        const tc_csr_view v = (i % 3 == 0 ? big : i % 3 == 1 ? small : bad).view();
+        const tc_status st = tc_server_submit(s, &v, (uint64_t)(c * 6 + i), TC_CHECK_SHAPE);
+        if (st != TC_OK) ++refused;
+      }
+    });
+  for (std::thread& t : all) t.join();
+  CHECK(refused == 16 && tc_server_drain(s, 60000) == TC_OK);
+  tc_request_result r[64];
+  int32_t n = 0;
+  CHECK(tc_server_poll(s, r, 64, &n, 1000) == TC_OK && n == 32);
+  for (int i = 0; i < n; ++i) CHECK(r[i].status == TC_OK && r[i].tag % 3 != 2);
+  tc_server_destroy(s);
+}
+
 int main(int argc, char** argv) {
   static const std::map<std::string, std::function<void(int, char**)>> all = {
       {"one_shot", one_shot},
       {"memory", memory},
       {"choice", choice},
       {"plain", plain},
+      {"clients", clients},
   };
   const auto it = argc > 1 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;

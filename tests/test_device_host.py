@@ -52,3 +52,7 @@ def test_which_graphs_get_codes_and_lines(fake):
 
 def test_a_plain_count_is_one_launch(fake):
     fake("plain")
+
+
+def test_clients_share_the_copy_threads(fake):
+    fake("clients")
