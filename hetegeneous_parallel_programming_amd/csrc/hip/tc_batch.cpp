@@ -36,6 +36,9 @@ struct tc_batch final : tcr::Spare {
   tc_tune captured{};
   int64_t bytes = 0;
 
+  // Words of scratch.outs: the counts and, with slots, those from the next line on.
+  int64_t slots_at() const { return ((int64_t)n + tck::kOutStride - 1) / tck::kOutStride * tck::kOutStride; }
+  int nslots() const { return c16 && n > 1 ? tck::batch_slots(n) : 1; }
   void drop_graph() {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
@@ -75,12 +78,15 @@ static tc_status capture(tc_ctx* ctx, tc_batch* b) {
   a.c16 = b->c16;
   a.core = b->c16 ? 1 : 0;
   a.core_kb = b->core_kb;
+  a.nslots = b->nslots();
+  if (a.nslots > 1) a.slots = a.bufs.outs + b->slots_at();
+  const int64_t words = a.slots ? b->slots_at() + (int64_t)b->n * a.nslots * tck::kOutStride : b->n;
   for (int32_t r : b->rows) a.wide_ids |= r > tck::kNarrowIds ? 1 : 0;
   hipStream_t s = ctx->stream;
   TC_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
   // Zero fills are kernels, not memset nodes.
   hipError_t e = tck::launch_zero(a.bufs.counters, tck::kNumCounters, s);
-  if (e == hipSuccess) e = tck::launch_zero(a.bufs.outs, 2 * (int64_t)b->n, s);
+  if (e == hipSuccess) e = tck::launch_zero(a.bufs.outs, 2 * words, s);
   if (e == hipSuccess) e = tck::launch_plan(a, s);
   // The first part on the capture stream, the others on forked branches.
   static_assert(tck::kCountParts == tc_ctx::kSides + 1, "one side stream per part past the first");
@@ -96,6 +102,7 @@ static tc_status capture(tc_ctx* ctx, tc_batch* b) {
     e = hipEventRecord(ctx->join[i], ctx->side[i]);
     if (e == hipSuccess) e = hipStreamWaitEvent(s, ctx->join[i], 0);
   }
+  if (e == hipSuccess && a.slots) e = tck::launch_batch_sums(a, s);
   if (e == hipSuccess)
     e = hipMemcpyAsync(b->pinned, a.bufs.outs, sizeof(uint64_t) * (size_t)b->n, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess)
@@ -142,7 +149,10 @@ static tc_status build_batch(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_gra
   if (st == TC_OK)
     st = dev_alloc((void**)&b->d_descs, sizeof(tck::GraphDesc) * (size_t)std::max(n_graphs, 1), "batch descs");
   if (st == TC_OK) st = b->partners.alloc(cio, pro, n_graphs);
-  if (st == TC_OK) st = b->scratch.ensure(b->P, n_graphs);
+  // counts, and room for slots whether or not there will be codes
+  const int64_t slots = tck::batch_slots(n_graphs);
+  const int64_t outs = slots > 1 ? b->slots_at() + n_graphs * slots * tck::kOutStride : n_graphs;
+  if (st == TC_OK) st = b->scratch.ensure(b->P, outs);
   if (st != TC_OK) {
     b->release();
     return st;
@@ -310,7 +320,7 @@ static tc_status build_batch(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_gra
     for (int32_t v : nv) b->nv += v;
   }
   b->bytes = sizeof(int64_t) * rpo + sizeof(int32_t) * cio + (int64_t)sizeof(tck::GraphDesc) * n_graphs +
-             b->partners.bytes + PlanScratch::bytes_for(b->P) + 8 * (int64_t)n_graphs + (b->c16 ? (int64_t)tck::code_bytes(cio) : 0);
+             b->partners.bytes + PlanScratch::bytes_for(b->P) + 8 * outs + (b->c16 ? (int64_t)tck::code_bytes(cio) : 0);
   if (b->c16) {
     try {
       ctx->spares.insert(b.get());

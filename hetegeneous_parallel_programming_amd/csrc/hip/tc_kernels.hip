@@ -2414,7 +2414,8 @@ __global__ __launch_bounds__(64 * NW, 8) void core_kernel(LaunchArgs a, int bin0
       uint32_t h = hits;
 #pragma unroll
       for (int o = 32; o >= 1; o >>= 1) h += __shfl_xor(h, o);
-      if (lane == 0 && h) atomicAdd(&a.bufs.outs[g], (unsigned long long)h);
+      uint64_t* out = a.slots ? a.slots + (g * a.nslots + (int)(blockIdx.x & (a.nslots - 1))) * kOutStride : a.bufs.outs + g;
+      if (lane == 0 && h) atomicAdd((unsigned long long*)out, (unsigned long long)h);
     } else {
       sum += hits;
     }
@@ -3073,6 +3074,22 @@ __global__ __launch_bounds__(kBlock) void finish_kernel(uint32_t* counters, uint
 
 hipError_t launch_finish(uint32_t* counters, uint64_t* outs, uint64_t* host, hipStream_t s) {
   finish_kernel<<<1, kBlock, 0, s>>>(counters, outs, host);
+  return hipGetLastError();
+}
+
+// A wave per graph.
+__global__ __launch_bounds__(kBlock) void batch_sums_kernel(const uint64_t* slots, int nslots, int64_t graphs, uint64_t* outs) {
+  const int64_t g = (int64_t)blockIdx.x * kWaves + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (g >= graphs) return;
+  uint64_t x = lane < nslots ? slots[(g * nslots + lane) * kOutStride] : 0;
+#pragma unroll
+  for (int d = kOutSlots / 2; d >= 1; d >>= 1) x += shfl_down_u64(x, d);
+  if (lane == 0) outs[g] += x;
+}
+
+hipError_t launch_batch_sums(const LaunchArgs& a, hipStream_t s) {
+  batch_sums_kernel<<<(unsigned)((a.ngraphs + kWaves - 1) / kWaves), kBlock, 0, s>>>(a.slots, a.nslots, a.ngraphs, a.bufs.outs);
   return hipGetLastError();
 }
 

@@ -191,6 +191,18 @@ struct PlanBufs {
 // ~12 ns (8192 waves: 0.1 ms).
 constexpr int kOutSlots = 32, kOutStride = 16, kOutWords = kOutSlots * kOutStride;
 
+// A batch of few graphs has the same trouble: every heavy row ends with an add
+// to its graph's word, and the words of 16 graphs share a line (8 graphs R-MAT
+// n=30000 of 1.2 M ids: 1.19 ms; so 0.42).  Words per graph: at most kOutSlots, at most
+// kBatchWords in all; 1 (no slots) from kBatchGraphs on, whose adds are spread
+// by the graphs themselves.
+constexpr int kBatchGraphs = 64, kBatchWords = 512;
+inline int batch_slots(int64_t graphs) {
+  if (graphs >= kBatchGraphs) return 1;
+  int s = kOutSlots;
+  while (s > 1 && s * graphs > kBatchWords) s /= 2;
+  return s;
+}
 
 // A list of the DAG as one word: offset in the colidx pool in the high 39
 // bits, length in the low 25 (out-degrees are below 2^25 by the upload
@@ -285,6 +297,10 @@ struct LaunchArgs {
   int32_t core_kb;
   int32_t wide_ids;     // 1 when ids reach 2^24: hash sets fold the high id bits into the bucket
   int32_t out_slots;    // kOutSlots where bufs.outs holds a single graph's slots, else 0
+  // A batch's bitmap kernels: null (they add to bufs.outs), or slots[g * nslots + i]
+  // a cache line apart, i < nslots (a power of two), added by launch_batch_sums.
+  uint64_t* slots;
+  int32_t nslots;
   int32_t gbase;        // partner build of a segment of graphs: index of descs[0] among all graphs
 };
 
@@ -438,6 +454,8 @@ hipError_t launch_rearm(uint32_t* counters, uint64_t* outs, int32_t nouts, hipSt
 // as much again between launches (R-MAT n=30011: 85 -> 72 us a call, R-MAT-18
 // 215 -> 200).
 hipError_t launch_finish(uint32_t* counters, uint64_t* outs, uint64_t* host, hipStream_t s);
+// outs[g] += the slots of graph g, for every graph of a batch with slots.
+hipError_t launch_batch_sums(const LaunchArgs& a, hipStream_t s);
 hipError_t launch_plan(const LaunchArgs& a, hipStream_t s);
 // Bytes of a pool of ids with its lists on lines.
 inline size_t line_bytes(int64_t ids) { return sizeof(int32_t) * (size_t)(2 * ids + kCiPad); }

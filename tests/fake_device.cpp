@@ -79,6 +79,7 @@ static tck::BuildBufs g_build;           // of the last partner build
 static unsigned long long g_closed = 0;  // what launch_big_codes reports
 static int g_big_codes = 0;              // its launches
 static tck::LaunchArgs g_args;           // of the last count
+static int g_sums = 0;                   // launches that add a batch's slots
 static bool g_single = false, g_direct = false;  // of the last plain launch
 static int g_launches = 0;               // plain, zero and rearm launches
 namespace tck {
@@ -105,6 +106,7 @@ hipError_t launch_local_prep(const int64_t*, int64_t, int32_t*, hipStream_t) { r
 hipError_t launch_local_parts(const int32_t*, const int32_t*, int64_t, int64_t, int64_t, const uint32_t*, const int32_t*, int32_t, unsigned long long*, int, hipStream_t) { return hipSuccess; }
 hipError_t launch_copy(const void*, void*, int64_t, int, hipStream_t) { return hipSuccess; }
 hipError_t launch_read(const void*, int64_t, uint32_t*, int, hipStream_t) { return hipSuccess; }
+hipError_t launch_batch_sums(const LaunchArgs& a, hipStream_t) { return ++g_sums, g_args = a, hipSuccess; }
 int count_blocks_per_cu() { return 4; }
 int plain_blocks_per_cu() { return 4; }
 hipError_t noalloc_scratch_address(void** p) { return *p = nullptr, hipSuccess; }
@@ -395,6 +397,31 @@ static void clients(int, char**) {
   tc_server_destroy(s);
 }
 
+// The words of a batch's sums: several a graph where there are few graphs, each
+// on a line of its own inside what the counts' buffer holds.
+static void batch_words(int, char**) {
+  Ctx ctx;
+  const Dag one = make(2000, 1500, 30), wide = make(70000, 1500, 30);
+  for (int n : {1, 2, 5, 15, 16, 17, 31, 33, 63, 64, 65, 200})
+    for (const Dag* g : {&one, &wide}) {
+      const std::vector<tc_csr_view> v((size_t)n, g->view());
+      std::vector<uint64_t> counts((size_t)n);
+      tc_batch* b = nullptr;
+      CHECK(tc_batch_create(ctx, v.data(), n, TC_CHECK_SHAPE, &b) == TC_OK);
+      g_sums = 0;
+      CHECK(tc_batch_count(ctx, b, counts.data(), nullptr) == TC_OK);
+      const bool slots = n > 1 && n < tck::kBatchGraphs && g == &one;  // (the other has no codes)
+      CHECK(g_sums == (slots ? 1 : 0) && (g_args.slots != nullptr) == slots);
+      if (slots) {
+        const int s = g_args.nslots;
+        CHECK(s > 1 && s <= tck::kOutSlots && (s & (s - 1)) == 0 && s * n <= tck::kBatchWords);
+        CHECK(g_args.slots - g_args.bufs.outs >= n && (g_args.slots - g_args.bufs.outs) % tck::kOutStride == 0);
+        CHECK((size_t)(g_args.slots - g_args.bufs.outs + (int64_t)n * s * tck::kOutStride) * 8 <= g_size[g_args.bufs.outs]);
+      }
+      tc_batch_free(ctx, b);
+    }
+}
+
 int main(int argc, char** argv) {
   static const std::map<std::string, std::function<void(int, char**)>> all = {
       {"one_shot", one_shot},
@@ -402,6 +429,7 @@ int main(int argc, char** argv) {
       {"choice", choice},
       {"plain", plain},
       {"clients", clients},
+      {"batch_words", batch_words},
   };
   const auto it = argc > 1 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;

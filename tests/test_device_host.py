@@ -56,3 +56,7 @@ def test_a_plain_count_is_one_launch(fake):
 
 def test_clients_share_the_copy_threads(fake):
     fake("clients")
+
+
+def test_words_of_a_batch(fake):
+    fake("batch_words")
