@@ -23,6 +23,7 @@ struct tc_batch final : tcr::Spare {
   std::vector<tck::GraphDesc> descs;
   std::vector<int32_t> rows;
   std::vector<uint8_t> short_lists;  // per graph, DagShape::short_lists
+  bool many_light = false;           // tck::LaunchArgs::many_light
   int64_t P = 0;        // plan indices (partner-row slots over all graphs)
   int64_t RP = 0;       // rowptr pool slots
   int64_t cio = 0;      // colidx pool slots
@@ -78,6 +79,7 @@ static tc_status capture(tc_ctx* ctx, tc_batch* b) {
   a.c16 = b->c16;
   a.core = b->c16 ? 1 : 0;
   a.core_kb = b->core_kb;
+  a.many_light = b->many_light ? 1 : 0;
   a.nslots = b->nslots();
   if (a.nslots > 1) a.slots = a.bufs.outs + b->slots_at();
   const int64_t words = a.slots ? b->slots_at() + (int64_t)b->n * a.nslots * tck::kOutStride : b->n;
@@ -128,16 +130,20 @@ static tc_status build_batch(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_gra
   b->descs.resize(n_graphs);
   b->rows.resize(n_graphs);
   b->short_lists.resize(n_graphs);
-  int64_t rpo = 0, cio = 0, pro = 0;
+  int64_t rpo = 0, cio = 0, pro = 0, short_rows = 0, wave_rows = 0;
   for (int32_t i = 0; i < n_graphs; ++i) {
     const int32_t nvm = tck::partner_rows_max(dags[i].n_rows, dags[i].nnz);
     b->descs[i] = tck::GraphDesc{rpo, cio, cio, rpo, pro, dags[i].n_rows, nvm, 0, dags[i].n_rows, cio};
     b->rows[i] = dags[i].n_rows;
-    b->short_lists[i] = DagShape(dags[i]).short_lists();
+    const DagShape shape(dags[i]);
+    b->short_lists[i] = shape.short_lists();
+    short_rows += shape.short_rows;
+    wave_rows += shape.wave_rows;
     rpo += dags[i].n_rows + 1;
     cio += dags[i].nnz;
     pro += (int64_t)nvm + 1;
   }
+  b->many_light = short_rows > tck::kManyLight * wave_rows;
   b->P = pro;
   b->RP = rpo;
   b->cio = cio;

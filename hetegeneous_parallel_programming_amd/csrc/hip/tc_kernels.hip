@@ -2248,7 +2248,6 @@ __global__ __launch_bounds__(kBlock, waves_per_eu(kLocal)) void count_kernel(Lau
 }
 
 // ---------------------------------------------------------------------------
-// bitmap count of heavy partner rows// ---------------------------------------------------------------------------
 // bitmap count of heavy partner rows
 // ---------------------------------------------------------------------------
 // When every id of a graph has a 16-bit code, a row's set is a bitmap of at
@@ -3149,8 +3148,8 @@ static void launch_hash(const LaunchArgs& a, int cus, int grid, uint32_t bins, c
   }
 }
 
-// The bitmap kernel of bins bin0..bin1,// The bitmap kernel of bins bin0..bin1, which use queue head `head`; rows as
-// for launch_bin.
+// The bitmap kernel of bins bin0..bin1, which use queue `head`; rows: how many
+// (-1: not known on the host).
 template <int NW>
 static int core_blocks_per_cu(int kb) {
   int k = 0;
@@ -3158,18 +3157,27 @@ static int core_blocks_per_cu(int kb) {
   return k > 0 ? k : 1;
 }
 // Workgroups per CU of the bitmap kernels where the hash kernel has rows of the
-// same count: they leave it 2 of a CU's 8 places from the start.  Workgroups
-// stay until the queue is empty, so at full residency the hash kernel's would
-// start when the bitmap kernels end, and work bound by memory would not run
-// beside work bound by latency (R-MAT-22: 3.45 ms; 5 and 4: 3.20; 4 and 4:
-// 3.22; 3 and 4: 3.54.  Part 0 of R-MAT-21 in four: 0.59 / 0.54 / 0.53 / 0.60).
-constexpr int kBlockBeside = 4, kWaveBeside = 3;
+// same count: they leave it three of a CU's eight places from the start (4
+// workgroups of 4 waves and 3 to 8 of one, of 32 waves).  Workgroups stay until
+// the queue is empty, so at full residency the hash kernel's would start when
+// the bitmap kernels end, and work bound by memory would not run beside work
+// bound by latency (R-MAT-22, workgroups of 4 waves and of one: at full
+// residency 3.45 ms; 5 and 4: 3.20; 4 and 4: 3.22; 3 and 4: 3.54.  Part 0 of
+// R-MAT-21 in four: 0.59 / 0.54 / 0.53 / 0.60).  The wave rows of a batch have
+// kWaveBeside where its lighter rows are at most kManyLight times as many (8
+// graphs ER n=20000 of 1.6 M ids, as many: 0.46 to 0.52 with 8, 0.91 to 0.96
+// with 3; 400 R-MAT n=2000 of 60 K ids, 8 times: 0.90, 1.09), else
+// kWaveBesideMany (the batch of 512 graphs, 59 times: 2.64 with 8, 2.52 with
+// 3).  For single graphs the two are even (R-MAT n=2000000 of 40 M ids, 7 times:
+// 1.94, 1.96; R-MAT-22, 10 times: 3.17, 3.17): kWaveBesideMany.
+constexpr int kBlockBeside = 4, kWaveBeside = 8, kWaveBesideMany = 3;
 template <int NW>
 static void launch_core(const LaunchArgs& a, int cus, int grid, hipStream_t s, int64_t rows, int bin0, int bin1,
-                        int head, bool beside) {
+                        int head, bool beside, bool many_light) {
   if (rows == 0) return;
   int64_t g = grid > 0 ? grid : (int64_t)core_blocks_per_cu<NW>(a.core_kb) * cus;
-  if (grid <= 0 && beside) g = min(g, (int64_t)cus * (NW == 1 ? kWaveBeside : kBlockBeside));
+  if (grid <= 0 && beside)
+    g = min(g, (int64_t)cus * (NW > 1 ? kBlockBeside : many_light ? kWaveBesideMany : kWaveBeside));
   if (rows > 0) g = min(g, (rows + 7) & ~(int64_t)7);
   core_kernel<NW><<<(unsigned)g, 64 * NW, (size_t)1 << a.core_kb, s>>>(a, bin0, bin1, head);
 }
@@ -3215,8 +3223,9 @@ hipError_t launch_count_part(const LaunchArgs& a, int cus, int grid, int part, c
     int64_t n = rows ? 0 : -1;
     for (int b = b0; rows && b <= b1; ++b) n += rows[b];
     const bool beside = !part_empty(a, kPartHash, rows);
-    if (part == kPartBlock) launch_core<kWaves>(a, cus, grid, s, n, b0, b1, kCoreHead, beside);
-    else launch_core<1>(a, cus, grid, s, n, b0, b1, kCoreHead + 1, beside);
+    const bool many_light = rows || a.many_light;
+    if (part == kPartBlock) launch_core<kWaves>(a, cus, grid, s, n, b0, b1, kCoreHead, beside, many_light);
+    else launch_core<1>(a, cus, grid, s, n, b0, b1, kCoreHead + 1, beside, many_light);
   }
   return hipGetLastError();
 }

@@ -301,6 +301,8 @@ struct LaunchArgs {
   // a cache line apart, i < nslots (a power of two), added by launch_batch_sums.
   uint64_t* slots;
   int32_t nslots;
+  int32_t many_light;   // a batch (whose rows per bin the host does not know): over kManyLight times as many
+                        // rows of the light bins as of the wave bin, by the lists' lengths
   int32_t gbase;        // partner build of a segment of graphs: index of descs[0] among all graphs
 };
 
@@ -492,6 +494,8 @@ hipError_t launch_count(const LaunchArgs& a, int cus, int grid, hipStream_t s);
 // resident wave on (the batch of 512 graphs, 215 K rows of the 32-lane bin:
 // 0.53 ms there, 0.64 ms here).
 constexpr int64_t kCoreLightRows = 32768;
+// launch_core's comment has both sides measured.
+constexpr int64_t kManyLight = 8;
 constexpr int kPartBlock = 0, kPartWave = 1, kPartHash = 2, kCountParts = 3;
 bool part_empty(const LaunchArgs& a, int part, const int64_t* rows);
 hipError_t launch_count_part(const LaunchArgs& a, int cus, int grid, int part, const int64_t* rows, hipStream_t s);

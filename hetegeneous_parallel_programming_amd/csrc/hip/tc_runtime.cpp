@@ -310,6 +310,8 @@ DagShape::DagShape(const tc_csr_view& dag) {
     max_out = std::max(max_out, d);
     squares += (uint64_t)d * (uint64_t)d;
     lists += d > 0;
+    short_rows += d > 0 && d < 64;
+    wave_rows += d >= 64 && d < 128;
   }
   if (lists) {
     mean = (double)squares / (double)dag.nnz;

@@ -422,6 +422,24 @@ static void batch_words(int, char**) {
     }
 }
 
+// Whether a batch has many light rows to a wave row.
+static void light(int, char**) {
+  Ctx ctx;
+  const struct {
+    Dag g;
+    int many;
+  } all[] = {{make(3000, 2500, 30), 1}, {make(3000, 2500, 80), 0}, {make(3000, 800, 63, 100, 64), 0},
+             {make(3000, 801, 63, 100, 64), 1}, {make(3000, 801, 63, 100, 127), 1}, {make(3000, 10, 5, 100, 128), 1}};
+  for (const auto& x : all) {
+    const tc_csr_view v[2] = {x.g.view(), x.g.view()};
+    tc_batch* b = nullptr;
+    uint64_t counts[2];
+    CHECK(tc_batch_create(ctx, v, 2, TC_CHECK_SHAPE, &b) == TC_OK && tc_batch_count(ctx, b, counts, nullptr) == TC_OK);
+    CHECK(g_args.many_light == x.many);
+    tc_batch_free(ctx, b);
+  }
+}
+
 int main(int argc, char** argv) {
   static const std::map<std::string, std::function<void(int, char**)>> all = {
       {"one_shot", one_shot},
@@ -430,6 +448,7 @@ int main(int argc, char** argv) {
       {"plain", plain},
       {"clients", clients},
       {"batch_words", batch_words},
+      {"light", light},
   };
   const auto it = argc > 1 ? all.find(argv[1]) : all.end();
   if (it == all.end()) return 2;

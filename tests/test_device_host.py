@@ -60,3 +60,7 @@ def test_clients_share_the_copy_threads(fake):
 
 def test_words_of_a_batch(fake):
     fake("batch_words")
+
+
+def test_batches_with_many_light_rows(fake):
+    fake("light")
