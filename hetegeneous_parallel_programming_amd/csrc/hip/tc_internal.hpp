@@ -1,4 +1,4 @@
-// Internal state of the device library shared by tc_runtime.cpp,
+// Internal state of the device library shared by tc_runtime.cpp, tc_copy.cpp,
 // tc_batch.cpp, tc_server.cpp and tc_tune.cpp.
 #pragma once
 
@@ -235,7 +235,7 @@ struct tc_ctx {
   tcr::PlanScratch scratch;
   tcr::Stager stager;
   std::unordered_set<tcr::Spare*> spares;  // the graphs and batches that hold any
-  uint64_t* pinned = nullptr;  // 64 B count + 64 B bin counters
+  uint64_t* pinned = nullptr;  // 256 B: a build's results and copied counts, plan counters, a count's sum
   uint64_t* pinned_dev = nullptr;  // its device address
   void* noalloc = nullptr;     // device address of the static scratch of tc_count_noalloc
   // device: the single-launch count's kOutWords words, which every call

@@ -25,10 +25,13 @@
 //
 // Scheduling.  A planning pass bins partner rows by set size and work (the
 // total length of their partners' lists) into workgroup, wave and 32/16/8-
-// lane groups; one persistent kernel per bin pulls tiles (runs of rows of
-// that bin) from a device queue, heaviest bins first.  Counts are u64 sums,
-// so the result does not depend on tile order.  Local variants of the bin
-// kernels also attribute every hit to its edge and corners.
+// lane groups.  A count is up to three persistent launches side by side: the
+// bitmap kernels of the workgroup and the wave bins, where ids have 16-bit
+// codes, and one hash kernel over all other bins, heaviest first.  They pull
+// tiles (runs of rows of a bin) from eight queues per bin, one per XCD.
+// Counts are u64 sums, so the result does not depend on tile order.  Local
+// variants of the hash kernel also attribute every hit to its edge and
+// corners.
 #include <algorithm>
 #include <climits>
 #include <type_traits>
@@ -3148,8 +3151,6 @@ static void launch_hash(const LaunchArgs& a, int cus, int grid, uint32_t bins, c
   }
 }
 
-// The bitmap kernel of bins bin0..bin1, which use queue `head`; rows: how many
-// (-1: not known on the host).
 template <int NW>
 static int core_blocks_per_cu(int kb) {
   int k = 0;
@@ -3171,6 +3172,9 @@ static int core_blocks_per_cu(int kb) {
 // 3).  For single graphs the two are even (R-MAT n=2000000 of 40 M ids, 7 times:
 // 1.94, 1.96; R-MAT-22, 10 times: 3.17, 3.17): kWaveBesideMany.
 constexpr int kBlockBeside = 4, kWaveBeside = 8, kWaveBesideMany = 3;
+
+// The bitmap kernel of bins bin0..bin1, which use queue `head`; rows: how many
+// (-1: not known on the host).
 template <int NW>
 static void launch_core(const LaunchArgs& a, int cus, int grid, hipStream_t s, int64_t rows, int bin0, int bin1,
                         int head, bool beside, bool many_light) {

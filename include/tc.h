@@ -192,7 +192,7 @@ tc_status tc_count_noalloc(tc_ctx* ctx, tc_graph* g, uint64_t* total, tc_stats* 
  * The reference emits none of these but the per-PE sums; they make a
  * split's attribution checkable.  A call without vertex_counts attributes
  * each triangle to its edge only (edge_counts and part_counts are the same;
- * RMAT-22: 11.8 ms against 19.5 ms with vertex_counts).  A call with
+ * RMAT-22: 9.4 ms against 19.4 ms with vertex_counts).  A call with
  * part_counts alone (edge_counts and vertex_counts null, parts > 0) adds
  * each partner row's triangles to its owner's part, which is the part that
  * computes the row's edges under the push/pull rule: no per-edge counts,
