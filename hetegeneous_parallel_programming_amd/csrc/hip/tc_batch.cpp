@@ -130,15 +130,20 @@ static tc_status build_batch(tc_ctx* ctx, const tc_csr_view* dags, int32_t n_gra
   b->descs.resize(n_graphs);
   b->rows.resize(n_graphs);
   b->short_lists.resize(n_graphs);
-  int64_t rpo = 0, cio = 0, pro = 0, short_rows = 0, wave_rows = 0;
+  int64_t rpo = 0, cio = 0, pro = 0;
+  // Lists of up to 63 ids, and of 64 to 127: about the rows of the light bins and
+  // of the wave bin (a row's work goes with the square of its list).
+  int64_t short_rows = 0, wave_rows = 0;
   for (int32_t i = 0; i < n_graphs; ++i) {
     const int32_t nvm = tck::partner_rows_max(dags[i].n_rows, dags[i].nnz);
     b->descs[i] = tck::GraphDesc{rpo, cio, cio, rpo, pro, dags[i].n_rows, nvm, 0, dags[i].n_rows, cio};
     b->rows[i] = dags[i].n_rows;
-    const DagShape shape(dags[i]);
-    b->short_lists[i] = shape.short_lists();
-    short_rows += shape.short_rows;
-    wave_rows += shape.wave_rows;
+    b->short_lists[i] = DagShape(dags[i]).short_lists();
+    for (int32_t v = 0; v < dags[i].n_rows; ++v) {
+      const int64_t d = dags[i].rowptr[v + 1] - dags[i].rowptr[v];
+      short_rows += d > 0 && d < 64;
+      wave_rows += d >= 64 && d < 128;
+    }
     rpo += dags[i].n_rows + 1;
     cio += dags[i].nnz;
     pro += (int64_t)nvm + 1;

@@ -145,9 +145,6 @@ struct DagShape {
   uint64_t squares = 0;  // sum of the out-degrees' squares: bounds the ids a count streams
   double mean = 0;       // squares per id: the mean length of the list an id is in
   double skew = 0;       // squares against those of lists of equal length
-  // Rows with lists of up to 63 ids, and of 64 to 127: about those of the light
-  // bins and of the wave bin (a row's work goes with the square of its list).
-  int64_t short_rows = 0, wave_rows = 0;
   DagShape() = default;
   explicit DagShape(const tc_csr_view& dag);  // (rowptr checked; squares stay below 2^64 where max_out passes)
   // ER graphs of mean out-degree 2 to 100 have 1.1 to 1.5, R-MAT graphs 3.5 and more.
